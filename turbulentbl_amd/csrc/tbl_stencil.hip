@@ -6,6 +6,8 @@
 // the reference's formulas.  Templates on the storage type T give the FP32
 // (mixed-precision) variants; quantities the reference accumulates (residual
 // norms) are always accumulated in double.
+#include <algorithm>
+
 #include "tbl_dev.h"
 #include "tbl_launch.h"
 
@@ -32,7 +34,7 @@ template <class T> __device__ __forceinline__ T tabs(T x) { return x < T(0) ? -x
 // Q = (U + dt (forc - conv)) - dt gradp.
 // ----------------------------------------------------------------------------
 #ifndef RHS_KCHUNK
-#define RHS_KCHUNK 32   // planes per workgroup (register-queue kernel)
+#define RHS_KCHUNK 32   // most planes per workgroup (register-queue kernel)
 #endif
 #define RHS_KCHUNK_F32 192   // most planes per workgroup of the FP32 tile kernel
 #define RHS_TJ 8   // span rows per workgroup (64 x RHS_TJ columns): fewer span-halo re-reads
@@ -682,7 +684,10 @@ __global__ __launch_bounds__(64 * ZL_MAXC) void k_helm_zline(Geo g, const T *__r
     // blocks run span-row-first inside panels of pw column tiles, so that the
     // rows j-1, j, j+1 (the span neighbours of row j) are swept at nearly the
     // same time and their second and third reads hit L2
-    const unsigned L = xcd_remap(blockIdx.x, nblk);
+    // a block sweeps one component (component slowest): the three do not read
+    // each other
+    const int p = (int)(blockIdx.x / nblk);
+    const unsigned L = xcd_remap(blockIdx.x - (unsigned)p * nblk, nblk);
     const unsigned nyr = nblk / nbx;
     const unsigned P = L / (pw * nyr), w_ = min(pw, nbx - P * pw), rem = L - P * pw * nyr;
     const int bx = (int)(P * pw + rem % w_), j = (int)(rem / w_) + 1;
@@ -1517,13 +1522,21 @@ static inline dim3 rgrid(const Geo &g, int *kchunk)
 }
 unsigned resid_blocks(const Geo &g) { RTiles r = rtiles_of(g.nX, g.nY, g.nZ); return (unsigned)(r.gx * r.gy * r.kb); }
 
-// planes per block of the FP32 tile kernel: the column is cut into the
+// planes per block of the momentum kernels: the column is cut into the
 // number of chunks that minimises (waves of blocks over the resident slots) x
-// (planes per chunk + 5, the queue prologue and halo planes); the slots are
-// MI355X's 256 CUs x 2 resident blocks of 512 threads at 128 VGPRs.  A
-// chunk's buffer range stays below 2^31 bytes (stores of lanes outside the
-// field go to offset 2^31).  0: no chunk fits, the register-queue kernel runs.
-static int rhs_chunk_f32(const Geo &g)
+// (planes per chunk + the queue prologue and halo planes); the slots are
+// MI355X's 256 CUs x 2 resident blocks of 512 threads at up to 128 VGPRs
+// (both kernels).  Chunks longer than kmax are not considered.
+//  * FP32 tile kernel: 5 prologue planes, chunks of at least 8 planes (its
+//    LDS tiles and prefetch ring fill over three planes); a chunk's buffer
+//    range stays below 2^31 bytes (stores of lanes outside the field go to
+//    offset 2^31).  0: no chunk fits, the register-queue kernel runs.
+//  * register-queue kernel: 4 prologue planes, up to 32 planes.  A plane costs
+//    a thread one load latency (2.5 us in FP64), so a grid that leaves the
+//    chip idle at 32 planes is cut down to one plane per block: 64x32x48
+//    94 -> 10 us, 256x64x96 96 -> 34 us; 512x128x128 and larger keep
+//    32 planes.
+static int rhs_chunk_of(const Geo &g, int kmax, int kmin, int over)
 {
     const long tiles = (long)((g.nX - 1 + 63) / 64) * ((g.nY - 2 + RHS_TJ - 1) / RHS_TJ), slots = 512;
     const int nz = g.nZ - 2;
@@ -1531,20 +1544,21 @@ static int rhs_chunk_f32(const Geo &g)
     long bestc = -1;
     for (int nbz = 1; nbz <= nz; nbz++) {
         const int kc = (nz + nbz - 1) / nbz, nb = (nz + kc - 1) / kc;
-        if (kc > RHS_KCHUNK_F32 || (long)(kc + MR_R + 5) * g.sZ * 4 >= (1L << 31)) continue;
-        const long cost = (tiles * nb + slots - 1) / slots * (kc + 5);
+        if (kc > kmax || (kmin > 1 && (long)(kc + MR_R + 5) * g.sZ * 4 >= (1L << 31))) continue;
+        const long cost = (tiles * nb + slots - 1) / slots * (kc + over);
         if (bestc < 0 || cost < bestc) { bestc = cost; best = kc; }
-        if (kc <= 8) break;
+        if (kc <= kmin) break;
     }
     return best;
 }
+static int rhs_chunk_f32(const Geo &g) { return rhs_chunk_of(g, RHS_KCHUNK_F32, 8, 5); }
 static bool rhs_tile_kernel(const Geo &g, bool single)
 {
     return single && g.scheme == TBL_SCHEME_SETBL && rhs_chunk_f32(g) > 0;
 }
 static int rhs_chunk(const Geo &g, bool single)
 {
-    return rhs_tile_kernel(g, single) ? rhs_chunk_f32(g) : RHS_KCHUNK;
+    return rhs_tile_kernel(g, single) ? rhs_chunk_f32(g) : rhs_chunk_of(g, RHS_KCHUNK, 1, 4);
 }
 // column tiles start at i = 0 (cache-line aligned) and cover i <= nX-2
 static unsigned rhs_nbx(const Geo &g, bool)
