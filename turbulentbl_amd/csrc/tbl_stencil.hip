@@ -685,7 +685,10 @@ __global__ __launch_bounds__(64 * ZL_MAXC) void k_helm_zline(Geo g, const T *__r
     // rows j-1, j, j+1 (the span neighbours of row j) are swept at nearly the
     // same time and their second and third reads hit L2
     // a block sweeps one component (component slowest): the three do not read
-    // each other
+    // each other, a small grid gets three times the blocks of its serial
+    // chains, and on a large one a block's barriers wait less on each other.
+    // One pass: FP64 64x32x48 33.5 -> 11 us, 256x64x96 40 -> 20 us,
+    // 512x128x128 95 -> 83 us; FP32 1024x256x192 275 -> 259 us
     const int p = (int)(blockIdx.x / nblk);
     const unsigned L = xcd_remap(blockIdx.x - (unsigned)p * nblk, nblk);
     const unsigned nyr = nblk / nbx;
@@ -838,7 +841,13 @@ __attribute__((amdgpu_waves_per_eu((sizeof(T) == 4 && LC == 16) ? 6 : 1))) void 
     // blocks run row-first inside panels of pw column tiles, so that the rows
     // j and j+2 of this colour, which share the span neighbour row j+1, are
     // swept at nearly the same time and its second read hits L2
-    const unsigned L = xcd_remap(blockIdx.x, nblk);
+    // a block sweeps one component (component slowest): the three do not read
+    // each other, a small grid gets three times the blocks of its serial
+    // chains, and on a large one a block's barriers wait less on each other.
+    // One pass: FP64 64x32x48 33.5 -> 11 us, 256x64x96 40 -> 20 us,
+    // 512x128x128 95 -> 83 us; FP32 1024x256x192 275 -> 259 us
+    const int p = (int)(blockIdx.x / nblk);
+    const unsigned L = xcd_remap(blockIdx.x - (unsigned)p * nblk, nblk);
     const unsigned nyr = nblk / nbx;
     const unsigned P = L / (pw * nyr), w_ = min(pw, nbx - P * pw), rem = L - P * pw * nyr;
     // ZB_REV: the second colour's rows run from the last to the first, so
@@ -872,98 +881,95 @@ __attribute__((amdgpu_waves_per_eu((sizeof(T) == 4 && LC == 16) ? 6 : 1))) void 
         sF[4 * ZL_MAXC + e] = in ? re[e] : T(0);
     }
     struct Op { T q, e, w, n, s; };
-    for (int p = 0; p < 3; p++) {
-        // per-lane bases at the chunk's first plane; every other offset
-        // (planes, neighbours, the other arrays) is wave-uniform
-        const T *cb = cur + (long)p * N + (c0 + sk * kb);
-        if (!ctrl->active[p]) {                                  // uniform over the grid
-            T *db = dst + (long)p * N + (c0 + sk * kb);
-            if (live)
-                for (int r = 0; r < M; r++) db[sk * r] = cb[sk * r];
-            continue;
-        }
-        const T *qb = Q + (long)p * N + (c0 + sk * kb);
-        const T *yb = ysrc + (long)p * N + (c0 + sk * kb);
-        auto ld = [&](int r, Op &o) {
-            const int o_ = sk * r;
-            o.q = qb[o_]; o.e = cb[o_ + 1]; o.w = cb[o_ - 1]; o.n = yb[o_ + dn]; o.s = yb[o_ + ds];
-        };
-        T dp[LC];
-        if (live) {
-            // the operands of the next ZPF planes are in flight.  Every load
-            // is unconditional (plane indices clamped to the chunk; the wall
-            // and top values, used by the first and last chunk only, are
-            // loaded once up front): a branch around a load makes the
-            // compiler's in-order wait counts drain the whole ring
-            const T wall = cb[-sk], top = cb[sk * M];
-            const T Abw = T(g.Ab[kb]), Att = T(g.At[kb + M - 1]);
-            // ZPF + 1 slots: the slot refilled in step r is never the one
-            // step r reads, so the new loads need not wait for its compute
-            Op ring[ZPF + 1];
+    // per-lane bases at the chunk's first plane; every other offset
+    // (planes, neighbours, the other arrays) is wave-uniform
+    const T *cb = cur + (long)p * N + (c0 + sk * kb);
+    if (!ctrl->active[p]) {                                  // uniform over the grid
+        T *db = dst + (long)p * N + (c0 + sk * kb);
+        if (live)
+            for (int r = 0; r < M; r++) db[sk * r] = cb[sk * r];
+        return;
+    }
+    const T *qb = Q + (long)p * N + (c0 + sk * kb);
+    const T *yb = ysrc + (long)p * N + (c0 + sk * kb);
+    auto ld = [&](int r, Op &o) {
+        const int o_ = sk * r;
+        o.q = qb[o_]; o.e = cb[o_ + 1]; o.w = cb[o_ - 1]; o.n = yb[o_ + dn]; o.s = yb[o_ + ds];
+    };
+    T dp[LC];
+    if (live) {
+        // the operands of the next ZPF planes are in flight.  Every load
+        // is unconditional (plane indices clamped to the chunk; the wall
+        // and top values, used by the first and last chunk only, are
+        // loaded once up front): a branch around a load makes the
+        // compiler's in-order wait counts drain the whole ring
+        const T wall = cb[-sk], top = cb[sk * M];
+        const T Abw = T(g.Ab[kb]), Att = T(g.At[kb + M - 1]);
+        // ZPF + 1 slots: the slot refilled in step r is never the one
+        // step r reads, so the new loads need not wait for its compute
+        Op ring[ZPF + 1];
 #pragma unroll
-            for (int r = 0; r < ZPF; r++) ld(min(r, M - 1), ring[r]);
+        for (int r = 0; r < ZPF; r++) ld(min(r, M - 1), ring[r]);
 #pragma unroll
-            for (int r = 0; r < LC; r++) {
-                // outside the r < M test (M is below LC by at most one plane)
-                ld(min(r + ZPF, M - 1), ring[(r + ZPF) % (ZPF + 1)]);
-                if (r < M) {
-                    const int k = kb + r;
-                    const Op cur_ = ring[r % (ZPF + 1)];
-                    T rhs = cur_.q + h * (Ae * cur_.e + Aw * cur_.w + An * cur_.n + As * cur_.s);
-                    if (k == 1) rhs = rhs + h * (Abw * wall);
-                    if (k == nZ - 2) rhs = rhs + h * (Att * top);
-                    if (r == 0) dp[0] = rhs;
-                    else dp[r] = (rhs - zA[k] * dp[r - 1]) * zR[k];
-                }
-                __builtin_amdgcn_sched_barrier(0);
+        for (int r = 0; r < LC; r++) {
+            // outside the r < M test (M is below LC by at most one plane)
+            ld(min(r + ZPF, M - 1), ring[(r + ZPF) % (ZPF + 1)]);
+            if (r < M) {
+                const int k = kb + r;
+                const Op cur_ = ring[r % (ZPF + 1)];
+                T rhs = cur_.q + h * (Ae * cur_.e + Aw * cur_.w + An * cur_.n + As * cur_.s);
+                if (k == 1) rhs = rhs + h * (Abw * wall);
+                if (k == nZ - 2) rhs = rhs + h * (Att * top);
+                if (r == 0) dp[0] = rhs;
+                else dp[r] = (rhs - zA[k] * dp[r - 1]) * zR[k];
             }
-#pragma unroll
-            for (int r = LC - 3; r >= 1; r--)
-                if (r <= M - 3) dp[r] = dp[r] - zC[kb + r] * dp[r + 1];
-            T DL = dp[1];
-#pragma unroll
-            for (int r = 2; r < LC; r++)
-                if (r == M - 1) DL = dp[r];
-            sD[(2 * w) * 64 + lane] = dp[0] - zc0[w] * dp[1];
-            sD[(2 * w + 1) * 64 + lane] = DL;
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
-        if (w == 0 && live) {
-            T y = sD[lane] * sF[2 * ZL_MAXC];
-            sD[lane] = y;
 #pragma unroll
-            for (int s2 = 1; s2 < 2 * ZL_MAXC; s2++) {
-                if (s2 < 2 * C) {
-                    y = (sD[s2 * 64 + lane] - sF[s2] * y) * sF[2 * ZL_MAXC + s2];
-                    sD[s2 * 64 + lane] = y;
-                }
-            }
-            T x = y;
+        for (int r = LC - 3; r >= 1; r--)
+            if (r <= M - 3) dp[r] = dp[r] - zC[kb + r] * dp[r + 1];
+        T DL = dp[1];
 #pragma unroll
-            for (int s2 = 2 * ZL_MAXC - 2; s2 >= 0; s2--) {
-                if (s2 <= 2 * C - 2) {
-                    x = sD[s2 * 64 + lane] - sF[4 * ZL_MAXC + s2] * x;
-                    sD[s2 * 64 + lane] = x;
-                }
+        for (int r = 2; r < LC; r++)
+            if (r == M - 1) DL = dp[r];
+        sD[(2 * w) * 64 + lane] = dp[0] - zc0[w] * dp[1];
+        sD[(2 * w + 1) * 64 + lane] = DL;
+    }
+    __syncthreads();
+    if (w == 0 && live) {
+        T y = sD[lane] * sF[2 * ZL_MAXC];
+        sD[lane] = y;
+#pragma unroll
+        for (int s2 = 1; s2 < 2 * ZL_MAXC; s2++) {
+            if (s2 < 2 * C) {
+                y = (sD[s2 * 64 + lane] - sF[s2] * y) * sF[2 * ZL_MAXC + s2];
+                sD[s2 * 64 + lane] = y;
             }
         }
-        __syncthreads();
-        if (live) {
-            T *db = dst + (long)p * N + (c0 + sk * kb);
-            const T xf = sD[(2 * w) * 64 + lane], xl = sD[(2 * w + 1) * 64 + lane];
+        T x = y;
 #pragma unroll
-            for (int r = 0; r < LC; r++) {
-                if (r < M) {
-                    const int k = kb + r;
-                    T x;
-                    if (r == 0) x = xf;
-                    else if (r == M - 1) x = xl;
-                    else x = dp[r] - zA2[k] * xf - zC2[k] * xl;
-                    db[sk * r] = x;
-                }
+        for (int s2 = 2 * ZL_MAXC - 2; s2 >= 0; s2--) {
+            if (s2 <= 2 * C - 2) {
+                x = sD[s2 * 64 + lane] - sF[4 * ZL_MAXC + s2] * x;
+                sD[s2 * 64 + lane] = x;
             }
         }
-        __syncthreads();                                         // sD is reused by the next component
+    }
+    __syncthreads();
+    if (live) {
+        T *db = dst + (long)p * N + (c0 + sk * kb);
+        const T xf = sD[(2 * w) * 64 + lane], xl = sD[(2 * w + 1) * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < LC; r++) {
+            if (r < M) {
+                const int k = kb + r;
+                T x;
+                if (r == 0) x = xf;
+                else if (r == M - 1) x = xl;
+                else x = dp[r] - zA2[k] * xf - zC2[k] * xl;
+                db[sk * r] = x;
+            }
+        }
     }
 }
 
@@ -1652,10 +1658,10 @@ void launch_helm_zebra(const Geo &g, const T *Q, const T *cur, const T *ysrc, T 
     // and FP64 free of spills
     constexpr int ZPF16 = 1;
     if (LC == 16)
-        hipLaunchKernelGGL((k_helm_zebra<T, 16, ZPF16>), dim3(nblk), dim3(64 * C), 0, s, g, Q, cur, ysrc, dst, zf,
+        hipLaunchKernelGGL((k_helm_zebra<T, 16, ZPF16>), dim3(3 * nblk), dim3(64 * C), 0, s, g, Q, cur, ysrc, dst, zf,
                            (const GsCtrl *)ctrl, colour, C, nbx, nblk, pw);
     else
-        hipLaunchKernelGGL((k_helm_zebra<T, 32, 1>), dim3(nblk), dim3(64 * C), 0, s, g, Q, cur, ysrc, dst, zf,
+        hipLaunchKernelGGL((k_helm_zebra<T, 32, 1>), dim3(3 * nblk), dim3(64 * C), 0, s, g, Q, cur, ysrc, dst, zf,
                            (const GsCtrl *)ctrl, colour, C, nbx, nblk, pw);
 }
 template <class T>
