@@ -1692,17 +1692,26 @@ void launch_ppe_rhs(const Geo &g, const T *Ut, double *pRhs, hipStream_t s, cons
 }
 
 #ifndef POISSON_KC
-#define POISSON_KC 16   // wall-normal planes per thread of the Poisson apply
+#define POISSON_KC 16   // most wall-normal planes per thread of the Poisson apply
 #endif
+// planes per thread: POISSON_KC, fewer where that leaves less than 2048 blocks
+// (256 CUs x 8 resident blocks): a plane costs a thread one load latency.
+// 64x32x48 17 -> 6 us, 256x64x96 21 -> 15 us
+static int poisson_chunk(const Geo &g)
+{
+    const long tiles = (long)((g.nX - 1 + 63) / 64) * ((g.nY - 2 + 3) / 4);
+    return (int)std::max(1L, std::min((long)POISSON_KC, (g.nZ - 2) * tiles / 2048));
+}
 unsigned poisson_blocks(const Geo &g)
 {
-    return (unsigned)(((g.nX - 1 + 63) / 64) * ((g.nY - 2 + 3) / 4) * ((g.nZ - 2 + POISSON_KC - 1) / POISSON_KC));
+    const int kc = poisson_chunk(g);
+    return (unsigned)(((g.nX - 1 + 63) / 64) * ((g.nY - 2 + 3) / 4) * ((g.nZ - 2 + kc - 1) / kc));
 }
 template <class T>
 unsigned launch_poisson(const Geo &g, const T *x, T *out, const int *active, const double *scale, hipStream_t s,
                         const T *v0, double *part)
 {
-    const int kchunk = POISSON_KC;
+    const int kchunk = poisson_chunk(g);
     unsigned nbx = (g.nX - 1 + 63) / 64, nby = (g.nY - 2 + 3) / 4, nbz = (g.nZ - 2 + kchunk - 1) / kchunk;
     hipLaunchKernelGGL(k_poisson<T>, dim3(nbx * nby * nbz), dim3(256), 0, s, g, x, out, active, scale, v0, part, kchunk,
                        nbx, nby, nbz);
