@@ -33,3 +33,36 @@ def test_momentum_and_poisson_chunks_bitwise(tbl, grid):
         y = sv.apply_operator(0, x)
     assert ulps(Q[I], g.momentum_rhs(s.Ut, s.Press)[1][I]) == 0
     assert ulps(y[I], g.poisson_apply(x)[I]) == 0
+
+
+@pytest.mark.parametrize("precision,rule,errtol,steps", [
+    ("fp64", "true", 1e-9, "one"), ("mixed", "true", 1e-9, "one"),      # unit steps accepted
+    ("fp64", "ref", 1e-9, "one"), ("mixed", "ref", 1e-4, "one"),
+    ("mixed", "ref", 1e-9, "more"),                                     # refused: Arnoldi steps follow
+    ("fp64", "true", 1e-9, "last")])                                    # one cycle allowed: not tried
+def test_unit_steps_of_the_fast_preconditioner(tbl, precision, rule, errtol, steps):
+    """a cycle tries the step of coefficient 1 first; accepted or refused, the
+    solve meets its own stopping rule (residual by the oracle's operator) and
+    counts its cycles as one-step cycles do"""
+    g, s = make_case((70, 12, 21), seed=4)
+    b = g.zeros()
+    b[I] = np.random.default_rng(22).standard_normal([n - 2 for n in (70, 12, 21)])
+    mode = tbl.TBL_TOL_TRUE if rule == "true" else tbl.TBL_TOL_REF
+    with gpu_from_case(g, s, precision=precision, tol_mode=mode, errtol=errtol, kmax=8) as sv:
+        sv.set_field(tbl.F_PCORR, g.zeros())
+        sv.set_field(tbl.F_PRHS, b)
+        out = sv.ppe_solve(errtol=errtol, kmax=8, mmax=1 if steps == "last" else 50)
+        x = sv.get_field(tbl.F_PCORR)
+    rn, bn = np.linalg.norm(b[I] - g.poisson_apply(x)[I]), np.linalg.norm(b[I])
+    assert abs(out["true_res"] - rn) <= 1e-6 * rn + 1e-15 * bn
+    # the preconditioned residual falls by errtol; A and its inverse are
+    # within a factor 1e3 of each other's scaling on this grid.  After refused
+    # FP32 steps the rule tests the Arnoldi estimate in FP32, not this residual
+    if steps != "more":
+        assert rn <= errtol * bn * (1 if rule == "true" else 1e3)
+    if steps == "one":
+        assert out["iters"] == out["cycles"] - (rule == "true")
+    elif steps == "more":
+        assert out["iters"] > 1
+    else:
+        assert out == dict(cycles=1, iters=1, true_res=out["true_res"])

@@ -1122,6 +1122,11 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
     const int *act = &c->gm->st.active;
     const int poll = (N > 2000000 || c->p.precond == TBL_PC_FAST) ? 1 : 4;
     bool final_res = false;                    // st.true_res is the residual of the final PCorr
+    // the second PCorr buffer of fused updates (TRUE) and unit steps
+    if (c->p.precond == TBL_PC_FAST || (mode == GM_MODE_TRUE && poll == 1)) {
+        if (!c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
+        launch_zero_faces(g, c->PCalt, c->s);
+    }
     if (mode == GM_MODE_TRUE) {
         // Flexible (right-preconditioned) GMRES: the Givens estimate is the true
         // residual, one preconditioner application per Arnoldi step, and the
@@ -1141,14 +1146,23 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         // behind that step's status read-back, gated on the cycle having ended
         // (off while the residual class is timed)
         const bool ahead_res = fuse_upd && !(c->tmask & (1u << TBL_K_RESID));
-        if (fuse_upd) {
-            if (!c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
-            launch_zero_faces(g, c->PCalt, c->s);
-        }
         bool pend = false;
         bool queued = false;                   // the cycle's residual pass ran behind the last read-back
+        // unit steps (k_fin_unit) while they are accepted: the fast
+        // preconditioner inverts A to its storage type's rounding, so a cycle
+        // is z_0 = M^{-1} r, the residual of PCorr + z_0 and one read-back; the
+        // operator apply, the dot product and the orthogonalisation pass of
+        // the Arnoldi step are not run, nor the read-back at the solve's start.
+        // The step's residual goes to the other of two vectors (v0, v1), so
+        // that a refused step leaves v_0 for the Arnoldi steps
+        bool unit = c->p.precond == TBL_PC_FAST;
+        bool opened = false;                   // the last unit step opened this cycle
+        bool head = false;                     // its first transform ran behind the last read-back
+        T *v0 = V, *v1 = r;
         for (int m = 0; m < mmax; m++) {
-            if (queued) {
+            const bool try_unit = unit && m + 1 < mmax;   // the last cycle allowed is not followed by a start
+            if (opened) {
+            } else if (queued) {
                 queued = false;
             } else if (pend) {
                 Tscope ts(c, TBL_K_RESID, (double)N * (24.0 + 2.0 * sizeof(T)));
@@ -1160,24 +1174,67 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                 Tscope ts(c, TBL_K_RESID, (double)N * (16.0 + sizeof(T)));
                 launch_resid<T>(g, c->pRhs, c->PCorr, V, part_r, c->s, m == 0 ? part_z : nullptr);
             }
-            if (m == 0) launch_fin_bnorm(c->gm, part_z, (int)nbr, c->s);
-            launch_fin_start(c->gm, part_r, (int)nbr, part_r, (int)nbr, m == 0 ? 1 : 0, c->s);
-            CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
-            // the first Arnoldi step's first transform is queued behind the
-            // status read-back, gated on st.active (0 exactly when the solve
-            // has ended), so the GPU works while the host waits for the status
-            CHK(poll_mark(c));
-            if (ahead) launch_precond<T>(g, c->p.precond, c->fast, V, scr, Z, act, c->s, FPC_HEAD);
-            CHK(poll_spin(c));
-            if (c->gm_h->outer_done) { final_res = true; break; }
+            if (!opened)
+                launch_fin_start(c->gm, part_r, (int)nbr, part_r, (int)nbr, m == 0 ? 1 : 0, c->s,
+                                 m == 0 ? part_z : nullptr);
+            bool have_z0 = false;
+            if (try_unit) {
+                {
+                    Tscope ts(c, TBL_K_PRECOND, precond_bytes(c, sizeof(T)));
+                    launch_precond<T>(g, c->p.precond, c->fast, v0, scr, Z, act, c->s, head ? FPC_TAIL : FPC_ALL);
+                }
+                {
+                    Tscope ts(c, TBL_K_RESID, (double)N * (24.0 + 2.0 * sizeof(T)));
+                    launch_resid_upd<T>(g, c->pRhs, c->PCorr, Z, c->gm, c->PCalt, v1, part_r, c->s, RU_UNIT);
+                }
+                launch_fin_unit(c->gm, part_r, (int)nbr, nullptr, 0, c->s);
+                HIPCHK(c, hipGetLastError());
+                CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
+                CHK(poll_mark(c));
+                if (ahead) launch_precond<T>(g, c->p.precond, c->fast, v1, scr, Z, act, c->s, FPC_HEAD);
+                CHK(poll_spin(c));
+                opened = head = false;
+                if (c->gm_h->unit_ok) {
+                    std::swap(c->PCorr, c->PCalt);
+                    std::swap(v0, v1);
+                    opened = true;
+                    head = ahead;
+                }
+                if (c->gm_h->outer_done) { final_res = true; break; }
+                if (opened) continue;
+                unit = false;
+                have_z0 = true;
+                if (v0 != V) HIPCHK(c, hipMemcpyAsync(V, v0, (size_t)N * sizeof(T), hipMemcpyDeviceToDevice, c->s));
+                v0 = V;
+            } else {
+                // after an accepted unit step the status is known and v_0 may
+                // lie in the other vector
+                if (opened && v0 != V) {
+                    HIPCHK(c, hipMemcpyAsync(V, v0, (size_t)N * sizeof(T), hipMemcpyDeviceToDevice, c->s));
+                    v0 = V;
+                }
+                if (!opened) {
+                    CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
+                    // the first Arnoldi step's first transform is queued behind the
+                    // status read-back, gated on st.active (0 exactly when the solve
+                    // has ended), so the GPU works while the host waits for the status
+                    CHK(poll_mark(c));
+                    if (ahead) launch_precond<T>(g, c->p.precond, c->fast, V, scr, Z, act, c->s, FPC_HEAD);
+                    CHK(poll_spin(c));
+                    if (c->gm_h->outer_done) { final_res = true; break; }
+                    head = ahead;
+                }
+                opened = false;
+            }
             bool one_step = false;             // the cycle stopped after its first Arnoldi step
             for (int j = 0; j < kmax; j++) {
                 T *vj = V + (long)j * ldv, *vj1 = V + (long)(j + 1) * ldv, *zj = Z + (long)j * ldv;
-                {
+                if (!(j == 0 && have_z0)) {
                     Tscope ts(c, TBL_K_PRECOND, precond_bytes(c, sizeof(T)));
                     launch_precond<T>(g, c->p.precond, c->fast, vj, scr, zj, act, c->s,
-                                      (ahead && j == 0) ? FPC_TAIL : FPC_ALL);
+                                      (head && j == 0) ? FPC_TAIL : FPC_ALL);
                 }
+                if (j == 0) head = false;
                 if (j == 0 && fuse_dot) {
                     // first Arnoldi step: the Poisson apply also forms <A z_0, v_0>
                     unsigned nbp;
@@ -1209,7 +1266,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                     CHK(poll_mark(c));
                     if (qa) {
                         launch_fin_cycle(c->gm, c->s, 1);
-                        launch_resid_upd<T>(g, c->pRhs, c->PCorr, Z, c->gm, c->PCalt, V, part_r, c->s, 1);
+                        launch_resid_upd<T>(g, c->pRhs, c->PCorr, Z, c->gm, c->PCalt, V, part_r, c->s, RU_GATED);
                     }
                     CHK(poll_spin(c));
                     if (!c->gm_h->active) {
@@ -1257,6 +1314,19 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         launch_norm2<T>(V, N, part_z, nullptr, c->s);
         launch_fin_start(c->gm, part_r, (int)nbr, part_z, (int)nbv, m == 0 ? 1 : 0, c->s);
         HIPCHK(c, hipGetLastError());
+        if (m == 0 && c->p.precond == TBL_PC_FAST) {
+            // unit step (k_fin_unit): the preconditioned residual of PCorr + V_0
+            // (into W; r holds the residual) ends the solve, or is dropped
+            launch_resid_upd<T>(g, c->pRhs, c->PCorr, V, c->gm, c->PCalt, r, part_r, c->s, RU_UNIT);
+            launch_precond<T>(g, c->p.precond, c->fast, r, scr, W, act, c->s);
+            launch_norm2<T>(W, N, part_z, act, c->s);
+            launch_fin_unit(c->gm, part_r, (int)nbr, part_z, (int)nbv, c->s);
+            HIPCHK(c, hipGetLastError());
+            CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
+            CHK(poll_wait(c));
+            if (c->gm_h->unit_ok) std::swap(c->PCorr, c->PCalt);
+            if (c->gm_h->outer_done) { final_res = true; break; }
+        }
         for (int j = 0; j < kmax; j++) {
             T *vj = V + (long)j * ldv, *vj1 = V + (long)(j + 1) * ldv;
             {

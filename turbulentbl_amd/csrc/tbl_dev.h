@@ -143,6 +143,7 @@ struct GmStatus {
     int cycle, total, nan;
     int conv;                // stopped by the tolerance (not by mmax)
     int zero_rhs;            // true-residual mode: ||pRhs|| = 0, the solution is PCorr = 0
+    int unit_ok, pad_;       // the last tentative unit step (k_fin_unit) was accepted
     double sumav, true_res, sumnor, rho;
 };
 struct GmCtrl {

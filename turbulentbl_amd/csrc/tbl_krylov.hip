@@ -105,31 +105,53 @@ __global__ __launch_bounds__(FB) void k_gm_init(GmCtrl *c, double errtol, double
     }
 }
 
-__global__ __launch_bounds__(FB) void k_fin_bnorm(GmCtrl *c, const double *part, int nb)
+// Start of a cycle in true-residual mode from the residual norm res (one thread)
+__device__ __forceinline__ void start_true(GmCtrl *c, double res)
 {
-    __shared__ double sh[FB / 64];
-    double s = fin_sum<FB>(part, nb, sh);
-    if (threadIdx.x == 0) c->bnorm = sqrt(s);
+    GmStatus &st = c->st;
+    c->inner_ref = res;
+    // stop the cycle at inner_tol, or earlier once the estimated reduction
+    // already brings the true residual below the target (with margin)
+    const double need = res > 0.0 ? 0.3 * c->errtol * c->bnorm / res : 1.0;
+    c->cycle_tol = need > c->inner_tol ? need : c->inner_tol;
+    // pRhs = 0: the exact solution is PCorr = 0, which the host sets (the
+    // relative test could only be met by an exact zero residual)
+    if (c->bnorm == 0.0) st.zero_rhs = 1;
+    const bool done = res <= c->errtol * c->bnorm || res == 0.0 || c->bnorm == 0.0;
+    st.sumav = c->bnorm > 0.0 ? res / c->bnorm : 0.0;
+    st.active = done ? 0 : 1;
+    if (done) { st.outer_done = 1; st.conv = 1; }
+}
+// V_0 with norm rho opens a cycle (all threads; before one thread's stores)
+__device__ __forceinline__ void open_cycle(GmCtrl *c, double rho)
+{
+    for (int q = threadIdx.x; q <= TBL_KMAX_LIMIT + 1; q += FB) c->g[q] = q ? 0.0 : rho;
+    if (threadIdx.x == 0) c->sigma[0] = rho > 0.0 ? 1.0 / rho : 0.0;
 }
 
 // Cycle start: r was formed in double (true residual partials part_r), and
-// V_0 = M^{-1} r (partials part_z of ||V_0||^2).  dnssetbl.f90:536-546.
+// V_0 = M^{-1} r (partials part_z of ||V_0||^2; part_r itself in true-residual
+// mode).  dnssetbl.f90:536-546.
 __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_r, int nb_r,
-                                                 const double *part_z, int nb_z, int first)
+                                                 const double *part_z, int nb_z, int first,
+                                                 const double *part_b)
 {
     __shared__ double sh[FB / 64];
-    double r2 = fin_sum<FB>(part_r, nb_r, sh);
-    double z2 = fin_sum<FB>(part_z, nb_z, sh);
+    __shared__ double rho_s;
+    const double r2 = fin_sum<FB>(part_r, nb_r, sh);
+    const double z2 = part_z == part_r ? r2 : fin_sum<FB>(part_z, nb_z, sh);
+    const double b2 = part_b ? fin_sum<FB>(part_b, nb_r, sh) : 0.0;
+    if (threadIdx.x == 0) rho_s = sqrt(z2);
+    __syncthreads();
+    const double rho = rho_s;
+    open_cycle(c, rho);
     if (threadIdx.x != 0) return;
     GmStatus &st = c->st;
+    if (part_b) c->bnorm = sqrt(b2);
     st.true_res = sqrt(r2);
-    const double rho = sqrt(z2);
     st.cycle += 1;
     st.kit = 0;
     st.rho = rho;
-    for (int q = 0; q <= TBL_KMAX_LIMIT + 1; q++) c->g[q] = 0.0;
-    c->g[0] = rho;
-    c->sigma[0] = rho > 0.0 ? 1.0 / rho : 0.0;
     if (!(rho == rho) || !(st.true_res == st.true_res)) { st.nan = 1; st.active = 0; st.outer_done = 1; return; }
     if (c->mode == GM_MODE_REF) {
         if (first) st.sumnor = rho;
@@ -138,19 +160,55 @@ __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_
         st.active = go ? 1 : 0;
         if (!go) { st.outer_done = 1; st.conv = 1; }
     } else {
-        c->inner_ref = rho;
-        // stop the cycle at inner_tol, or earlier once the estimated reduction
-        // already brings the true residual below the target (with margin)
-        const double need = st.true_res > 0.0 ? 0.3 * c->errtol * c->bnorm / st.true_res : 1.0;
-        c->cycle_tol = need > c->inner_tol ? need : c->inner_tol;
-        // pRhs = 0: the exact solution is PCorr = 0, which the host sets (the
-        // relative test could only be met by an exact zero residual)
-        if (c->bnorm == 0.0) st.zero_rhs = 1;
-        const bool done = st.true_res <= c->errtol * c->bnorm || rho == 0.0 || c->bnorm == 0.0;
-        st.sumav = c->bnorm > 0.0 ? st.true_res / c->bnorm : 0.0;
-        st.active = done ? 0 : 1;
-        if (done) { st.outer_done = 1; st.conv = 1; }
+        start_true(c, rho);
     }
+}
+
+// A cycle whose preconditioner inverts A nearly exactly needs no Arnoldi step:
+// PCorr + z_0 (z_0 = M^{-1} r, the Krylov step with coefficient 1) is formed
+// together with its own residual (k_resid_upd, RU_UNIT), and that residual
+// decides.  Accepted when it meets what the cycle asked for, it counts as the
+// cycle's one step:
+//  * true-residual mode: the residual reached the target, or fell by the
+//    cycle's tolerance; the next cycle is open (its V_0 is that residual);
+//  * the reference's rule: ||M^{-1} r|| (part_z) fell by errtol; the solve
+//    has ended.
+// Otherwise the cycle stays open and the host runs its Arnoldi steps from
+// z_0 as if nothing had been tried.
+__global__ __launch_bounds__(FB) void k_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z,
+                                                int nb_z)
+{
+    __shared__ double sh[FB / 64];
+    __shared__ double res_s;
+    __shared__ int ok_s;
+    GmStatus &st = c->st;
+    if (!st.active) {
+        if (threadIdx.x == 0) st.unit_ok = 0;
+        return;
+    }
+    const bool ref = c->mode == GM_MODE_REF;
+    const double r2 = fin_sum<FB>(part_r, nb_r, sh);
+    const double z2 = ref ? fin_sum<FB>(part_z, nb_z, sh) : 0.0;
+    if (threadIdx.x == 0) {
+        const double res = sqrt(r2), rho = sqrt(z2);
+        bool ok;
+        if (!(res == res) || !(rho == rho)) {
+            st.nan = 1; st.active = 0; st.outer_done = 1;
+            ok = false;
+        } else if (ref) {
+            ok = rho / st.sumnor <= c->errtol;
+            if (ok) { st.sumav = rho / st.sumnor; st.active = 0; st.outer_done = 1; st.conv = 1; }
+        } else {
+            ok = res <= c->errtol * c->bnorm || res <= c->cycle_tol * c->inner_ref;
+            if (ok) { st.cycle += 1; start_true(c, res); }
+        }
+        if (ok) { st.total += 1; st.kit = ref ? 1 : 0; st.rho = ref ? rho : res; st.true_res = res; }
+        st.unit_ok = ok ? 1 : 0;
+        ok_s = ok && !ref;
+        res_s = res;
+    }
+    __syncthreads();
+    if (ok_s) open_cycle(c, res_s);
 }
 
 // d_i = <V_i, z> for i = 0..j, streamed in groups of DG basis vectors.
@@ -386,17 +444,18 @@ void launch_norm2(const T *x, long N, double *part, const int *active, hipStream
 {
     hipLaunchKernelGGL(k_norm2<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, x, N, part, active);
 }
-void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s)
+void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
+                      const double *part_b)
 {
-    hipLaunchKernelGGL(k_fin_start, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, first);
+    hipLaunchKernelGGL(k_fin_start, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, first, part_b);
+}
+void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_fin_unit, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z);
 }
 void launch_gm_init(GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax, int mode, hipStream_t s)
 {
     hipLaunchKernelGGL(k_gm_init, dim3(1), dim3(FB), 0, s, c, errtol, inner_tol, kmax, mmax, mode);
-}
-void launch_fin_bnorm(GmCtrl *c, const double *part, int nb, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_fin_bnorm, dim3(1), dim3(FB), 0, s, c, part, nb);
 }
 template <class T>
 void launch_dots(const T *V, long ldv, int j, long N, const GmCtrl *c, double *part, hipStream_t s)

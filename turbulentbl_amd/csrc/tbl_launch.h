@@ -48,10 +48,13 @@ unsigned launch_poisson(const Geo &g, const T *x, T *out, const int *active, con
 // bpart (optional): block partials of ||pRhs||^2, as many as part
 template <class Tr> void launch_resid(const Geo &g, const double *pRhs, const double *PC, Tr *r, double *part, hipStream_t s,
                                       double *bpart = nullptr);
+// mode: RU_CYCLE the correction of a finished one-step cycle; RU_GATED the
+// same, doing nothing while gc's cycle is active (queued ahead of a host
+// poll); RU_UNIT the tentative unit step PC + z0, doing nothing unless it is
+enum { RU_CYCLE = 0, RU_GATED = 1, RU_UNIT = 2 };
 template <class Tr>
-// gated: does nothing while gc's cycle is active (queued ahead of a host poll)
 void launch_resid_upd(const Geo &g, const double *pRhs, const double *PC, const Tr *Z, const GmCtrl *gc, double *PCn,
-                      Tr *r, double *part, hipStream_t s, int gated = 0);
+                      Tr *r, double *part, hipStream_t s, int mode = RU_CYCLE);
 // part (FPC_*) applies to the fast preconditioner only
 template <class T> void launch_precond(const Geo &g, int pc, const FastPC *fast, const T *r, T *scratch, T *out, const int *active, hipStream_t s,
                                        int part = 0);
@@ -81,9 +84,13 @@ unsigned vec_blocks(long N);
 // x[0..n) = v (a kernel, not a memset: safe inside captured graphs)
 void launch_fill(double *x, double v, long n, hipStream_t s);
 template <class T> void launch_norm2(const T *x, long N, double *part, const int *active, hipStream_t s);
-void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s);
+// part_b (optional): nb_r block partials of ||pRhs||^2 (start of a true-residual solve)
+void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
+                      const double *part_b = nullptr);
+// judges the tentative unit step: residual partials part_r, and the block
+// partials of its preconditioned residual (part_z, reference's stopping rule)
+void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, hipStream_t s);
 void launch_gm_init(GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax, int mode, hipStream_t s);
-void launch_fin_bnorm(GmCtrl *c, const double *part, int nb, hipStream_t s);
 template <class T> void launch_dots(const T *V, long ldv, int j, long N, const GmCtrl *c, double *part, hipStream_t s);
 void launch_fin_dots(GmCtrl *c, const double *part, int nb, int j, hipStream_t s);
 template <class T> void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s);

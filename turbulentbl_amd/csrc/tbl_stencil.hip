@@ -1121,11 +1121,12 @@ __global__ __launch_bounds__(RT_T) void k_resid_upd(Geo g, const double *__restr
                                                   const double *__restrict__ PC, const Tr *__restrict__ Z,
                                                   const GmCtrl *__restrict__ gc, double *__restrict__ PCn,
                                                   Tr *__restrict__ r, double *__restrict__ part, int kchunk,
-                                                  int gated)
+                                                  int mode)
 {
-    // gated: queued before the host knows that the Krylov cycle has ended;
-    // returns at once while the cycle is still active
-    if (gated && gc->st.active) return;
+    // RU_GATED: queued before the host knows that the Krylov cycle has ended;
+    // returns at once while the cycle is still active.  RU_UNIT: the
+    // coefficient is 1; returns at once when the solve has ended
+    if (mode != RU_CYCLE && (gc->st.active != 0) == (mode == RU_GATED)) return;
     __shared__ double sh[RT_T / 64];
     __shared__ double tl[3][TL_N];
     const int nX = g.nX, nY = g.nY, nZ = g.nZ;
@@ -1135,7 +1136,7 @@ __global__ __launch_bounds__(RT_T) void k_resid_upd(Geo g, const double *__restr
     const int i = i0 + (t & 63) + 1;
     const int j = j0 + (t >> 6);
     const int k0 = 1 + blockIdx.z * kchunk, k1 = min(k0 + kchunk, nZ - 1);
-    const double y = gc->st.kit >= 1 ? gc->coef[0] : 0.0;
+    const double y = mode == RU_UNIT ? 1.0 : gc->st.kit >= 1 ? gc->coef[0] : 0.0;
     const bool live = i >= 1 && i <= nX - 2 && j <= nY - 2;
     const int sk = (int)g.sZ;                                    // N < 2^31 (checked at create)
     auto upd = [&](int cc) { return PC[cc] + (double)Z[cc] * y; };
@@ -1729,11 +1730,11 @@ void launch_resid(const Geo &g, const double *pRhs, const double *PC, Tr *r, dou
 
 template <class Tr>
 void launch_resid_upd(const Geo &g, const double *pRhs, const double *PC, const Tr *Z, const GmCtrl *gc, double *PCn,
-                      Tr *r, double *part, hipStream_t s, int gated)
+                      Tr *r, double *part, hipStream_t s, int mode)
 {
     int kc;
     dim3 grid = rgrid(g, &kc);
-    hipLaunchKernelGGL(k_resid_upd<Tr>, grid, dim3(RT_T), 0, s, g, pRhs, PC, Z, gc, PCn, r, part, kc, gated);
+    hipLaunchKernelGGL(k_resid_upd<Tr>, grid, dim3(RT_T), 0, s, g, pRhs, PC, Z, gc, PCn, r, part, kc, mode);
 }
 
 // ----------------------------------------------------------------------------
