@@ -66,3 +66,33 @@ def test_unit_steps_of_the_fast_preconditioner(tbl, precision, rule, errtol, ste
         assert out["iters"] > 1
     else:
         assert out == dict(cycles=1, iters=1, true_res=out["true_res"])
+
+
+# partial 64-column tiles, partial row tiles, one and several k chunks with a
+# shorter last one
+@pytest.mark.parametrize("grid", [(66, 20, 13), (130, 10, 70), (101, 34, 45)])
+def test_adjoint_momentum_tiles(tbl, grid):
+    """the gradient along seeded directions against central differences (the
+    switches replayed); eps 1e-6 of a quadratic map: 1e-5 relative, as over the
+    longer windows"""
+    import torch
+    from turbulentbl_amd.autograd import wall_shear_objective
+    from tests.case_util import load_case
+    g, s = make_case(grid, seed=6)
+    i0, i1 = int(0.6 * (g.nX - 1)) + 1, int(0.9 * (g.nX - 1)) + 1
+    rng = np.random.default_rng(8)
+    base = torch.from_numpy(1e-3 * g.Ue * rng.standard_normal((g.nX, g.nY)))
+
+    def reset(solver):
+        load_case(solver, s)
+
+    with gpu_from_case(g, s) as sv:
+        w = base.clone().requires_grad_(True)
+        wall_shear_objective(w, sv, reset, 3, i0, i1, nsnap=2, freeze=True).backward()
+        for _ in range(2):
+            d = torch.from_numpy(rng.standard_normal((g.nX, g.nY)) * g.Ue)
+            ad, eps = float((w.grad * d).sum()), 1e-6
+            with torch.no_grad():
+                Jp = wall_shear_objective(base + eps * d, sv, reset, 3, i0, i1, freeze=True)
+                Jm = wall_shear_objective(base - eps * d, sv, reset, 3, i0, i1, freeze=True)
+            assert abs(float((Jp - Jm) / (2 * eps)) - ad) <= 1e-5 * abs(ad)

@@ -14,10 +14,13 @@
 // contributions of the forward outputs that read it, so no two threads write
 // the same address and the result is deterministic.  Indices are 0-based;
 // the interior is i in [1,nX-2], j in [1,nY-2], k in [1,nZ-2].
+#include <algorithm>
+
 #include "tbl_dev.h"
 #include "tbl_launch.h"
 
 namespace tbl {
+
 
 __device__ __forceinline__ bool inner(const Geo &g, int i, int j, int k)
 {
@@ -139,16 +142,34 @@ __global__ void k_adj_span(Geo g, double *__restrict__ lam)
     lam[g0] = 0.0;
     lam[g1] = 0.0;
 }
+// What the reversed boundary conditions read of the velocity at the end of a
+// step: u(0,j,k) at E[j + nY k], then w(i,j,0) and w(i,j,1), nX nY values each
+// (adj_end_len values; keeping the whole field took two copies of it a step).
+long adj_end_len(const Geo &g) { return (long)g.nY * g.nZ + 2 * g.sZ; }
+template <class T>
+__global__ void k_adj_save_end(Geo g, const T *__restrict__ U, double *__restrict__ E)
+{
+    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x, nu = (long)g.nY * g.nZ;
+    if (e < nu) E[e] = (double)U[e * g.nX];
+    else if (e < nu + 2 * g.sZ) E[e] = (double)U[2 * g.N + e - nu];
+}
+template <class T> void launch_adj_save_end(const Geo &g, const T *U, double *E, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_adj_save_end<T>, dim3((unsigned)((adj_end_len(g) + 255) / 256)), dim3(256), 0, s, g, U, E);
+}
+template void launch_adj_save_end<double>(const Geo &, const double *, double *, hipStream_t);
+template void launch_adj_save_end<float>(const Geo &, const float *, double *, hipStream_t);
+
 // inflow pressure P(0,j,k) (:773-794); with the inflow plane fixed it depends
 // on U(1), U(2), P(1), P(2) only.  Thread per interior (j, k).
-__global__ void k_adj_pin(Geo g, const double *__restrict__ Uend, double *__restrict__ lamU, double *__restrict__ lamP)
+__global__ void k_adj_pin(Geo g, const double *__restrict__ E, double *__restrict__ lamU, double *__restrict__ lamP)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x + 1, k = blockIdx.y + 1;
     if (j > g.nY - 2 || k > g.nZ - 2) return;
     const long c = lin(g, 0, j, k);
     const double L = lamP[c];
     lamP[c] = 0.0;
-    const double dx = g.dx, Re = g.Re, u1 = Uend[c];
+    const double dx = g.dx, Re = g.Re, u1 = E[j + (long)g.nY * k];
     const double f = 2.0 * dx / 3.0 * L;
     lamU[c + 1] += f * (u1 / dx + 2.0 / (dx * dx * Re));
     lamU[c + 2] += f * (-1.0 / (dx * dx * Re));
@@ -187,7 +208,7 @@ __global__ void k_adj_ptop(Geo g, double *__restrict__ lamW, double *__restrict_
 //   rt3 = (2 df1 w3 - 2 df2 w2 + 2 (df2 - df1) w1)/(df1 df2^2 - df2 df1^2).
 // (1) gather into lamW(.,.,0) over every wall point incl. span ghosts; reads
 // the targets' lamP(.,.,0) without changing it
-__global__ void k_adj_pbot_w0(Geo g, const double *__restrict__ Uend, const double *__restrict__ lamP,
+__global__ void k_adj_pbot_w0(Geo g, const double *__restrict__ E, const double *__restrict__ lamP,
                               double *__restrict__ lamW)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
@@ -201,8 +222,9 @@ __global__ void k_adj_pbot_w0(Geo g, const double *__restrict__ Uend, const doub
     if (tgt(i, j + 1)) acc += lamP[lin(g, i, j + 1, 0)] / (dy * dy * Re);
     acc = -df1 * acc;
     if (tgt(i, j)) {
-        const long c = lin(g, i, j, 0), sk = g.sZ, N = g.N;
-        const double w1 = Uend[2 * N + c], w2 = Uend[2 * N + c + sk];
+        const long c = lin(g, i, j, 0);
+        const double *w = E + (long)g.nY * g.nZ + c;
+        const double w1 = w[0], w2 = w[g.sZ];
         const double den = (df1 * (df2 * df2) - (df2 * (df1 * df1)));
         const double d = -(w2 - 2.0 * w1) / df1 + (-2.0 / (dx * dx) - 2.0 / (dy * dy) + 2.0 * (df2 - df1) / den) / Re;
         acc += -df1 * lamP[c] * d;
@@ -210,17 +232,17 @@ __global__ void k_adj_pbot_w0(Geo g, const double *__restrict__ Uend, const doub
     lamW[lin(g, i, j, 0)] += acc;
 }
 // (2) per target: P(i,j,1) and W(i,j,1..2) terms, then the target is consumed
-__global__ void k_adj_pbot_loc(Geo g, const double *__restrict__ Uend, double *__restrict__ lamP,
+__global__ void k_adj_pbot_loc(Geo g, const double *__restrict__ E, double *__restrict__ lamP,
                                double *__restrict__ lamW)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y + 1;
     if (i > g.nX - 2) return;
     const double df1 = g.df1, df2 = g.df2, Re = g.Re;
-    const long c = lin(g, i, j, 0), sk = g.sZ, N = g.N;
+    const long c = lin(g, i, j, 0), sk = g.sZ;
     const double L = lamP[c];
     lamP[c] = 0.0;
     lamP[c + sk] += L;
-    const double w1 = Uend[2 * N + c];
+    const double w1 = E[(long)g.nY * g.nZ + c];
     const double den = (df1 * (df2 * df2) - (df2 * (df1 * df1)));
     lamW[c + sk] += -df1 * L * (-w1 / df1 + (-2.0 * df2 / den) / Re);
     lamW[c + 2 * sk] += -df1 * L * ((2.0 * df1 / den) / Re);
@@ -341,138 +363,231 @@ __global__ __launch_bounds__(256) void k_adj_div(Geo g, const double *__restrict
 // momentum RHS + Helmholtz boundary data + inflow, reversed
 // (dnssetbl.f90:257-369,371-433)
 // ============================================================================
-// Coefficient with which the convection of a target t reads F at offset o of
-// one direction, given the target's advecting velocity a, branch flags and
-// grid spacing factor inv (invdx, invdy or invdXi).
-__device__ __forceinline__ double conv_coef(int o, double a, bool edge, bool kk, double inv, double c12)
+// One direction of the transposed convection at a point s, from the values at
+// offsets -2..2 (index q = offset + 2): f(p, q) the components, l(p, q) their
+// adjoints (zero off the interior), component P the advecting velocity.
+//  * A target at index q reads s at offset 2 - q, with the coefficient its own
+//    advecting velocity, branch and second-order flag (bit q of `edge`) give:
+//    acc[p] += coefficient l(p, q).
+//  * The derivative of s's own term with respect to its advecting velocity,
+//    summed over the components with their adjoints, is returned.
+// d(q): the spacing of the target's Peclet number; jz(q) scales its coefficient
+// (wall-normal: JacInv of its plane).  The values are read where they are
+// used, a few at a time (the scheduling barriers keep it so): read up front
+// they need 230 registers, one block per CU instead of two.
+template <int P, class Ff, class Fl, class Fd, class Fj>
+__device__ __forceinline__ double conv_adj(Ff f, Fl l, Fd d, Fj jz, unsigned edge, double Re, double inv, double c12,
+                                           double (&acc)[3])
 {
-    if (edge) return (o == 1) ? a * 0.5 * inv : (o == -1) ? -a * 0.5 * inv : 0.0;
-    const double wc = (o == -2) ? 1.0 : (o == -1) ? -8.0 : (o == 1) ? 8.0 : (o == 2) ? -1.0 : 0.0;
-    double v = a * wc * (c12 * inv);
-    if (kk) {
-        const double w4 = (o == -2 || o == 2) ? 1.0 : (o == -1 || o == 1) ? -4.0 : 6.0;
-        v += fabs(a) * w4 * (0.25 * inv);
+    const double ci = c12 * inv, qi = 0.25 * inv, hi = 0.5 * inv;
+    constexpr double wc[5] = {-1.0, 8.0, 0.0, -8.0, 1.0}, w4[5] = {1.0, -4.0, 6.0, -4.0, 1.0};   // at offset 2 - q
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        const double a = f(P, q);
+        const double B = fabs(Re * a * d(q)) > 2.0 ? fabs(a) * qi : 0.0;
+        const double full = __builtin_fma(w4[q], B, wc[q] * (a * ci));
+        const double half = q == 1 ? a * hi : q == 3 ? -(a * hi) : 0.0;
+        const double cf = ((edge >> q) & 1 ? half : full) * jz(q);
+#pragma unroll
+        for (int p = 0; p < 3; p++) acc[p] = __builtin_fma(cf, l(p, q), acc[p]);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    return v;
-}
-// derivative of one direction's term with respect to the advecting velocity a,
-// given the five stencil values f[-2..2] (f[0] at index 2)
-__device__ __forceinline__ double conv_dadv(const double *f, double a, bool edge, bool kk, double inv, double c12)
-{
-    if (edge) return (f[3] - f[1]) * 0.5 * inv;
-    double v = (f[0] - 8.0 * f[1] + 8.0 * f[3] - f[4]) * (c12 * inv);
-    if (kk) v += sgn(a) * (f[4] - 4.0 * f[3] + 6.0 * f[2] - 4.0 * f[1] + f[0]) * (0.25 * inv);
-    return v;
+    double E = 0.0, M = 0.0, D = 0.0;
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        const double lc = l(p, 2), f0 = f(p, 0), f1 = f(p, 1), f3 = f(p, 3), f4 = f(p, 4);
+        E = __builtin_fma(lc, f3 - f1, E);
+        M = __builtin_fma(lc, f0 - f4, M);
+        D = __builtin_fma(lc, __builtin_fma(-4.0, f3 + f1, __builtin_fma(6.0, f(p, 2), f4 + f0)), D);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const double a = f(P, 2);
+    const double sk = fabs(Re * a * d(2)) > 2.0 ? sgn(a) * qi : 0.0;
+    return ((edge >> 2) & 1 ? hi * E : __builtin_fma(sk, D, ci * __builtin_fma(8.0, E, M))) * jz(2);
 }
 
-// Thread per point s.  U is the step's linearisation point (after the inflow
-// overwrite), lamQ the adjoint of Q (interior, zero elsewhere), lamU the
-// adjoint of the Helmholtz output on entry.  On exit lamU holds the adjoint of
-// the step's input velocity; lamP receives -dt Gp^T lamQ.
-__global__ __launch_bounds__(256) void k_adj_mom(Geo g, const double *__restrict__ U, const double *__restrict__ lamQ,
-                                                double *__restrict__ lamU, double *__restrict__ lamP)
+// U is the step's linearisation point (after the inflow overwrite), lamQ the
+// adjoint of Q (interior, zero elsewhere), lamU the adjoint of the Helmholtz
+// output on entry.  On exit lamU holds the adjoint of the step's input
+// velocity; lamP receives -dt Gp^T lamQ.  The span ghost rows pass through and
+// are not visited.
+//
+// A block of 64 x AM_TJ columns marches a chunk of k planes.  The planes
+// k-2..k+2 of U and lamQ live in register queues; plane k of the six fields,
+// with its two-point halo (periodic span rows, streamwise columns clamped to
+// the faces, where lamQ is zero), is staged in LDS (two buffers by plane
+// parity, one LDS-only barrier a plane), so a thread loads each plane's six
+// centre values and at most one halo element per field, a plane before they
+// are used.  A thread per point that read its 100 stencil values through L1
+// and L2 spent its time waiting for them, and so did a k march that took only
+// the wall-normal ones from registers.  At 1024x192x160 (FP32 states) these
+// took 2.22 and 1.87 ms, this one 1.04 ms (256x64x96 FP64: 91, 121 and 54 us);
+// 0.50 ms is the field traffic at a copy's rate.
+// T: storage type of U (mixed contexts keep FP32 states; the arithmetic and
+// the adjoint are FP64).
+#define AM_TJ 8
+#define AM_W 68
+#define AM_SINK (AM_W * (AM_TJ + 4))       // tile slot of threads and elements outside the field
+#define AM_F (AM_SINK + 2)
+#define AM_KMAX 32
+template <class T>
+__global__ __launch_bounds__(64 * AM_TJ) __attribute__((amdgpu_waves_per_eu(3)))
+void k_adj_mom(Geo g, const T *__restrict__ U, const double *__restrict__ lamQ, double *__restrict__ lamU,
+               double *__restrict__ lamP, int kchunk, unsigned nbx, unsigned nby, unsigned nbz)
 {
-    ALL3_IDX
+    __shared__ T tu[2][3][AM_F];
+    __shared__ double tq[2][3][AM_F];
+    __shared__ double sz[2][AM_KMAX + 4];                         // dz3, JacInv of the planes k0-2 .. (0: no target)
+    const unsigned L = xcd_remap(blockIdx.x, nbx * nby * nbz);
+    const unsigned bx = L % nbx, by = (L / nbx) % nby, bz = L / (nbx * nby);
     const int nX = g.nX, nY = g.nY, nZ = g.nZ;
-    const long N = g.N, sk = g.sZ, c = lin(g, i, j, k);
+    const int t = threadIdx.x, lx = t & 63, ly = t >> 6;
+    const int i0 = bx * 64, j0 = by * AM_TJ + 1;
+    const int ti = min(64, nX - i0), tj = min(AM_TJ, nY - 1 - j0);    // tile columns and rows inside the field
+    const bool live = lx < ti && ly < tj;
+    const int i = i0 + min(lx, ti - 1), j = j0 + min(ly, tj - 1);
+    const int k0 = (int)bz * kchunk, k1 = min(k0 + kchunk, nZ);
+    const int sk = (int)g.sZ, c0 = i + nX * j;                   // 3N < 2^31 (checked at create)
+    const long N = g.N;
     const double dt = g.dt, Re = g.Re, c12 = g.c12, h = g.dt / g.Re;
-    const double *Uu = U, *Uv = U + N, *Uw = U + 2 * N;
-    const bool si = inner(g, i, j, k);
-    double out[3];
-    // base: the Helmholtz solve overwrote the interior (its input adjoint is
-    // lamQ through Q's U term); faces pass through and feed the Helmholtz
-    // right-hand side h B u(face)
-    for (int p = 0; p < 3; p++) {
-        const double *lq = lamQ + p * N;
-        if (si) {
-            out[p] = lq[c];
-        } else {
-            double o = lamU[p * N + c];
-            if (j >= 1 && j <= nY - 2 && k >= 1 && k <= nZ - 2) {
-                if (i == 0 && nX - 2 >= 1) o += h * g.Aw * lq[c + 1];
-                if (i == nX - 1) o += h * g.Ae * lq[c - 1];
+    const bool in_i = i >= 1 && i <= nX - 2;
+    if (t < kchunk + 4) {
+        const int kk = k0 - 2 + t;
+        const bool ok = kk >= 1 && kk <= nZ - 2;
+        sz[0][t] = ok ? g.x3[kk + 1] - g.x3[kk] : 0.0;
+        sz[1][t] = ok ? g.JacInv[kk] : 0.0;
+    }
+    // second-order rows: bit q for the target at offset q - 2
+    unsigned ex = 0, ey = 0;
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        const int tx = i + q - 2, ty = j + q - 2;
+        if (tx <= 1 || tx >= nX - 2) ex |= 1u << q;
+        if (ty == 1 || ty == nY - 2 || ty == nY - 1 || ty == 0) ey |= 1u << q;   // rows 0 and nY-1 stand for nY-2 and 1
+    }
+    // the thread's tile slot and its halo element (at most one per field)
+    const int cslot = live ? (2 + ly) * AM_W + 2 + lx : AM_SINK;
+    int hslot = AM_SINK, hoff = c0;
+    {
+        const int n = nY - 2;
+        if (t < 256) {
+            const int hr = t >> 6, hc = t & 63;
+            const int v = hr < 2 ? j0 - 2 + hr : j0 + tj + hr - 2;
+            if (hc < ti) {
+                hslot = (hr < 2 ? hr : tj + hr) * AM_W + 2 + hc;
+                hoff = ((((v - 1) % n + n) % n) + 1) * nX + i0 + hc;
             }
-            if (i >= 1 && i <= nX - 2 && j >= 1 && j <= nY - 2) {
-                if (k == 0) o += h * g.Ab[1] * lq[c + sk];
-                if (k == nZ - 1) o += h * g.At[nZ - 2] * lq[c - sk];
+        } else if (t < 256 + 4 * AM_TJ) {
+            const int hr = (t - 256) >> 2, hc = (t - 256) & 3;
+            const int ii = hc < 2 ? i0 - 2 + hc : i0 + ti + hc - 2;
+            if (hr < tj) {
+                hslot = (2 + hr) * AM_W + (hc < 2 ? hc : ti + hc);
+                hoff = (j0 + hr) * nX + min(max(ii, 0), nX - 1);
             }
-            out[p] = o;
         }
     }
-    // stencil part of the convection: targets t in the x, y, z stencils of s
-    double gp = 0.0;                  // -dt Gp^T lamQ at s
-    // x direction
-    if (j >= 1 && j <= nY - 2 && k >= 1 && k <= nZ - 2) {
-        for (int o = -2; o <= 2; o++) {
-            const int ti = i - o;     // target reads F(ti + o) = F(s)
-            if (ti < 1 || ti > nX - 2) continue;
-            const long t = c - o;
-            const double a = Uu[t];
-            const bool edge = (ti <= 1 || ti >= nX - 2);
-            const bool kk = fabs(Re * a * g.dx) > 2.0;
-            const double cf = conv_coef(o, a, edge, kk, g.invdx, c12);
-            for (int p = 0; p < 3; p++) out[p] += -dt * cf * lamQ[p * N + t];
-        }
-        if (i - 1 >= 1 && i - 1 <= nX - 2) gp += 0.5 * g.invdx * lamQ[c - 1];
-        if (i + 1 >= 1 && i + 1 <= nX - 2) gp -= 0.5 * g.invdx * lamQ[c + 1];
-    }
-    // y direction (periodic tables: the target whose jp_o neighbour is j)
-    if (si) {
-        const int tj[5] = {jp2_of(j, nY), jp1_of(j, nY), j, jm1_of(j, nY), jm2_of(j, nY)};   // o = -2..2
-        for (int q = 0; q < 5; q++) {
-            const int o = q - 2;
-            const long t = lin(g, i, tj[q], k);
-            const double a = Uv[t];
-            const bool edge = (tj[q] == 1 || tj[q] == nY - 2);
-            const bool kk = fabs(Re * a * g.dy) > 2.0;
-            const double cf = conv_coef(o, a, edge, kk, g.invdy, c12);
-            for (int p = 0; p < 3; p++) out[p] += -dt * cf * lamQ[p * N + t];
-        }
-        gp += 0.5 * g.invdy * (lamQ[N + lin(g, i, jm1_of(j, nY), k)] - lamQ[N + lin(g, i, jp1_of(j, nY), k)]);
-    }
-    // z direction (the term is scaled by JacInv of the target)
-    if (i >= 1 && i <= nX - 2 && j >= 1 && j <= nY - 2) {
-        for (int o = -2; o <= 2; o++) {
-            const int tk = k - o;
-            if (tk < 1 || tk > nZ - 2) continue;
-            const long t = c - (long)o * sk;
-            const double a = Uw[t];
-            const bool edge = (tk <= 1 || tk >= nZ - 2);
-            const bool kk = fabs(Re * a * (g.x3[tk + 1] - g.x3[tk])) > 2.0;
-            const double cf = conv_coef(o, a, edge, kk, g.invdXi, c12) * g.JacInv[tk];
-            for (int p = 0; p < 3; p++) out[p] += -dt * cf * lamQ[p * N + t];
-        }
-        if (k - 1 >= 1 && k - 1 <= nZ - 2) gp += 0.5 * g.invdXi * g.JacInv[k - 1] * lamQ[2 * N + c - sk];
-        if (k + 1 >= 1 && k + 1 <= nZ - 2) gp -= 0.5 * g.invdXi * g.JacInv[k + 1] * lamQ[2 * N + c + sk];
-    }
-    // advecting-velocity part at s itself
-    if (si) {
-        const double a = Uu[c], b = Uv[c], w = Uw[c];
-        const bool xe = (i <= 1 || i >= nX - 2), ye = (j == 1 || j == nY - 2), ze = (k <= 1 || k >= nZ - 2);
-        const bool xk = fabs(Re * a * g.dx) > 2.0, yk = fabs(Re * b * g.dy) > 2.0;
-        const bool zk = fabs(Re * w * (g.x3[k + 1] - g.x3[k])) > 2.0;
-        const long cy[5] = {lin(g, i, jm2_of(j, nY), k), lin(g, i, jm1_of(j, nY), k), c, lin(g, i, jp1_of(j, nY), k),
-                            lin(g, i, jp2_of(j, nY), k)};
-        double du = 0.0, dv = 0.0, dw = 0.0;
+    auto kp = [&](int kk) { return sk * max(0, min(kk, nZ - 1)); };
+    // queues before step k's shift: planes k-3..k+1; then the loads in flight:
+    // centre values of plane k+2, halo values of plane k
+    double zU[3][5], zL[3][5], pl[3], hl[3];
+    T pu[3], hu[3];
+#pragma unroll
+    for (int q = 1; q < 5; q++) {
+        const int o = c0 + kp(k0 - 3 + q);
+#pragma unroll
         for (int p = 0; p < 3; p++) {
-            const double *F = U + p * N;
-            const double ap = -dt * lamQ[p * N + c];
-            double f[5];
-            for (int q = 0; q < 5; q++) f[q] = (xe && (q == 0 || q == 4)) ? 0.0 : F[c + (q - 2)];
-            du += ap * conv_dadv(f, a, xe, xk, g.invdx, c12);
-            for (int q = 0; q < 5; q++) f[q] = (ye && (q == 0 || q == 4)) ? 0.0 : F[cy[q]];
-            dv += ap * conv_dadv(f, b, ye, yk, g.invdy, c12);
-            for (int q = 0; q < 5; q++) f[q] = (ze && (q == 0 || q == 4)) ? 0.0 : F[c + (long)(q - 2) * sk];
-            dw += ap * conv_dadv(f, w, ze, zk, g.invdXi, c12) * g.JacInv[k];
+            zU[p][q] = (double)U[p * N + o];
+            zL[p][q] = lamQ[p * N + o];
         }
-        out[0] += du;
-        out[1] += dv;
-        out[2] += dw;
     }
-    // the inflow plane is overwritten by the (frozen) recycling inflow
-    if (i == 0 && j >= 1 && j <= nY - 2 && k >= 1 && k <= nZ - 2) out[0] = out[1] = out[2] = 0.0;
-    for (int p = 0; p < 3; p++) lamU[p * N + c] = out[p];
-    lamP[c] += -dt * gp;
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        pu[p] = U[p * N + c0 + kp(k0 + 2)];
+        pl[p] = lamQ[p * N + c0 + kp(k0 + 2)];
+        hu[p] = U[p * N + hoff + kp(k0)];
+        hl[p] = lamQ[p * N + hoff + kp(k0)];
+    }
+    const int a0 = (2 + min(ly, tj - 1)) * AM_W + 2 + min(lx, ti - 1);
+    for (int k = k0; k < k1; k++) {
+        const int b = k & 1, c = c0 + sk * k;
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                zU[p][q] = zU[p][q + 1];
+                zL[p][q] = zL[p][q + 1];
+            }
+            zU[p][4] = (double)pu[p];
+            zL[p][4] = pl[p];
+            tu[b][p][cslot] = (T)zU[p][2];
+            tq[b][p][cslot] = zL[p][2];
+            tu[b][p][hslot] = hu[p];
+            tq[b][p][hslot] = hl[p];
+        }
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            pu[p] = U[p * N + c0 + kp(k + 3)];
+            pl[p] = lamQ[p * N + c0 + kp(k + 3)];
+            hu[p] = U[p * N + hoff + kp(k + 1)];
+            hl[p] = lamQ[p * N + hoff + kp(k + 1)];
+        }
+        const double lp = lamP[c];
+        lds_barrier();
+        const bool in_k = k >= 1 && k <= nZ - 2, si = in_i && in_k;
+        double acc[3] = {0.0, 0.0, 0.0}, gp = 0.0, adv[3] = {0.0, 0.0, 0.0};
+        auto one = [](int) { return 1.0; };
+        __builtin_amdgcn_sched_barrier(0);
+        if (in_k) {                                              // uniform over the block
+            auto fx = [&](int p, int q) { return q == 2 ? zU[p][2] : (double)tu[b][p][a0 + q - 2]; };
+            auto lqx = [&](int p, int q) { return q == 2 ? zL[p][2] : tq[b][p][a0 + q - 2]; };
+            adv[0] = conv_adj<0>(fx, lqx, [&](int) { return g.dx; }, one, ex, Re, g.invdx, c12, acc);
+            gp = 0.5 * g.invdx * (lqx(0, 1) - lqx(0, 3));
+            auto fy = [&](int p, int q) { return q == 2 ? zU[p][2] : (double)tu[b][p][a0 + (q - 2) * AM_W]; };
+            auto lqy = [&](int p, int q) { return q == 2 ? zL[p][2] : tq[b][p][a0 + (q - 2) * AM_W]; };
+            adv[1] = conv_adj<1>(fy, lqy, [&](int) { return g.dy; }, one, ey, Re, g.invdy, c12, acc);   // l = 0 in the face columns
+            gp += 0.5 * g.invdy * (lqy(1, 1) - lqy(1, 3));
+        }
+        // wall-normal (targets off the interior have lamQ = 0 and JacInv = 0 here)
+        {
+            unsigned ez = 0;
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+                if (k + q - 2 <= 1 || k + q - 2 >= nZ - 2) ez |= 1u << q;
+            auto jz = [&](int q) { return sz[1][k - k0 + q]; };
+            adv[2] = conv_adj<2>([&](int p, int q) { return zU[p][q]; }, [&](int p, int q) { return zL[p][q]; },
+                                 [&](int q) { return sz[0][k - k0 + q]; }, jz, ez, Re, g.invdXi, c12, acc);
+            gp += 0.5 * g.invdXi * (jz(1) * zL[2][1] - jz(3) * zL[2][3]);
+        }
+        double out[3];
+        // base: the Helmholtz solve overwrote the interior (its input adjoint is
+        // lamQ through Q's U term); faces pass through and feed the Helmholtz
+        // right-hand side h B u(face)
+        if (si) {
+#pragma unroll
+            for (int p = 0; p < 3; p++) out[p] = __builtin_fma(-dt, acc[p] + adv[p], zL[p][2]);
+        } else {
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                double o = lamU[p * N + c];
+                if (in_k) {
+                    if (i == 0) o += h * g.Aw * tq[b][p][a0 + 1];
+                    if (i == nX - 1) o += h * g.Ae * tq[b][p][a0 - 1];
+                }
+                if (in_i) {
+                    if (k == 0) o += h * g.Ab[1] * zL[p][3];
+                    if (k == nZ - 1) o += h * g.At[nZ - 2] * zL[p][1];
+                }
+                out[p] = __builtin_fma(-dt, acc[p], o);
+                // the inflow plane is overwritten by the (frozen) recycling inflow
+                if (i == 0 && in_k) out[p] = 0.0;
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int p = 0; p < 3; p++) lamU[p * N + c] = out[p];
+            lamP[c] = lp - dt * gp;
+        }
+    }
 }
 
 // J += cJ * sum_{i in [i0,i1]} tau(i), one thread, fixed order
@@ -524,17 +639,17 @@ void launch_adj_tau(const Geo &g, double *lamU, int i0, int i1, double cJ, hipSt
     hipLaunchKernelGGL(k_adj_tau, dim3((g.nX + 255) / 256, g.nY - 2), dim3(256), 0, s, g, lamU, i0, i1, cJ);
 }
 // pressure then velocity boundary conditions, reversed; grad += adjoint of wall_w
-void launch_adj_bcs(const Geo &g, const double *Uend, double *lamU, double *lamP, double *grad, hipStream_t s)
+void launch_adj_bcs(const Geo &g, const double *E, double *lamU, double *lamP, double *grad, hipStream_t s)
 {
     const long N = g.N;
     double *lamW = lamU + 2 * N;
     const dim3 b256(256);
     hipLaunchKernelGGL(k_adj_span, dim3((g.nX + 255) / 256, g.nZ), b256, 0, s, g, lamP);
-    hipLaunchKernelGGL(k_adj_pin, dim3((g.nY - 2 + 255) / 256, g.nZ - 2), b256, 0, s, g, Uend, lamU, lamP);
+    hipLaunchKernelGGL(k_adj_pin, dim3((g.nY - 2 + 255) / 256, g.nZ - 2), b256, 0, s, g, E, lamU, lamP);
     hipLaunchKernelGGL(k_adj_pout, dim3((g.nY - 2 + 255) / 256, g.nZ - 2), b256, 0, s, g, lamU, lamP);
     hipLaunchKernelGGL(k_adj_ptop, dim3((g.nX - 2 + 255) / 256, g.nY - 2), b256, 0, s, g, lamW, lamP);
-    hipLaunchKernelGGL(k_adj_pbot_w0, dim3((g.nX + 255) / 256, g.nY), b256, 0, s, g, Uend, (const double *)lamP, lamW);
-    hipLaunchKernelGGL(k_adj_pbot_loc, dim3((g.nX - 2 + 255) / 256, g.nY - 2), b256, 0, s, g, Uend, lamP, lamW);
+    hipLaunchKernelGGL(k_adj_pbot_w0, dim3((g.nX + 255) / 256, g.nY), b256, 0, s, g, E, (const double *)lamP, lamW);
+    hipLaunchKernelGGL(k_adj_pbot_loc, dim3((g.nX - 2 + 255) / 256, g.nY - 2), b256, 0, s, g, E, lamP, lamW);
     for (int p = 0; p < 3; p++) {
         double *l = lamU + p * N;
         hipLaunchKernelGGL(k_adj_span, dim3((g.nX + 255) / 256, g.nZ), b256, 0, s, g, l);
@@ -552,9 +667,24 @@ void launch_adj_div(const Geo &g, const double *lamB, double *lamU, hipStream_t 
 {
     hipLaunchKernelGGL(k_adj_div, all3(g), dim3(256), 0, s, g, lamB, lamU);
 }
-void launch_adj_mom(const Geo &g, const double *U, const double *lamQ, double *lamU, double *lamP, hipStream_t s)
+// planes per block of k_adj_mom: the chunk with the least (rounds of blocks
+// over the 256 CUs, one block of 8 waves each at 156 registers; 6 rows a block
+// and two blocks were 1-2 % slower, 128 registers spill) x (planes + 4 queue
+// planes), at most AM_KMAX
+template <class T>
+void launch_adj_mom(const Geo &g, const T *U, const double *lamQ, double *lamU, double *lamP, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_adj_mom, all3(g), dim3(256), 0, s, g, U, lamQ, lamU, lamP);
+    const unsigned nbx = (g.nX + 63) / 64, nby = (g.nY - 2 + AM_TJ - 1) / AM_TJ;
+    int kc = 1;
+    long best = -1;
+    for (int q = AM_KMAX; q >= 1; q--) {
+        const long cost = ((long)nbx * nby * ((g.nZ + q - 1) / q) + 255) / 256 * (q + 4);
+        if (best < 0 || cost < best) { best = cost; kc = q; }
+    }
+    const unsigned nbz = (g.nZ + kc - 1) / kc;
+    hipLaunchKernelGGL(k_adj_mom<T>, dim3(nbx * nby * nbz), dim3(64 * AM_TJ), 0, s, g, U, lamQ, lamU, lamP, kc, nbx, nby, nbz);
 }
+template void launch_adj_mom<double>(const Geo &, const double *, const double *, double *, double *, hipStream_t);
+template void launch_adj_mom<float>(const Geo &, const float *, const double *, double *, double *, hipStream_t);
 
 }  // namespace tbl

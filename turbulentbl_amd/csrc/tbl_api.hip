@@ -1647,11 +1647,11 @@ extern "C" int tbl_step(tbl_ctx *c, int nsteps, tbl_diag *diag)
 // Work buffers of one adjoint window (allocated per call).
 struct AdjWin {
     double *lamU = nullptr, *lamP = nullptr, *lamQ = nullptr, *lamPhi = nullptr, *lamB = nullptr;
-    double *rhs = nullptr, *r = nullptr, *d = nullptr, *Uend = nullptr, *Utmp = nullptr, *grad = nullptr;
+    double *rhs = nullptr, *r = nullptr, *d = nullptr, *grad = nullptr;
+    float *rf = nullptr, *df = nullptr;  // mixed contexts: FP32 residual and correction of the transposed solves
+    double *E = nullptr, *Enew = nullptr;   // end-of-step boundary values (launch_adj_save_end): of this step, of the one before
     double *Jd = nullptr;
     char *snapbuf = nullptr;             // nslots states: Ut, Press in the storage type, PCorr in double
-    double *Ud = nullptr;                // mixed contexts: the FP64 copy of the linearisation velocity
-    float *rf = nullptr, *df = nullptr;  // mixed contexts: FP32 residual and correction of the transposed solves
     size_t slot_bytes = 0;
     int nslots = 0;
     std::vector<int> sn, sc;
@@ -1664,7 +1664,7 @@ struct AdjWin {
 };
 static void adj_free(AdjWin &A)
 {
-    void *p[] = {A.lamU, A.lamP, A.lamQ, A.lamPhi, A.lamB, A.rhs, A.r, A.d, A.Uend, A.Utmp, A.grad, A.Jd, A.snapbuf, A.Ud, A.rf, A.df};
+    void *p[] = {A.lamU, A.lamP, A.lamQ, A.lamPhi, A.lamB, A.rhs, A.r, A.d, A.E, A.Enew, A.grad, A.Jd, A.snapbuf, A.rf, A.df};
     for (void *q : p)
         if (q) hipFree(q);
 }
@@ -1773,26 +1773,23 @@ static int solve_T(tbl_ctx *c, AdjWin &A, const double *b, double *x, double alp
     return 0;
 }
 // adjoint of step n: on entry the fields hold the state after step n-1,
-// A.Uend the velocity after step n, A.lamU / A.lamP the adjoint of the state
-// after step n; on exit they hold the adjoint of the state after step n-1
-// (including dJ_{n-1}/dU) and A.Uend the velocity after step n-1.
-// In a mixed context the states are FP32; the adjoint kernels read them
-// converted to double (A.Ud, A.Uend), so the adjoint is accumulated in FP64
-// about the mixed-precision trajectory.
+// A.E the boundary values of the velocity after step n, A.lamU / A.lamP the
+// adjoint of the state after step n; on exit they hold the adjoint of the
+// state after step n-1 (including dJ_{n-1}/dU) and A.E the boundary values of
+// the velocity after step n-1.
+// In a mixed context the states are FP32; the adjoint kernels convert what
+// they read to double, so the adjoint is accumulated in FP64 about the
+// mixed-precision trajectory.
 static int adj_step(tbl_ctx *c, AdjWin &A, int n)
 {
     const Geo &g = c->g;
     const size_t N = (size_t)g.N;
     const double h = c->p.dt / c->p.Re;
-    HIPCHK(c, hipMemcpyAsync(A.Utmp, c->Ut, 3 * N * c->es, hipMemcpyDeviceToDevice, c->s));
+    if (c->mixed) launch_adj_save_end<float>(g, F<float>(c->Ut), A.Enew, c->s);
+    else launch_adj_save_end<double>(g, F<double>(c->Ut), A.Enew, c->s);
     CHK(tbl_begin_step(c));
     CHK(tbl_recycle_inflow(c));               // linearisation point of the convection
-    const double *Ulin = (const double *)c->Ut;
-    if (c->mixed) {
-        launch_convert<double, float>((const float *)c->Ut, A.Ud, 3 * (long)N, c->s);
-        Ulin = A.Ud;
-    }
-    launch_adj_bcs(g, A.Uend, A.lamU, A.lamP, A.grad, c->s);
+    launch_adj_bcs(g, A.E, A.lamU, A.lamP, A.grad, c->s);
     launch_adj_proj(g, A.lamU, A.lamP, A.lamPhi, c->s);
     CHK(solve_T(c, A, A.lamPhi, A.lamB, 0.0, 1.0));
     launch_adj_div(g, A.lamB, A.lamU, c->s);
@@ -1800,9 +1797,9 @@ static int adj_step(tbl_ctx *c, AdjWin &A, int n)
         launch_copy_interior(g, A.lamU + p * N, A.rhs, c->s);
         CHK(solve_T(c, A, A.rhs, A.lamQ + p * N, 1.0, -h));
     }
-    launch_adj_mom(g, Ulin, A.lamQ, A.lamU, A.lamP, c->s);
-    if (c->mixed) launch_convert<double, float>((const float *)A.Utmp, A.Uend, 3 * (long)N, c->s);
-    else HIPCHK(c, hipMemcpyAsync(A.Uend, A.Utmp, 3 * N * 8, hipMemcpyDeviceToDevice, c->s));
+    if (c->mixed) launch_adj_mom<float>(g, F<float>(c->Ut), A.lamQ, A.lamU, A.lamP, c->s);
+    else launch_adj_mom<double>(g, F<double>(c->Ut), A.lamQ, A.lamU, A.lamP, c->s);
+    std::swap(A.E, A.Enew);
     if (n - 1 >= 1) launch_adj_tau(g, A.lamU, A.i0, A.i1, A.cJ, c->s);
     HIPCHK(c, hipGetLastError());
     A.nadj++;
@@ -1952,16 +1949,15 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         CHK(dalloc(c, &A.rhs, N * 8));
         CHK(dalloc(c, &A.r, N * 8));
         CHK(dalloc(c, &A.d, N * 8));
-        CHK(dalloc(c, &A.Uend, 3 * N * 8));
-        CHK(dalloc(c, &A.Utmp, 3 * N * c->es));
+        CHK(dalloc(c, &A.E, (size_t)adj_end_len(c->g) * 8));
+        CHK(dalloc(c, &A.Enew, (size_t)adj_end_len(c->g) * 8));
         if (c->mixed) {
-            CHK(dalloc(c, &A.Ud, 3 * N * 8));
             CHK(dalloc(c, &A.rf, N * 4));
             CHK(dalloc(c, &A.df, N * 4));
         }
         CHK(dalloc(c, &A.grad, (size_t)p.nX * p.nY * 8));
-        if (c->mixed) launch_convert<double, float>((const float *)c->Ut, A.Uend, 3 * (long)N, c->s);
-        else HIPCHK(c, hipMemcpyAsync(A.Uend, c->Ut, 3 * N * 8, hipMemcpyDeviceToDevice, c->s));
+        if (c->mixed) launch_adj_save_end<float>(c->g, F<float>(c->Ut), A.E, c->s);
+        else launch_adj_save_end<double>(c->g, F<double>(c->Ut), A.E, c->s);
         launch_adj_tau(c->g, A.lamU, A.i0, A.i1, A.cJ, c->s);
         CHK(revolve_top(c, A, 0, o->nsteps, 0, o->nsnap));
         CHK(snap_restore(c, A, fin));

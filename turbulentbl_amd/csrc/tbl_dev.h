@@ -69,6 +69,14 @@ template <class T> __device__ __forceinline__ T bldT(__amdgpu_buffer_rsrc_t r, u
     else return bld(r, voff, soff);
 }
 
+// barrier on LDS data only: the thread's LDS writes are complete, global loads
+// may stay in flight (the "memory" clobber keeps the compiler from moving
+// memory accesses across it)
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Plane loops over a register prefetch ring of R slots are unrolled by R so
 // that each slot lives in fixed registers: IC<S> names the slot of a step,
 // ring_steps runs steps S..R-1 of one ring cycle and ring_tail the steps of

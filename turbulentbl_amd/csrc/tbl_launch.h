@@ -131,10 +131,14 @@ void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha
 void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, float *r, hipStream_t s);
 void launch_copy_interior(const Geo &g, const double *in, double *out, hipStream_t s);
 void launch_adj_tau(const Geo &g, double *lamU, int i0, int i1, double cJ, hipStream_t s);
-void launch_adj_bcs(const Geo &g, const double *Uend, double *lamU, double *lamP, double *grad, hipStream_t s);
+// boundary values of a step's end velocity that the reversed conditions read (E, adj_end_len doubles)
+long adj_end_len(const Geo &g);
+template <class T> void launch_adj_save_end(const Geo &g, const T *U, double *E, hipStream_t s);
+void launch_adj_bcs(const Geo &g, const double *E, double *lamU, double *lamP, double *grad, hipStream_t s);
 void launch_adj_proj(const Geo &g, const double *lamU, const double *lamP, double *lamPhi, hipStream_t s);
 void launch_adj_div(const Geo &g, const double *lamB, double *lamU, hipStream_t s);
-void launch_adj_mom(const Geo &g, const double *U, const double *lamQ, double *lamU, double *lamP, hipStream_t s);
+template <class T>
+void launch_adj_mom(const Geo &g, const T *U, const double *lamQ, double *lamU, double *lamP, hipStream_t s);
 void launch_pc_extrap(double *pc, double *prev, long N, hipStream_t s);
 void launch_tau_acc(const Geo &g, const double *tau, int i0, int i1, double cJ, double *J, hipStream_t s);
 

@@ -214,14 +214,6 @@ void k_momentum_rhs(Geo g, const T *__restrict__ Ut,
 // neighbours never waits for a wall-normal (HBM) load of the same or the
 // previous plane, and the queue shift copies values loaded a plane earlier.
 // ----------------------------------------------------------------------------
-// barrier on LDS data only: the thread's LDS writes are complete, global loads
-// may stay in flight (the "memory" clobber keeps the compiler from moving
-// memory accesses across it)
-__device__ __forceinline__ void lds_barrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // one convection derivative with fused multiply-adds: uc = u c12/h,
 // ua = |u|/(4h) where the Kawamura-Kuwahara form applies (else 0),
 // uh = u/(2h) for the edge form
