@@ -39,6 +39,14 @@ static inline dim3 all3(const Geo &g) { return dim3((g.nX + 63) / 64, (g.nY + 3)
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6);             \
     const int k = blockIdx.z;                                      \
     if (i >= g.nX || j >= g.nY) return;
+// the same over ncomp components (N values apart, nZ plane rows each)
+#define COMP3_IDX                                                  \
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63);            \
+    const int j = blockIdx.y * 4 + (threadIdx.x >> 6);             \
+    const int k = blockIdx.z % g.nZ;                               \
+    const long comp = (long)(blockIdx.z / g.nZ) * g.N;             \
+    if (i >= g.nX || j >= g.nY) return;
+static inline dim3 comp3(const Geo &g, int ncomp) { return dim3((g.nX + 63) / 64, (g.nY + 3) / 4, g.nZ * ncomp); }
 
 // ============================================================================
 // direct Helmholtz solve (forward): residual field and interior update
@@ -49,21 +57,14 @@ template <class T>
 __global__ __launch_bounds__(256) void k_helm_rfield(Geo g, const T *__restrict__ Q, const T *__restrict__ u,
                                                     T *__restrict__ r)
 {
-    ALL3_IDX
+    COMP3_IDX
+    Q += comp; u += comp; r += comp;
     if (!inner(g, i, j, k)) return;
     const long c = lin(g, i, j, k), sk = g.sZ;
     const long cp = lin(g, i, jp1_of(j, g.nY), k), cm = lin(g, i, jm1_of(j, g.nY), k);
     const double rt1 = g.Ae * (double)u[c + 1] + g.Aw * (double)u[c - 1] + g.An * (double)u[cp] + g.As * (double)u[cm];
     const double rt2 = g.At[k] * (double)u[c + sk] + g.Ab[k] * (double)u[c - sk];
     r[c] = (T)((double)Q[c] - (1.0 - g.dt / g.Re * g.Ap[k]) * (double)u[c] + g.dt * (rt1 + rt2) / g.Re);
-}
-template <class T, class Td>
-__global__ __launch_bounds__(256) void k_add_interior(Geo g, T *__restrict__ u, const Td *__restrict__ d)
-{
-    ALL3_IDX
-    if (!inner(g, i, j, k)) return;
-    const long c = lin(g, i, j, k);
-    u[c] = u[c] + (T)d[c];
 }
 
 // ============================================================================
@@ -78,20 +79,14 @@ template <class To>
 __global__ __launch_bounds__(256) void k_opT_res(Geo g, const double *__restrict__ b, const double *__restrict__ x,
                                                  double alpha, double beta, To *__restrict__ r)
 {
-    ALL3_IDX
+    COMP3_IDX
+    b += comp; x += comp; r += comp;
     if (!inner(g, i, j, k)) return;
     const long c = lin(g, i, j, k), sk = g.sZ;
     const long cp = lin(g, i, jp1_of(j, g.nY), k), cm = lin(g, i, jm1_of(j, g.nY), k);
     const double ax = g.Ap[k] * x[c] + g.Aw * x[c + 1] + g.Ae * x[c - 1] + g.As * x[cp] + g.An * x[cm] +
                       g.Ab[k + 1] * x[c + sk] + g.At[k - 1] * x[c - sk];
     r[c] = (To)(b[c] - (alpha * x[c] + beta * ax));
-}
-// out = in on the interior, 0 elsewhere
-__global__ __launch_bounds__(256) void k_copy_interior(Geo g, const double *__restrict__ in, double *__restrict__ out)
-{
-    ALL3_IDX
-    const long c = lin(g, i, j, k);
-    out[c] = inner(g, i, j, k) ? in[c] : 0.0;
 }
 
 // ============================================================================
@@ -607,33 +602,19 @@ void launch_tau_acc(const Geo &g, const double *tau, int i0, int i1, double cJ, 
     hipLaunchKernelGGL(k_tau_acc, dim3(1), dim3(64), 0, s, tau, i0, i1, cJ, J);
 }
 template <class T>
-void launch_helm_rfield(const Geo &g, const T *Q, const T *u, T *r, hipStream_t s)
+void launch_helm_rfield(const Geo &g, const T *Q, const T *u, T *r, int ncomp, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_helm_rfield<T>, all3(g), dim3(256), 0, s, g, Q, u, r);
+    hipLaunchKernelGGL(k_helm_rfield<T>, comp3(g, ncomp), dim3(256), 0, s, g, Q, u, r);
 }
-template <class T, class Td>
-void launch_add_interior(const Geo &g, T *u, const Td *d, hipStream_t s)
+template void launch_helm_rfield<double>(const Geo &, const double *, const double *, double *, int, hipStream_t);
+template void launch_helm_rfield<float>(const Geo &, const float *, const float *, float *, int, hipStream_t);
+template <class To>
+void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, To *r, int ncomp, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_add_interior<T, Td>), all3(g), dim3(256), 0, s, g, u, d);
+    hipLaunchKernelGGL(k_opT_res<To>, comp3(g, ncomp), dim3(256), 0, s, g, b, x, alpha, beta, r);
 }
-template void launch_helm_rfield<double>(const Geo &, const double *, const double *, double *, hipStream_t);
-template void launch_helm_rfield<float>(const Geo &, const float *, const float *, float *, hipStream_t);
-template void launch_add_interior<double, double>(const Geo &, double *, const double *, hipStream_t);
-template void launch_add_interior<float, float>(const Geo &, float *, const float *, hipStream_t);
-template void launch_add_interior<double, float>(const Geo &, double *, const float *, hipStream_t);
-
-void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, double *r, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_opT_res<double>, all3(g), dim3(256), 0, s, g, b, x, alpha, beta, r);
-}
-void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, float *r, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_opT_res<float>, all3(g), dim3(256), 0, s, g, b, x, alpha, beta, r);
-}
-void launch_copy_interior(const Geo &g, const double *in, double *out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_copy_interior, all3(g), dim3(256), 0, s, g, in, out);
-}
+template void launch_opT_res<double>(const Geo &, const double *, const double *, double, double, double *, int, hipStream_t);
+template void launch_opT_res<float>(const Geo &, const double *, const double *, double, double, float *, int, hipStream_t);
 void launch_adj_tau(const Geo &g, double *lamU, int i0, int i1, double cJ, hipStream_t s)
 {
     hipLaunchKernelGGL(k_adj_tau, dim3((g.nX + 255) / 256, g.nY - 2), dim3(256), 0, s, g, lamU, i0, i1, cJ);

@@ -50,6 +50,7 @@ struct tbl_ctx {
     double *PCalt = nullptr;             // second PCorr buffer: the fused update + residual writes it
     int pc_hist = 0;                     // previous solutions available for the extrapolation
     void *V = nullptr, *W = nullptr, *scr = nullptr, *r = nullptr;
+    void *r3 = nullptr;                  // three-component residual of the direct and transposed solves (zero faces)
     void *Z = nullptr;                   // flexible-GMRES preconditioned vectors (true-residual mode)
     long ldv = 0;
     double *part = nullptr;
@@ -520,7 +521,7 @@ extern "C" int tbl_destroy(tbl_ctx *c)
     void *dev[] = {c->mesh, c->Ut, c->Ualt, c->Utold, c->Q, c->Press, c->PCorr, c->pRhs, c->V, c->W, c->scr, c->r, c->Z,
                    c->part, c->gm, c->gs, c->sums, c->avg, c->Wt, c->Ume, c->uf, c->bltkns, c->dstar,
                    c->theta, c->tau, c->tausum, c->taumean, c->cf, c->wall_w, c->scan, c->newk, c->rec, c->guard, c->dd, c->zf, c->br, c->PCprev,
-                   c->PCalt, c->slab, c->halo};
+                   c->PCalt, c->slab, c->halo, c->r3};
     for (void *d : dev)
         if (d) hipFree(d);
     if (c->fast) fastpc_destroy(c->fast);
@@ -918,7 +919,15 @@ extern "C" int tbl_momentum_rhs(tbl_ctx *c)
     return c->mixed ? rhs_impl<float>(c) : rhs_impl<double>(c);
 }
 
-// exact Helmholtz solve per component: u += (I - hA)^{-1} (Q - H u), by fast
+// work of the direct and transposed solves, allocated by the first of them
+static int direct_work(tbl_ctx *c)
+{
+    if (!c->r3) CHK(dalloc(c, &c->r3, 3 * (size_t)c->g.N * c->es));
+    if (fastpc_reserve(c->fast, c->g, solve_batched(c->g, c->mixed) ? 3 : 1, c->s))
+        return fail(c, TBL_EARG, "fast solver: no memory for the solves of three components");
+    return 0;
+}
+// exact Helmholtz solve of the three components: u += (I - hA)^{-1} (Q - H u), by fast
 // diagonalisation; in FP64 twice (one refinement step on the residual).  In
 // FP32 storage once: I - hA is well conditioned (the stretched grid's
 // largest h lambda is about 2), so one FP32 fast solve is already at the
@@ -928,19 +937,22 @@ template <class T> static int helm_direct(tbl_ctx *c, int *sweeps, double *res)
     if (!c->fast) return fail(c, TBL_ESTATE, "direct Helmholtz solve without the fast solver");
     const Geo &g = c->g;
     const long N = g.N;
-    T *r = F<T>(c->r), *d = F<T>(c->scr);
+    CHK(direct_work(c));
+    const int nc = solve_batched(g, c->mixed) ? 3 : 1;         // components per solve
     const double h = c->p.dt / c->p.Re;
     const int passes = sizeof(T) == sizeof(double) ? 2 : 1;
-    launch_zero_faces<T>(g, r, c->s);
-    for (int p = 0; p < 3; p++) {
-        T *u = F<T>(c->Ut) + p * N;
-        const T *q = F<T>(c->Q) + p * N;
+    for (int p = 0; p < 3; p += nc) {
+        FastIO io;
+        io.in = c->r3;
+        io.out = F<T>(c->Ut) + p * N;
+        io.in64 = io.out64 = sizeof(T) == sizeof(double);
+        io.add = 1;
+        io.ncomp = nc;
         for (int it = 0; it < passes; it++) {
-            Tscope ts(c, TBL_K_HELM, 4.0 * (double)N * sizeof(T));
-            launch_helm_rfield<T>(g, q, u, r, c->s);
-            if (run_fastpc_ext<T>(c->fast, g, r, d, nullptr, 1.0, -h, false, c->s))
+            Tscope ts(c, TBL_K_HELM, 4.0 * nc * (double)N * sizeof(T));
+            launch_helm_rfield<T>(g, F<T>(c->Q) + p * N, F<T>(c->Ut) + p * N, F<T>(c->r3), nc, c->s);
+            if (run_fast_solve(c->fast, g, io, nullptr, 1.0, -h, false, c->s))
                 return fail(c, TBL_EARG, "fast solver failure in the direct Helmholtz solve");
-            launch_add_interior<T>(g, u, d, c->s);
         }
     }
     HIPCHK(c, hipGetLastError());
@@ -1647,8 +1659,7 @@ extern "C" int tbl_step(tbl_ctx *c, int nsteps, tbl_diag *diag)
 // Work buffers of one adjoint window (allocated per call).
 struct AdjWin {
     double *lamU = nullptr, *lamP = nullptr, *lamQ = nullptr, *lamPhi = nullptr, *lamB = nullptr;
-    double *rhs = nullptr, *r = nullptr, *d = nullptr, *grad = nullptr;
-    float *rf = nullptr, *df = nullptr;  // mixed contexts: FP32 residual and correction of the transposed solves
+    double *grad = nullptr;
     double *E = nullptr, *Enew = nullptr;   // end-of-step boundary values (launch_adj_save_end): of this step, of the one before
     double *Jd = nullptr;
     char *snapbuf = nullptr;             // nslots states: Ut, Press in the storage type, PCorr in double
@@ -1664,7 +1675,7 @@ struct AdjWin {
 };
 static void adj_free(AdjWin &A)
 {
-    void *p[] = {A.lamU, A.lamP, A.lamQ, A.lamPhi, A.lamB, A.rhs, A.r, A.d, A.E, A.Enew, A.grad, A.Jd, A.snapbuf, A.rf, A.df};
+    void *p[] = {A.lamU, A.lamP, A.lamQ, A.lamPhi, A.lamB, A.E, A.Enew, A.grad, A.Jd, A.snapbuf};
     for (void *q : p)
         if (q) hipFree(q);
 }
@@ -1702,15 +1713,18 @@ static int snap_restore(tbl_ctx *c, AdjWin &A, int slot)
 template <class T> static int ppe_direct(tbl_ctx *c)
 {
     const Geo &g = c->g;
-    T *r = F<T>(c->r), *d = F<T>(c->scr);
+    T *r = F<T>(c->r);                         // its faces stay zero
+    FastIO io;
+    io.in = r;
+    io.out = c->PCorr;
+    io.in64 = sizeof(T) == sizeof(double);
+    io.out64 = io.add = 1;
     launch_zero_faces<double>(g, c->PCorr, c->s);
-    launch_zero_faces<T>(g, r, c->s);
     const int passes = 2;
     for (int it = 0; it < passes; it++) {
         launch_resid<T>(g, c->pRhs, c->PCorr, r, c->part, c->s);
-        if (run_fastpc_ext<T>(c->fast, g, r, d, nullptr, 0.0, 1.0, false, c->s))
+        if (run_fast_solve(c->fast, g, io, nullptr, 0.0, 1.0, false, c->s))
             return fail(c, TBL_EARG, "fast solver failure in the direct pressure solve");
-        launch_add_interior<double, T>(g, c->PCorr, d, c->s);
     }
     HIPCHK(c, hipGetLastError());
     return 0;
@@ -1748,27 +1762,32 @@ static int win_step(tbl_ctx *c, AdjWin &A, bool accJ)
 // M^{-T} the transposed fast solve.  FP64 contexts: the FP64 fast solver,
 // two passes.  Mixed contexts: the FP32 fast solver on the FP64 residual
 // rounded to FP32, also two passes (each gains about the FP32 solver's
-// accuracy, 1e-6), x and the residual accumulated in FP64.  b is zero off the interior;
-// x is written on planes 1..nZ-2 (zero on their face rows).
-static int solve_T(tbl_ctx *c, AdjWin &A, const double *b, double *x, double alpha, double beta)
+// accuracy, 1e-6), x and the residual accumulated in FP64.  Values of b off
+// the interior are not read; x is written on planes 1..nZ-2 (zero on their
+// face rows).  The transforms read b and write and correct x in FP64
+// themselves: copies of b without its faces and in FP32, and the passes that
+// widened and added the result, moved 60 bytes a cell more.
+static int solve_T(tbl_ctx *c, const double *b, double *x, double alpha, double beta, int ncomp)
 {
     const Geo &g = c->g;
-    const FastPC *f = c->fast;
-    if (!c->mixed) {
-        if (run_fastpc_ext<double>(f, g, b, x, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
-        launch_opT_res(g, b, x, alpha, beta, A.r, c->s);
-        if (run_fastpc_ext<double>(f, g, A.r, A.d, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
-        launch_add_interior<double>(g, x, A.d, c->s);
-        return 0;
-    }
-    const long pst = g.sZ, nzp = (long)(g.nZ - 2) * pst;
-    launch_convert<float, double>(b + pst, A.rf + pst, nzp, c->s);
-    if (run_fastpc_ext<float>(f, g, A.rf, A.df, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
-    launch_convert<double, float>(A.df + pst, x + pst, nzp, c->s);
-    for (int it = 1; it < 2; it++) {
-        launch_opT_res(g, b, x, alpha, beta, A.rf, c->s);
-        if (run_fastpc_ext<float>(f, g, A.rf, A.df, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
-        launch_add_interior<double, float>(g, x, A.df, c->s);
+    const int nc = solve_batched(g, c->mixed) ? ncomp : 1;
+    CHK(direct_work(c));
+    for (int p = 0; p < ncomp; p += nc) {
+        const double *bp = b + (long)p * g.N;
+        double *xp = x + (long)p * g.N;
+        FastIO io;
+        io.in = bp;
+        io.out = xp;
+        io.in64 = io.out64 = io.mask = 1;
+        io.ncomp = nc;
+        if (run_fast_solve(c->fast, g, io, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
+        if (c->mixed) launch_opT_res<float>(g, bp, xp, alpha, beta, F<float>(c->r3), nc, c->s);
+        else launch_opT_res<double>(g, bp, xp, alpha, beta, F<double>(c->r3), nc, c->s);
+        io.in = c->r3;
+        io.in64 = !c->mixed;
+        io.mask = 0;
+        io.add = 1;
+        if (run_fast_solve(c->fast, g, io, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
     }
     return 0;
 }
@@ -1791,12 +1810,9 @@ static int adj_step(tbl_ctx *c, AdjWin &A, int n)
     CHK(tbl_recycle_inflow(c));               // linearisation point of the convection
     launch_adj_bcs(g, A.E, A.lamU, A.lamP, A.grad, c->s);
     launch_adj_proj(g, A.lamU, A.lamP, A.lamPhi, c->s);
-    CHK(solve_T(c, A, A.lamPhi, A.lamB, 0.0, 1.0));
+    CHK(solve_T(c, A.lamPhi, A.lamB, 0.0, 1.0, 1));
     launch_adj_div(g, A.lamB, A.lamU, c->s);
-    for (int p = 0; p < 3; p++) {
-        launch_copy_interior(g, A.lamU + p * N, A.rhs, c->s);
-        CHK(solve_T(c, A, A.rhs, A.lamQ + p * N, 1.0, -h));
-    }
+    CHK(solve_T(c, A.lamU, A.lamQ, 1.0, -h, 3));
     if (c->mixed) launch_adj_mom<float>(g, F<float>(c->Ut), A.lamQ, A.lamU, A.lamP, c->s);
     else launch_adj_mom<double>(g, F<double>(c->Ut), A.lamQ, A.lamU, A.lamP, c->s);
     std::swap(A.E, A.Enew);
@@ -1946,15 +1962,8 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         CHK(dalloc(c, &A.lamQ, 3 * N * 8));
         CHK(dalloc(c, &A.lamPhi, N * 8));
         CHK(dalloc(c, &A.lamB, N * 8));
-        CHK(dalloc(c, &A.rhs, N * 8));
-        CHK(dalloc(c, &A.r, N * 8));
-        CHK(dalloc(c, &A.d, N * 8));
         CHK(dalloc(c, &A.E, (size_t)adj_end_len(c->g) * 8));
         CHK(dalloc(c, &A.Enew, (size_t)adj_end_len(c->g) * 8));
-        if (c->mixed) {
-            CHK(dalloc(c, &A.rf, N * 4));
-            CHK(dalloc(c, &A.df, N * 4));
-        }
         CHK(dalloc(c, &A.grad, (size_t)p.nX * p.nY * 8));
         if (c->mixed) launch_adj_save_end<float>(c->g, F<float>(c->Ut), A.E, c->s);
         else launch_adj_save_end<double>(c->g, F<double>(c->Ut), A.E, c->s);

@@ -41,7 +41,8 @@ namespace tbl {
 struct FastPC {
     int nx = 0, ny = 0, nz = 0;                          // interior sizes
     double *ly = nullptr, *lz = nullptr;                 // eigenvalues (full-index arrays)
-    void *t1 = nullptr, *t2 = nullptr;                   // work fields (storage type)
+    void *t1 = nullptr, *t2 = nullptr;                   // work fields (storage type), ncap components each
+    int ncap = 1;
     bool single = false;
     // FP32 storage: the transform matrices split into three bf16 parts in
     // matrix-core fragment order (see k_xform): z forward, y forward, y
@@ -162,11 +163,27 @@ __device__ __forceinline__ void xf_split2(float x0, float x1, unsigned &h, unsig
 #ifndef XF_MAXT
 #define XF_MAXT 8
 #endif
-template <int NT>
-__global__ __launch_bounds__(256) void k_xform(const float *__restrict__ A, float *__restrict__ C,
-                                              const xf_v4u *__restrict__ Bf, int K, int KG, int N, long Mtot, long Mp,
-                                              long bstride, long lda, long ldc, int NTt, int ncb,
-                                              const int *__restrict__ active)
+// Ti: type of A (FP64 operands are rounded to FP32 as they are loaded).
+// out: XO_* -- C in FP32 or FP64, stored or added to (an FP64 field corrected by
+// an FP32 solve needs no pass of its own).
+// mask (nX or 0): the rows are (i, j) points of a plane of nX columns and rows
+// `mask_ny`, and face points are read as zero.
+enum { XO_F32 = 0, XO_F32_ADD = 1, XO_F64 = 2, XO_F64_ADD = 3 };
+struct XMap {              // row map and leading dimensions of a transform
+    long Mtot, Mp, bstride, lda, ldc;
+    int mask, mask_ny;
+};
+__device__ __forceinline__ bool xf_inner(const XMap &x, long in_period)
+{
+    if (!x.mask) return true;
+    const int i = (int)(in_period % x.mask), j = (int)(in_period / x.mask);
+    return i >= 1 && i <= x.mask - 2 && j >= 1 && j <= x.mask_ny - 2;
+}
+// two waves per SIMD: with 8 tiles the accumulators take half the registers
+template <int NT, class Ti>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_xform(const Ti *__restrict__ A, void *Cv,
+                                              const xf_v4u *__restrict__ Bf, int K, int KG, int N, XMap X, int NTt,
+                                              int ncb, int out, const int *__restrict__ active)
 {
     if (active && !*active) return;                          // gated launch of an ended solve
     constexpr int SL = 3 * NT * 64;                          // fragments of one k group
@@ -179,24 +196,25 @@ __global__ __launch_bounds__(256) void k_xform(const float *__restrict__ A, floa
     const long rb = (long)(L / (unsigned)ncb);
     const int nt0 = cb * NT;                                 // first tile of this column block
     const long m = rb * XF_ROWS + wv * 32 + (lane & 31);
-    const bool mok = m < Mtot;
-    const float *Ar = A + (mok ? (m % Mp) + (m / Mp) * bstride : 0);
+    const bool mok = m < X.Mtot, aok = mok && xf_inner(X, m % X.Mp);
+    const long row = mok ? (m % X.Mp) + (m / X.Mp) * X.bstride : 0;
     const int kh = (lane >> 5) * 8;
     xf_v16f acc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) acc[nt] = xf_v16f{};
     // loads are unconditional at in-range addresses, masked after (the
     // padding k >= K and rows m >= Mtot are zeroed at the split, so that
-    // nothing consumes a load before it is needed).  Offsets are 32-bit (the
-    // field holds fewer than 2^30 values, checked at create time):
+    // nothing consumes a load before it is needed).  Offsets are 32-bit (FP32
+    // operands span fewer than 2^30 values, see solve_batched):
     // row + min(k lda, (K-1) lda), with the uniform part k0 lda scalar.
-    const int row32 = (int)(Ar - A), lda32 = (int)lda, khl = kh * lda32, kcap = (K - 1) * lda32;
-    auto ldA = [&](int kgl, float *dst) {
+    const int row32 = (int)row, lda32 = (int)X.lda, khl = kh * lda32, kcap = (K - 1) * lda32;
+    auto ldA = [&](int kgl, Ti *dst) {
         const int s0 = kgl * 16 * lda32;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const unsigned off = (unsigned)(row32 + min(s0 + e * lda32 + khl, kcap));
-            dst[e] = __builtin_nontemporal_load((const float *)((const char *)A + off * 4u));
+            if constexpr (sizeof(Ti) == 4) dst[e] = __builtin_nontemporal_load((const float *)((const char *)A + off * 4u));
+            else dst[e] = __builtin_nontemporal_load(A + off);
         }
     };
     // staged fragment e of a group: part e / (NT 64), tile nt0 + (e / 64) % NT
@@ -219,7 +237,7 @@ __global__ __launch_bounds__(256) void k_xform(const float *__restrict__ A, floa
     // buffer g % 2, then stores the B slice of group g + 1 (loaded one step
     // earlier) into the other buffer.  The group count is padded to even; a
     // padding group is masked to zero at the split.
-    float an[2][8];
+    Ti an[2][8];
     xf_v4u st[2][PT];
     ldA(0, an[0]);
     ldB(0, st[0]);
@@ -235,8 +253,8 @@ __global__ __launch_bounds__(256) void k_xform(const float *__restrict__ A, floa
         for (int p = 0; p < 4; p++) {
             unsigned h, mm, l;
             const int k0 = kg * 16 + kh + 2 * p;
-            xf_split2((mok && k0 < K) ? an[b][2 * p] : 0.0f, (mok && k0 + 1 < K) ? an[b][2 * p + 1] : 0.0f, h, mm,
-                      l);
+            xf_split2((aok && k0 < K) ? (float)an[b][2 * p] : 0.0f, (aok && k0 + 1 < K) ? (float)an[b][2 * p + 1] : 0.0f,
+                      h, mm, l);
             ah[p] = h; am[p] = mm; al[p] = l;
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -276,14 +294,24 @@ __global__ __launch_bounds__(256) void k_xform(const float *__restrict__ A, floa
         step(kg + 1, std::integral_constant<int, 1>{});
     }
     if (mok) {
-        float *Cr = C + (Ar - A);
+        auto store = [&](auto *Cr, auto add) {
+            using To = std::remove_pointer_t<decltype(Cr)>;
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++)
+            for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int n = (nt0 + nt) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (n < N) Cr[(long)n * ldc] = acc[nt][r];
-            }
+                for (int r = 0; r < 16; r++) {
+                    const int n = (nt0 + nt) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    if (n < N) {
+                        To *c = Cr + (long)n * X.ldc;
+                        if constexpr (decltype(add)::value) *c = *c + (To)acc[nt][r];
+                        else *c = (To)acc[nt][r];
+                    }
+                }
+        };
+        if (out == XO_F32) store((float *)Cv + row, std::false_type{});
+        else if (out == XO_F32_ADD) store((float *)Cv + row, std::true_type{});
+        else if (out == XO_F64) store((double *)Cv + row, std::false_type{});
+        else store((double *)Cv + row, std::true_type{});
     }
 }
 
@@ -310,14 +338,15 @@ static std::vector<unsigned short> xform_split(int K, int N, Fn b)
     return out;
 }
 
-static void launch_xform(int K, int N, const unsigned short *Bf, const float *A, float *C, long Mtot, long Mp,
-                         long bstride, long lda, long ldc, hipStream_t s, const int *active = nullptr)
+template <class Ti>
+static void launch_xform(int K, int N, const unsigned short *Bf, const Ti *A, void *C, const XMap &X, hipStream_t s,
+                         const int *active, int out = XO_F32)
 {
     const int KG = (K + 15) / 16, NTt = (N + 31) / 32;
     const int ncb = (NTt + XF_MAXT - 1) / XF_MAXT, NT = (NTt + ncb - 1) / ncb;   // at most XF_MAXT tiles per block
-    const dim3 grid((unsigned)(((Mtot + XF_ROWS - 1) / XF_ROWS) * ncb)), blk(256);
+    const dim3 grid((unsigned)(((X.Mtot + XF_ROWS - 1) / XF_ROWS) * ncb)), blk(256);
     const xf_v4u *B = (const xf_v4u *)Bf;
-#define XF_CASE(q) case q: hipLaunchKernelGGL(k_xform<q>, grid, blk, 0, s, A, C, B, K, KG, N, Mtot, Mp, bstride, lda, ldc, NTt, ncb, active); break;
+#define XF_CASE(q) case q: hipLaunchKernelGGL((k_xform<q, Ti>), grid, blk, 0, s, A, C, B, K, KG, N, X, NTt, ncb, out, active); break;
     switch (NT) {
         XF_CASE(1) XF_CASE(2) XF_CASE(3) XF_CASE(4) XF_CASE(5) XF_CASE(6) XF_CASE(7) XF_CASE(8)
         default: break;
@@ -347,11 +376,10 @@ static void launch_xform(int K, int N, const unsigned short *Bf, const float *A,
 // ----------------------------------------------------------------------------
 typedef double xd_v4d __attribute__((ext_vector_type(4)));
 
-template <int MT, int NT>
-__global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, double *__restrict__ C,
-                                                const double *__restrict__ Bf, int K, int KG, int N, long Mtot,
-                                                long Mp, long bstride, long lda, long ldc, int NTt, int ncb,
-                                                const int *__restrict__ active)
+template <int MT, int NT, bool ADD>
+__global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, double *C,
+                                                const double *__restrict__ Bf, int K, int KG, int N, XMap X, int NTt,
+                                                int ncb, const int *__restrict__ active)
 {
     if (active && !*active) return;                          // gated launch of an ended solve
     __shared__ double sB[2][NT * 256];
@@ -364,15 +392,16 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
     // row offsets (element units; fields hold fewer than 2^31 values), rows
     // past Mtot clamped to the last row: loaded, never stored
     unsigned rowo[MT];
-    bool mok[MT];
+    bool mok[MT], aok[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const long m = rb * (64 * MT) + wv * (16 * MT) + mt * 16 + (lane & 15);
-        mok[mt] = m < Mtot;
-        const long mm = mok[mt] ? m : Mtot - 1;
-        rowo[mt] = (unsigned)((mm % Mp) + (mm / Mp) * bstride);
+        mok[mt] = m < X.Mtot;
+        const long mm = mok[mt] ? m : X.Mtot - 1;
+        aok[mt] = xf_inner(X, mm % X.Mp);
+        rowo[mt] = (unsigned)((mm % X.Mp) + (mm / X.Mp) * X.bstride);
     }
-    const unsigned lda32 = (unsigned)lda;
+    const unsigned lda32 = (unsigned)X.lda;
     // A values of group kgl: element mt * 4 + ks is A[m(mt), kgl 16 + 4 ks + kl]
     // (k clamped in range; the value is masked to zero at use when k >= K)
     auto ldA = [&](int kgl, double *dst) {
@@ -418,7 +447,7 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
         for (int ks = 0; ks < 4; ks++) {
             const bool kin = kg * 16 + ks * 4 + kl < K;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) a[mt * 4 + ks] = kin ? an[b][mt * 4 + ks] : 0.0;
+            for (int mt = 0; mt < MT; mt++) a[mt * 4 + ks] = kin && aok[mt] ? an[b][mt * 4 + ks] : 0.0;
         }
         __builtin_amdgcn_sched_barrier(0);
         ldA(kg + 2, an[b]);
@@ -450,7 +479,10 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int n = (nt0 + nt) * 16 + 4 * r + kl;
-                if (n < N) Cr[(long)n * ldc] = acc[mt][nt][r];
+                if (n < N) {
+                    double *cp = Cr + (long)n * X.ldc;
+                    *cp = ADD ? *cp + acc[mt][nt][r] : acc[mt][nt][r];
+                }
             }
     }
 }
@@ -477,18 +509,19 @@ static std::vector<double> xform64_pack(int K, int N, Fn b)
 // unless that leaves fewer than 2048 workgroups, then one; narrower column
 // blocks while the grid is still below 2048 workgroups and a block keeps at
 // least two tiles.
-static void launch_xform64(int K, int N, const double *Bf, const double *A, double *C, long Mtot, long Mp,
-                           long bstride, long lda, long ldc, hipStream_t s, const int *active = nullptr)
+template <bool ADD>
+static void launch_xform64(int K, int N, const double *Bf, const double *A, double *C, const XMap &X, hipStream_t s,
+                           const int *active)
 {
     const int KG = (K + 15) / 16, NTt = (N + 15) / 16;
     int ncb = (NTt + 7) / 8;
-    auto blocks = [&](int mt, int nc) { return ((Mtot + 64 * mt - 1) / (64 * mt)) * nc; };
+    auto blocks = [&](int mt, int nc) { return ((X.Mtot + 64 * mt - 1) / (64 * mt)) * nc; };
     const int MT = blocks(2, ncb) >= 2048 ? 2 : 1;
     while (blocks(MT, ncb) < 2048 && (NTt + ncb) / (ncb + 1) >= 2) ncb++;
     const int NT = (NTt + ncb - 1) / ncb;
     ncb = (NTt + NT - 1) / NT;
     const dim3 grid((unsigned)blocks(MT, ncb)), blk(256);
-#define XD_CASE(m, q) case q: hipLaunchKernelGGL((k_xform64<m, q>), grid, blk, 0, s, A, C, Bf, K, KG, N, Mtot, Mp, bstride, lda, ldc, NTt, ncb, active); break;
+#define XD_CASE(m, q) case q: hipLaunchKernelGGL((k_xform64<m, q, ADD>), grid, blk, 0, s, A, C, Bf, K, KG, N, X, NTt, ncb, active); break;
     if (MT == 2) {
         switch (NT) {
             XD_CASE(2, 1) XD_CASE(2, 2) XD_CASE(2, 3) XD_CASE(2, 4) XD_CASE(2, 5) XD_CASE(2, 6) XD_CASE(2, 7) XD_CASE(2, 8)
@@ -636,7 +669,7 @@ template <class T, int M>
 __global__ __launch_bounds__(64 * LS_WAVES) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1)))
 void k_line_solve(Geo g, T *__restrict__ d, const double *__restrict__ ly,
                                                              const double *__restrict__ lz, const int *__restrict__ active,
-                                                             double alpha, double beta)
+                                                             double alpha, double beta, int ncomp)
 {
     if (active && !*active) return;
     constexpr int P = 64 * M + 64;                    // one pad slot per lane chunk
@@ -644,9 +677,10 @@ void k_line_solve(Geo g, T *__restrict__ d, const double *__restrict__ ly,
     const int n = g.nX - 2, ny = g.nY - 2, nz = g.nZ - 2;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const long L = (long)blockIdx.x * LS_WAVES + wv;
-    const bool live = L < (long)ny * nz;
-    const int j = live ? (int)(L % ny) + 1 : 1, k = live ? (int)(L / ny) + 1 : 1;
-    T *line = d + 1 + (long)g.nX * ((long)j + (long)g.nY * k);
+    const bool live = L < (long)ncomp * ny * nz;
+    const long Lc = live ? L : 0;
+    const int j = (int)(Lc % ny) + 1, kc = (int)(Lc / ny), k = kc % nz + 1;   // line (j, k) of component kc / nz
+    T *line = d + (kc / nz) * g.N + 1 + (long)g.nX * ((long)j + (long)g.nY * k);
     T *s = sl[wv];
     auto pos = [](int i) { return i + i / M; };
 #pragma unroll
@@ -742,62 +776,96 @@ void k_line_solve(Geo g, T *__restrict__ d, const double *__restrict__ ly,
 
 template <class T>
 static void launch_line_solve(const Geo &g, T *d, const double *ly, const double *lz, const int *active, double alpha,
-                              double beta, hipStream_t st)
+                              double beta, int ncomp, hipStream_t st)
 {
     const int n = g.nX - 2;
-    const long lines = (long)(g.nY - 2) * (g.nZ - 2);
+    const long lines = (long)ncomp * (g.nY - 2) * (g.nZ - 2);
     const dim3 grid((unsigned)((lines + LS_WAVES - 1) / LS_WAVES)), blk(64 * LS_WAVES);
     const int m = (n + 63) / 64;
-    if (m <= 2) hipLaunchKernelGGL((k_line_solve<T, 2>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta);
-    else if (m <= 4) hipLaunchKernelGGL((k_line_solve<T, 4>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta);
-    else if (m <= 8) hipLaunchKernelGGL((k_line_solve<T, 8>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta);
-    else if (m <= 16) hipLaunchKernelGGL((k_line_solve<T, 16>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta);
-    else hipLaunchKernelGGL((k_line_solve<T, 32>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta);
+    if (m <= 2) hipLaunchKernelGGL((k_line_solve<T, 2>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta, ncomp);
+    else if (m <= 4) hipLaunchKernelGGL((k_line_solve<T, 4>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta, ncomp);
+    else if (m <= 8) hipLaunchKernelGGL((k_line_solve<T, 8>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta, ncomp);
+    else if (m <= 16) hipLaunchKernelGGL((k_line_solve<T, 16>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta, ncomp);
+    else hipLaunchKernelGGL((k_line_solve<T, 32>), grid, blk, 0, st, g, d, ly, lz, active, alpha, beta, ncomp);
 }
 
-// out = (alpha I + beta A)^{-1} r, or its transpose, on the interior planes
-// (face rows of out come out zero).  The transposed system
-// (Wi^T Y Wf^T)^T = Wf Y Wi is solved with the z transforms exchanged and
-// transposed (Ay and the line matrices are symmetric).
-// Rows: the z transforms map all (i,j) rows of planes 1..nz (face rows of r
-// are zero: Krylov vectors and residuals are never written there, so they
-// map to zero rows); the y transforms map the rows i = 0..nX-1 of planes
-// 1..nz, batched over planes (face rows are zero in and out).
+// Three components go through one solve while its two work fields stay in
+// the 256 MB last-level cache (6 N values; FP32 operands of a batch then also
+// stay within the transforms' 32-bit byte offsets).  Beyond it a solve of one
+// component still keeps them there and the batch does not: 1024x192x160 FP32,
+// a
+// component's launches take 509 us batched, 379 us one by one.
+bool solve_batched(const Geo &g, bool single) { return 6.0 * (double)g.N * (single ? 4 : 8) <= 256e6; }
+
+int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s)
+{
+    if (!f || ncomp <= f->ncap) return f ? 0 : 1;
+    const size_t b = (f->single ? sizeof(float) : sizeof(double)) * (size_t)g.N * ncomp;
+    void *n1 = nullptr, *n2 = nullptr;
+    if (hipStreamSynchronize(s) != hipSuccess) return 1;
+    if (hipMalloc(&n1, b) != hipSuccess) return 1;
+    if (hipMalloc(&n2, b) != hipSuccess) { hipFree(n1); return 1; }
+    hipFree(f->t1);
+    hipFree(f->t2);
+    f->t1 = n1;
+    f->t2 = n2;
+    f->ncap = ncomp;
+    return hipMemsetAsync(n1, 0, b, s) == hipSuccess && hipMemsetAsync(n2, 0, b, s) == hipSuccess ? 0 : 1;
+}
+
+// out = (alpha I + beta A)^{-1} in, or its transpose, on the interior planes
+// (face rows of out come out zero, or unchanged when the result is added).
+// The transposed system (Wi^T Y Wf^T)^T = Wf Y Wi is solved with the z
+// transforms exchanged and transposed (Ay and the line matrices are symmetric).
+// Rows: the z transforms map all (i,j) rows of planes 1..nz (the face rows of
+// `in` are zero, or read as zero with `mask`, so they map to zero rows); the y
+// transforms map the rows i = 0..nX-1 of planes 1..nz, batched over planes
+// (face rows are zero in and out).
+// ncomp components, N values apart, go through each launch together: the z
+// rows as further periods, the y rows as further planes (the two face planes
+// between components are zero rows), the lines as further lines.  A solve of
+// three components one by one takes three times the launches, each with its own
+// ramp and tail: 256x64x96 FP64, the launches of three solves 194 -> 162 us;
+// 64x32x48 85 -> 43 us.
 // part: the whole solve (FPC_ALL), its first z transform only (FPC_HEAD) or
 // the rest (FPC_TAIL), so that the first transform can be queued ahead of a
 // host poll.  With active, every launch returns at once when *active is 0.
-template <class T>
-int run_fastpc_ext(const FastPC *f, const Geo &g, const T *r, T *out, const int *active, double alpha, double beta,
+int run_fast_solve(const FastPC *f, const Geo &g, const FastIO &io, const int *active, double alpha, double beta,
                    bool transpose, hipStream_t s, int part)
 {
     const bool head = part != FPC_TAIL, tail = part != FPC_HEAD;
-    const int ny = f->ny, nz = f->nz, nX = g.nX;
+    const int ny = f->ny, nz = f->nz, nX = g.nX, nc = io.ncomp;
+    if (nc < 1 || nc > f->ncap || (!f->single && !(io.in64 && io.out64))) return 1;
     const long pst = g.sZ;                     // plane stride nX*nY
     const long y0 = (long)nX + pst;            // (i,j,k) = (0,1,1)
-    T *u1 = (T *)f->t1, *u2 = (T *)f->t2;
-    if (sizeof(T) == sizeof(float)) {
-        if (!f->single) return 1;
-        const float *rf = (const float *)(const void *)r;
-        float *of = (float *)(void *)out, *v1 = (float *)(void *)u1, *v2 = (float *)(void *)u2;
+    XMap Z = {nc * pst, pst, g.N, pst, pst, 0, 0}, Y = {(long)nX * ((long)nc * g.nZ - 2), nX, pst, nX, nX, 0, 0};
+    XMap Zin = Z;
+    if (io.mask) { Zin.mask = nX; Zin.mask_ny = g.nY; }
+    if (f->single) {
+        float *v1 = (float *)f->t1, *v2 = (float *)f->t2;
         const unsigned short *zf = transpose ? f->bz_ft : f->bz_f, *zi = transpose ? f->bz_it : f->bz_i;
-        if (head) launch_xform(nz, nz, zf, rf + pst, v1 + pst, pst, pst, 0, pst, pst, s, active);
+        if (head) {
+            if (io.in64) launch_xform(nz, nz, zf, (const double *)io.in + pst, v1 + pst, Zin, s, active);
+            else launch_xform(nz, nz, zf, (const float *)io.in + pst, v1 + pst, Zin, s, active);
+        }
         if (tail) {
-            launch_xform(ny, ny, f->by_f, v1 + y0, v2 + y0, (long)nX * nz, nX, pst, nX, nX, s, active);
-            launch_line_solve<float>(g, v2, f->ly, f->lz, active, alpha, beta, s);
-            launch_xform(ny, ny, f->by_i, v2 + y0, v1 + y0, (long)nX * nz, nX, pst, nX, nX, s, active);
-            launch_xform(nz, nz, zi, v1 + pst, of + pst, pst, pst, 0, pst, pst, s, active);
+            launch_xform(ny, ny, f->by_f, (const float *)v1 + y0, v2 + y0, Y, s, active);
+            launch_line_solve<float>(g, v2, f->ly, f->lz, active, alpha, beta, nc, s);
+            launch_xform(ny, ny, f->by_i, (const float *)v2 + y0, v1 + y0, Y, s, active);
+            void *o = io.out64 ? (void *)((double *)io.out + pst) : (void *)((float *)io.out + pst);
+            launch_xform(nz, nz, zi, (const float *)v1 + pst, o, Z, s, active,
+                         io.out64 ? (io.add ? XO_F64_ADD : XO_F64) : (io.add ? XO_F32_ADD : XO_F32));
         }
     } else {
-        if (f->single) return 1;
-        const double *rd = (const double *)(const void *)r;
-        double *od = (double *)(void *)out, *v1 = (double *)(void *)u1, *v2 = (double *)(void *)u2;
+        double *v1 = (double *)f->t1, *v2 = (double *)f->t2;
         const double *zf = transpose ? f->dz_ft : f->dz_f, *zi = transpose ? f->dz_it : f->dz_i;
-        if (head) launch_xform64(nz, nz, zf, rd + pst, v1 + pst, pst, pst, 0, pst, pst, s, active);
+        if (head) launch_xform64<false>(nz, nz, zf, (const double *)io.in + pst, v1 + pst, Zin, s, active);
         if (tail) {
-            launch_xform64(ny, ny, f->dy_f, v1 + y0, v2 + y0, (long)nX * nz, nX, pst, nX, nX, s, active);
-            launch_line_solve<double>(g, v2, f->ly, f->lz, active, alpha, beta, s);
-            launch_xform64(ny, ny, f->dy_i, v2 + y0, v1 + y0, (long)nX * nz, nX, pst, nX, nX, s, active);
-            launch_xform64(nz, nz, zi, v1 + pst, od + pst, pst, pst, 0, pst, pst, s, active);
+            launch_xform64<false>(ny, ny, f->dy_f, v1 + y0, v2 + y0, Y, s, active);
+            launch_line_solve<double>(g, v2, f->ly, f->lz, active, alpha, beta, nc, s);
+            launch_xform64<false>(ny, ny, f->dy_i, v2 + y0, v1 + y0, Y, s, active);
+            if (io.add) launch_xform64<true>(nz, nz, zi, v1 + pst, (double *)io.out + pst, Z, s, active);
+            else launch_xform64<false>(nz, nz, zi, v1 + pst, (double *)io.out + pst, Z, s, active);
         }
     }
     return hipGetLastError() == hipSuccess ? 0 : 1;
@@ -807,14 +875,15 @@ int run_fastpc_ext(const FastPC *f, const Geo &g, const T *r, T *out, const int 
 template <class T>
 int run_fastpc(const FastPC *f, const Geo &g, const T *r, T *out, const int *active, hipStream_t s, int part)
 {
-    return run_fastpc_ext<T>(f, g, r, out, active, 0.0, 1.0, false, s, part);
+    if (f->single != (sizeof(T) == sizeof(float))) return 1;
+    FastIO io;
+    io.in = r;
+    io.out = out;
+    io.in64 = io.out64 = sizeof(T) == sizeof(double);
+    return run_fast_solve(f, g, io, active, 0.0, 1.0, false, s, part);
 }
 
 template int run_fastpc<double>(const FastPC *, const Geo &, const double *, double *, const int *, hipStream_t, int);
-template int run_fastpc_ext<double>(const FastPC *, const Geo &, const double *, double *, const int *, double, double,
-                                    bool, hipStream_t, int);
 template int run_fastpc<float>(const FastPC *, const Geo &, const float *, float *, const int *, hipStream_t, int);
-template int run_fastpc_ext<float>(const FastPC *, const Geo &, const float *, float *, const int *, double, double,
-                                   bool, hipStream_t, int);
 
 }  // namespace tbl

@@ -432,12 +432,6 @@ __global__ __launch_bounds__(VB) void k_xupd(const T *__restrict__ V, long ldv, 
     }
 }
 
-template <class Td, class Ts>
-__global__ __launch_bounds__(VB) void k_convert(const Ts *__restrict__ s, Td *__restrict__ d, long n)
-{
-    for (long e = (long)blockIdx.x * VB + threadIdx.x; e < n; e += (long)gridDim.x * VB) d[e] = (Td)s[e];
-}
-
 // ---------------------------------------------------------------- launchers
 template <class T>
 void launch_norm2(const T *x, long N, double *part, const int *active, hipStream_t s)
@@ -484,15 +478,6 @@ void launch_xupd(const T *V, long ldv, long N, const GmCtrl *c, double *PC, hipS
 {
     hipLaunchKernelGGL(k_xupd<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, N, c, PC);
 }
-template <class Td, class Ts>
-void launch_convert(const Ts *src, Td *dst, long n, hipStream_t s)
-{
-    long nb = (n + VB * 8 - 1) / (VB * 8);
-    if (nb > 65536) nb = 65536;
-    if (nb < 1) nb = 1;
-    hipLaunchKernelGGL((k_convert<Td, Ts>), dim3((unsigned)nb), dim3(VB), 0, s, src, dst, n);
-}
-
 #define TBL_INST(T)                                                                                 \
     template void launch_norm2<T>(const T *, long, double *, const int *, hipStream_t);             \
     template void launch_dots<T>(const T *, long, int, long, const GmCtrl *, double *, hipStream_t); \
@@ -501,9 +486,6 @@ void launch_convert(const Ts *src, Td *dst, long n, hipStream_t s)
 TBL_INST(double)
 TBL_INST(float)
 #undef TBL_INST
-template void launch_convert<float, double>(const double *, float *, long, hipStream_t);
-template void launch_convert<double, float>(const float *, double *, long, hipStream_t);
-template void launch_convert<double, double>(const double *, double *, long, hipStream_t);
 
 // pc <- 2 pc - prev, prev <- old pc (linear extrapolation of the pressure
 // correction in time, the initial guess of the next solve)

@@ -75,9 +75,21 @@ void fastpc_destroy(FastPC *f);
 enum { FPC_ALL = 0, FPC_HEAD = 1, FPC_TAIL = 2 };
 template <class T> int run_fastpc(const FastPC *f, const Geo &g, const T *r, T *out, const int *active, hipStream_t s,
                                   int part = FPC_ALL);
-// out = (alpha I + beta A)^{-1} r, or its transpose (double only)
-template <class T> int run_fastpc_ext(const FastPC *f, const Geo &g, const T *r, T *out, const int *active, double alpha,
-                                      double beta, bool transpose, hipStream_t s, int part = FPC_ALL);
+// one fast solve of ncomp components (N values apart): operand and result in
+// FP64 or in the storage type (FP64 contexts: FP64 both); add: out += result;
+// mask: the operand's face rows are read as zero
+struct FastIO {
+    const void *in = nullptr;
+    void *out = nullptr;
+    int in64 = 0, out64 = 0, add = 0, mask = 0, ncomp = 1;
+};
+// out = (alpha I + beta A)^{-1} in, or its transpose
+int run_fast_solve(const FastPC *f, const Geo &g, const FastIO &io, const int *active, double alpha, double beta,
+                   bool transpose, hipStream_t s, int part = FPC_ALL);
+// work fields for solves of ncomp components (synchronises when they grow);
+// solve_batched: whether three components may go through one solve
+int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s);
+bool solve_batched(const Geo &g, bool single);
 
 // Krylov kernels (tbl_krylov.hip)
 unsigned vec_blocks(long N);
@@ -98,7 +110,6 @@ void launch_fin_update(GmCtrl *c, const double *part, int nb, int j, hipStream_t
 // gated: does nothing while the cycle is active (queued ahead of a host poll)
 void launch_fin_cycle(GmCtrl *c, hipStream_t s, int gated = 0);
 template <class T> void launch_xupd(const T *V, long ldv, long N, const GmCtrl *c, double *PC, hipStream_t s);
-template <class Td, class Ts> void launch_convert(const Ts *src, Td *dst, long n, hipStream_t s);
 
 // diagnostics (tbl_diag.hip)
 struct RecDev {            // device-resident scalars of the recycling state
@@ -124,12 +135,9 @@ template <class T> void launch_wall_shear(const Geo &g, const T *Ut, double *tau
 void launch_tau_window(const Geo &g, int window, double *acc, double *mean, double *cf, hipStream_t s);
 
 // direct Helmholtz solve and the discrete adjoint (tbl_adjoint.hip)
-template <class T> void launch_helm_rfield(const Geo &g, const T *Q, const T *u, T *r, hipStream_t s);
-// u += d on the interior (d may be narrower than u: an FP32 correction of FP64 u)
-template <class T, class Td = T> void launch_add_interior(const Geo &g, T *u, const Td *d, hipStream_t s);
-void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, double *r, hipStream_t s);
-void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, float *r, hipStream_t s);
-void launch_copy_interior(const Geo &g, const double *in, double *out, hipStream_t s);
+template <class T> void launch_helm_rfield(const Geo &g, const T *Q, const T *u, T *r, int ncomp, hipStream_t s);
+template <class To>
+void launch_opT_res(const Geo &g, const double *b, const double *x, double alpha, double beta, To *r, int ncomp, hipStream_t s);
 void launch_adj_tau(const Geo &g, double *lamU, int i0, int i1, double cJ, hipStream_t s);
 // boundary values of a step's end velocity that the reversed conditions read (E, adj_end_len doubles)
 long adj_end_len(const Geo &g);
