@@ -179,9 +179,13 @@ __device__ __forceinline__ bool xf_inner(const XMap &x, long in_period)
     const int i = (int)(in_period % x.mask), j = (int)(in_period / x.mask);
     return i >= 1 && i <= x.mask - 2 && j >= 1 && j <= x.mask_ny - 2;
 }
-// two waves per SIMD: with 8 tiles the accumulators take half the registers
-template <int NT, class Ti>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_xform(const Ti *__restrict__ A, void *Cv,
+// PLAIN: FP32 in and out, no mask -- the transforms inside a solve and of the
+// preconditioner, compiled apart (with the other outputs' stores in it the
+// kernel took 4 % longer: 8 tiles, K = 254 at 1024x192x256 145 -> 150 us).
+// The general form keeps two waves per SIMD with 8 tiles, whose accumulators
+// take half the registers.
+template <int NT, class Ti, bool PLAIN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN ? 1 : 2))) void k_xform(const Ti *__restrict__ A, void *Cv,
                                               const xf_v4u *__restrict__ Bf, int K, int KG, int N, XMap X, int NTt,
                                               int ncb, int out, const int *__restrict__ active)
 {
@@ -196,7 +200,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const long rb = (long)(L / (unsigned)ncb);
     const int nt0 = cb * NT;                                 // first tile of this column block
     const long m = rb * XF_ROWS + wv * 32 + (lane & 31);
-    const bool mok = m < X.Mtot, aok = mok && xf_inner(X, m % X.Mp);
+    const bool mok = m < X.Mtot, aok = mok && (PLAIN || xf_inner(X, m % X.Mp));
     const long row = mok ? (m % X.Mp) + (m / X.Mp) * X.bstride : 0;
     const int kh = (lane >> 5) * 8;
     xf_v16f acc[NT];
@@ -308,7 +312,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                     }
                 }
         };
-        if (out == XO_F32) store((float *)Cv + row, std::false_type{});
+        if (PLAIN || out == XO_F32) store((float *)Cv + row, std::false_type{});
         else if (out == XO_F32_ADD) store((float *)Cv + row, std::true_type{});
         else if (out == XO_F64) store((double *)Cv + row, std::false_type{});
         else store((double *)Cv + row, std::true_type{});
@@ -346,11 +350,16 @@ static void launch_xform(int K, int N, const unsigned short *Bf, const Ti *A, vo
     const int ncb = (NTt + XF_MAXT - 1) / XF_MAXT, NT = (NTt + ncb - 1) / ncb;   // at most XF_MAXT tiles per block
     const dim3 grid((unsigned)(((X.Mtot + XF_ROWS - 1) / XF_ROWS) * ncb)), blk(256);
     const xf_v4u *B = (const xf_v4u *)Bf;
-#define XF_CASE(q) case q: hipLaunchKernelGGL((k_xform<q, Ti>), grid, blk, 0, s, A, C, B, K, KG, N, X, NTt, ncb, out, active); break;
-    switch (NT) {
-        XF_CASE(1) XF_CASE(2) XF_CASE(3) XF_CASE(4) XF_CASE(5) XF_CASE(6) XF_CASE(7) XF_CASE(8)
-        default: break;
+#define XF_CASE(q, plain) case q: hipLaunchKernelGGL((k_xform<q, Ti, plain>), grid, blk, 0, s, A, C, B, K, KG, N, X, NTt, ncb, out, active); break;
+#define XF_CASES(plain) XF_CASE(1, plain) XF_CASE(2, plain) XF_CASE(3, plain) XF_CASE(4, plain) XF_CASE(5, plain) XF_CASE(6, plain) XF_CASE(7, plain) XF_CASE(8, plain)
+    if (std::is_same<Ti, float>::value && out == XO_F32 && !X.mask) {
+        if constexpr (std::is_same<Ti, float>::value) {
+            switch (NT) { XF_CASES(true) default: break; }
+        }
+    } else {
+        switch (NT) { XF_CASES(false) default: break; }
     }
+#undef XF_CASES
 #undef XF_CASE
 }
 
@@ -730,9 +739,11 @@ void k_line_solve(Geo g, T *__restrict__ d, const double *__restrict__ ly,
     if (M == 2) { AF = a0; BF = b0; CF = c0; DF = d0; }
     else { AF = a0; BF = b0 - c0 * ap[1]; CF = -(c0 * cp[1]); DF = d0 - c0 * dp[1]; }
     T AL = ap[M - 1], BL = T(1), CL = cp[M - 1], DL = dp[M - 1];
-    // cyclic reduction over the 128-row sequence F0 L0 F1 L1 ...
-    auto red = [](T &A, T &B, T &C, T &D, T Am, T Bm, T Cm, T Dm, T Ap, T Bp, T Cp, T Dp) {
-        const T k1 = ls_div(A, Bm), k2 = ls_div(C, Bp);
+    // cyclic reduction over the 128-row sequence F0 L0 F1 L1 ...; a row hands
+    // its neighbours the reciprocal r of its diagonal (one division a row and
+    // level, where each of its two neighbours divided by it)
+    auto red = [](T &A, T &B, T &C, T &D, T Am, T rm, T Cm, T Dm, T Ap, T rp, T Cp, T Dp) {
+        const T k1 = A * rm, k2 = C * rp;
         B = B - Cm * k1 - Ap * k2;
         D = D - Dm * k1 - Dp * k2;
         A = -(Am * k1);
@@ -740,26 +751,36 @@ void k_line_solve(Geo g, T *__restrict__ d, const double *__restrict__ ly,
     };
     {
         // stride 1: F(l) sits between L(l-1) and L(l); L(l) between F(l) and F(l+1)
-        const T lA = __shfl(AL, lane - 1), lB = __shfl(BL, lane - 1), lC = __shfl(CL, lane - 1), lD = __shfl(DL, lane - 1);
-        const T uA = __shfl(AF, lane + 1), uB = __shfl(BF, lane + 1), uC = __shfl(CF, lane + 1), uD = __shfl(DF, lane + 1);
+        // (the L rows' diagonal is 1)
+        const T rF = ls_div(T(1), BF);
+        const T lA = __shfl(AL, lane - 1), lC = __shfl(CL, lane - 1), lD = __shfl(DL, lane - 1);
+        const T uA = __shfl(AF, lane + 1), uR = __shfl(rF, lane + 1), uC = __shfl(CF, lane + 1), uD = __shfl(DF, lane + 1);
         const bool hl = lane > 0, hu = lane < 63;
-        const T fA = AF, fB = BF, fC = CF, fD = DF, gA = AL, gB = BL, gC = CL, gD = DL;
-        red(AF, BF, CF, DF, hl ? lA : T(0), hl ? lB : T(1), hl ? lC : T(0), hl ? lD : T(0), gA, gB, gC, gD);
-        red(AL, BL, CL, DL, fA, fB, fC, fD, hu ? uA : T(0), hu ? uB : T(1), hu ? uC : T(0), hu ? uD : T(0));
+        const T fA = AF, fC = CF, fD = DF;
+        red(AF, BF, CF, DF, hl ? lA : T(0), T(1), hl ? lC : T(0), hl ? lD : T(0), AL, T(1), CL, DL);
+        red(AL, BL, CL, DL, fA, rF, fC, fD, hu ? uA : T(0), hu ? uR : T(1), hu ? uC : T(0), hu ? uD : T(0));
     }
-#pragma unroll
+    // Each level squares the couplings (relative to the diagonal), and most
+    // lines have a diagonal far above 2 |ow|: once no coupling of the line
+    // reaches LS_TINY, what it could still move is 2^-40 (FP32) or 2^-80
+    // (FP64) of the line's largest value, below what the transforms round off,
+    // and the remaining levels are not run.
+    constexpr T LS_TINY = sizeof(T) == 4 ? T(0x1p-40) : T(0x1p-80);
     for (int h = 1; h < 64; h <<= 1) {
+        const T big = LS_TINY * fabs(BF), bil = LS_TINY * fabs(BL);
+        if (!__any(fabs(AF) > big || fabs(CF) > big || fabs(AL) > bil || fabs(CL) > bil)) break;
         // stride 2h: rows of the same kind h lanes away
         const bool hl = lane >= h, hu = lane + h < 64;
         const int sl_ = hl ? lane - h : lane, su = hu ? lane + h : lane;
-        const T fmA = __shfl(AF, sl_), fmB = __shfl(BF, sl_), fmC = __shfl(CF, sl_), fmD = __shfl(DF, sl_);
-        const T fpA = __shfl(AF, su), fpB = __shfl(BF, su), fpC = __shfl(CF, su), fpD = __shfl(DF, su);
-        const T lmA = __shfl(AL, sl_), lmB = __shfl(BL, sl_), lmC = __shfl(CL, sl_), lmD = __shfl(DL, sl_);
-        const T lpA = __shfl(AL, su), lpB = __shfl(BL, su), lpC = __shfl(CL, su), lpD = __shfl(DL, su);
-        red(AF, BF, CF, DF, hl ? fmA : T(0), hl ? fmB : T(1), hl ? fmC : T(0), hl ? fmD : T(0),
-            hu ? fpA : T(0), hu ? fpB : T(1), hu ? fpC : T(0), hu ? fpD : T(0));
-        red(AL, BL, CL, DL, hl ? lmA : T(0), hl ? lmB : T(1), hl ? lmC : T(0), hl ? lmD : T(0),
-            hu ? lpA : T(0), hu ? lpB : T(1), hu ? lpC : T(0), hu ? lpD : T(0));
+        auto level = [&](T &A, T &B, T &C, T &D) {
+            const T r = ls_div(T(1), B);
+            const T mA = __shfl(A, sl_), mR = __shfl(r, sl_), mC = __shfl(C, sl_), mD = __shfl(D, sl_);
+            const T pA = __shfl(A, su), pR = __shfl(r, su), pC = __shfl(C, su), pD = __shfl(D, su);
+            red(A, B, C, D, hl ? mA : T(0), hl ? mR : T(1), hl ? mC : T(0), hl ? mD : T(0),
+                hu ? pA : T(0), hu ? pR : T(1), hu ? pC : T(0), hu ? pD : T(0));
+        };
+        level(AF, BF, CF, DF);
+        level(AL, BL, CL, DL);
     }
     const T xf = ls_div(DF, BF), xl = ls_div(DL, BL);
     s[pos(i0)] = xf;
