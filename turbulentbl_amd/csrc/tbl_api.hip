@@ -56,8 +56,12 @@ struct tbl_ctx {
     double *part = nullptr;
     size_t npart = 0;
     GmCtrl *gm = nullptr;
-    GmStatus *gm_h = nullptr;            // pinned
-    void *gs = nullptr, *gs_h = nullptr; // Gauss-Seidel control (device / pinned)
+    // pinned host block that kernels publish their results to (see Pub), and
+    // its parts: GMRES status, Gauss-Seidel control, diagnostics record
+    struct HostPub *hp = nullptr;
+    unsigned pseq = 0;                   // sequence number of the last result asked for
+    GmStatus *gm_h = nullptr;
+    void *gs = nullptr, *gs_h = nullptr; // Gauss-Seidel control (device / published)
     double *sums = nullptr, *avg = nullptr, *Wt = nullptr, *Ume = nullptr, *uf = nullptr;
     double *bltkns = nullptr, *dstar = nullptr, *theta = nullptr, *wall_w = nullptr, *tau = nullptr;
     double *tausum = nullptr, *taumean = nullptr, *cf = nullptr;   // wall-shear window (a17)
@@ -67,10 +71,10 @@ struct tbl_ctx {
     void *zf = nullptr;                  // z-line Gauss-Seidel elimination factors (storage type)
     int *newk = nullptr;
     RecDev *rec = nullptr;
-    int *guard = nullptr;
+    int *guard = nullptr;                // in the diagnostics record
     double *dd = nullptr;                // device diagnostics record
     double *noalloc = nullptr;           // this device's copy of `scratch` (tbl_div_check_noalloc)
-    double *dh = nullptr;                // pinned copy
+    double *dh = nullptr;                // published copy
     bool have_wall_w = false;
     // Peclet-switch patterns of an adjoint window (record / replay): one byte
     // per cell and step, window of br_steps steps starting after step br_nstep0
@@ -86,16 +90,20 @@ struct tbl_ctx {
     unsigned tmask = 0;
     std::vector<TimerRec> pend;
     std::vector<hipEvent_t> pool;
-    hipEvent_t poll_ev = nullptr;        // marks a stopping-test read-back the host spins on
     int tcount[TBL_K_NCLASS] = {0};
     double tms[TBL_K_NCLASS] = {0};
     double tbytes[TBL_K_NCLASS] = {0};
     std::string err;
 };
 
-// device diagnostics record layout
 // device diagnostics record; the mass-flux partials (5 * MF_BLK) follow it
-enum { DD_DIV = 0, DD_MASS = 1, DD_KE = 6, DD_BNORM = 7, DD_NCOUNT = 8 };
+enum { DD_DIV = 0, DD_MASS = 1, DD_KE = 6, DD_BNORM = 7, DD_GUARD = 8, DD_NCOUNT = 9 };
+
+struct HostPub {
+    unsigned seq, pad;
+    GmStatus gm;
+    double gs[16], dd[DD_NCOUNT];
+};
 
 #define HIPCHK(ctx, call)                                                                    \
     do {                                                                                     \
@@ -424,9 +432,14 @@ static int create_impl(tbl_ctx *c)
     c->npart = std::max(c->npart, 6 * (size_t)rhs_blocks(c->g, c->mixed));             // fused first residual pass fits
     CHK(dalloc(c, &c->part, c->npart * sizeof(double)));
     CHK(dalloc(c, &c->gm, sizeof(GmCtrl)));
-    HIPCHK(c, hipHostMalloc((void **)&c->gm_h, sizeof(GmStatus), hipHostMallocDefault));
+    // fine-grained (coherent), so that a running kernel's stores reach the host
+    HIPCHK(c, hipHostMalloc((void **)&c->hp, sizeof(HostPub), hipHostMallocCoherent));
+    memset(c->hp, 0, sizeof(HostPub));
+    if (gs_ctrl_bytes() > sizeof(c->hp->gs)) return fail(c, TBL_EARG, "Gauss-Seidel control block above its host copy");
+    c->gm_h = &c->hp->gm;
+    c->gs_h = c->hp->gs;
+    c->dh = c->hp->dd;
     CHK(dalloc(c, &c->gs, gs_ctrl_bytes()));
-    HIPCHK(c, hipHostMalloc(&c->gs_h, gs_ctrl_bytes(), hipHostMallocDefault));
     const long M = (long)p.nX * p.nZ;
     CHK(dalloc(c, &c->sums, 9 * M * sizeof(double)));
     CHK(dalloc(c, &c->avg, 9 * M * sizeof(double)));
@@ -444,9 +457,8 @@ static int create_impl(tbl_ctx *c)
     CHK(dalloc(c, &c->scan, 2 * (p.nZ + 2) * sizeof(double)));
     CHK(dalloc(c, &c->newk, p.nZ * sizeof(int)));
     CHK(dalloc(c, &c->rec, sizeof(RecDev)));
-    CHK(dalloc(c, &c->guard, sizeof(int)));
     CHK(dalloc(c, &c->dd, (DD_NCOUNT + 5 * MF_BLK) * sizeof(double)));
-    HIPCHK(c, hipHostMalloc((void **)&c->dh, DD_NCOUNT * sizeof(double), hipHostMallocDefault));
+    c->guard = (int *)(c->dd + DD_GUARD);
     RecDev r0 = {1.0, 1.0, 0};
     HIPCHK(c, hipMemcpyAsync(c->rec, &r0, sizeof(r0), hipMemcpyHostToDevice, c->s));
     std::vector<int> nk(p.nZ);
@@ -517,17 +529,14 @@ extern "C" int tbl_destroy(tbl_ctx *c)
     if (c->s) hipStreamSynchronize(c->s);
     timer_flush(c);
     for (auto e : c->pool) hipEventDestroy(e);
-    if (c->poll_ev) hipEventDestroy(c->poll_ev);
     void *dev[] = {c->mesh, c->Ut, c->Ualt, c->Utold, c->Q, c->Press, c->PCorr, c->pRhs, c->V, c->W, c->scr, c->r, c->Z,
                    c->part, c->gm, c->gs, c->sums, c->avg, c->Wt, c->Ume, c->uf, c->bltkns, c->dstar,
-                   c->theta, c->tau, c->tausum, c->taumean, c->cf, c->wall_w, c->scan, c->newk, c->rec, c->guard, c->dd, c->zf, c->br, c->PCprev,
+                   c->theta, c->tau, c->tausum, c->taumean, c->cf, c->wall_w, c->scan, c->newk, c->rec, c->dd, c->zf, c->br, c->PCprev,
                    c->PCalt, c->slab, c->halo, c->r3};
     for (void *d : dev)
         if (d) hipFree(d);
     if (c->fast) fastpc_destroy(c->fast);
-    if (c->gm_h) hipHostFree(c->gm_h);
-    if (c->gs_h) hipHostFree(c->gs_h);
-    if (c->dh) hipHostFree(c->dh);
+    if (c->hp) hipHostFree(c->hp);
     if (c->s) hipStreamDestroy(c->s);
     delete c;
     return 0;
@@ -657,38 +666,49 @@ static int d2h(tbl_ctx *c, void *h, const void *d, size_t b)
     return 0;
 }
 
-// wait for the stream before the host reads a stopping test: spin on an event
-// rather than block in a stream synchronise, since the next launch waits on
-// the host's wake-up.  The first POLL_SPIN_US microseconds spin tightly; after
-// that every query yields the core (sched_yield), so a long wait does not keep
-// a host core from the caller's other threads.
-// poll_mark / poll_spin split the wait so that work gated on the device's
-// own stopping flags can be queued behind the read-back: the GPU then runs it
-// while the host waits for the flags.
+// Results the host waits for (stopping tests, diagnostics): a kernel publishes
+// them (Pub) and pub_wait spins on the sequence number, since the next launch
+// waits on the host's wake-up.  Work gated on the device's own stopping flags
+// can be queued in between: the GPU then runs it while the host waits.  The
+// first POLL_SPIN_US microseconds spin tightly; after that every turn asks the
+// stream for errors and yields the core (sched_yield), so a long wait does not
+// keep a host core from the caller's other threads, and a stream that has
+// failed or drained without publishing ends the wait.
 #define POLL_SPIN_US 20
-static int poll_mark(tbl_ctx *c)
+static Pub pub_of(tbl_ctx *c, void *dst)
 {
-    if (!c->poll_ev) HIPCHK(c, hipEventCreateWithFlags(&c->poll_ev, hipEventDisableTiming));
-    HIPCHK(c, hipEventRecord(c->poll_ev, c->s));
-    return 0;
+    Pub p;
+    p.seq = &c->hp->seq;
+    p.dst = dst;
+    p.val = ++c->pseq;
+    return p;
 }
-static int poll_spin(tbl_ctx *c)
+static int pub_wait(tbl_ctx *c)
 {
-    hipError_t e;
+    auto there = [&] { return (int)(__atomic_load_n(&c->hp->seq, __ATOMIC_ACQUIRE) - c->pseq) >= 0; };
     const auto t0 = std::chrono::steady_clock::now();
     bool spin = true;
-    while ((e = hipEventQuery(c->poll_ev)) == hipErrorNotReady) {
-        if (spin) spin = std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(POLL_SPIN_US);
-        else sched_yield();
+    while (!there()) {
+        if (spin) {
+            spin = std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(POLL_SPIN_US);
+            continue;
+        }
+        const hipError_t e = hipStreamQuery(c->s);
+        if (e == hipSuccess && !there()) return fail(c, TBL_ESTATE, "a kernel ended without publishing its result");
+        if (e != hipSuccess && e != hipErrorNotReady) HIPCHK(c, e);
+        sched_yield();
     }
-    HIPCHK(c, e);
     return 0;
 }
-static int poll_wait(tbl_ctx *c)
+// the diagnostics record, after the kernels queued so far
+static int read_diag(tbl_ctx *c)
 {
-    CHK(poll_mark(c));
-    return poll_spin(c);
+    launch_publish(c->dd, DD_NCOUNT, pub_of(c, c->dh), c->s);
+    HIPCHK(c, hipGetLastError());
+    return pub_wait(c);
 }
+// the GMRES status, likewise
+static void ask_status(tbl_ctx *c) { launch_publish(&c->gm->st, sizeof(GmStatus) / 8, pub_of(c, c->gm_h), c->s); }
 
 extern "C" int tbl_set_state(tbl_ctx *c, const tbl_state *st)
 {
@@ -973,10 +993,6 @@ template <class T> static int helm_impl(tbl_ctx *c, double errorstop, int mmax, 
     if (ppe_done) *ppe_done = false;
     if (c->p.helm_mode == TBL_HELM_DIRECT) return helm_direct<T>(c, sweeps, res);
     const bool ppe_ahead = ppe_done && !(c->tmask & (1u << TBL_K_DIV));
-    gs_ctrl_init(c->gs_h, 7);
-    // stream-ordered copy from the pinned control block; the host next
-    // touches gs_h after a synchronised read-back
-    CHK(h2d(c, c->gs, c->gs_h, gs_ctrl_bytes()));
     // the z-line sweep converges in a few iterations: poll the stopping test
     // of every residual pass (odd it >= 3) before launching the sweeps, so
     // that no sweep is launched for components that have all stopped; point
@@ -987,7 +1003,8 @@ template <class T> static int helm_impl(tbl_ctx *c, double errorstop, int mmax, 
     // zebra: sweeps read cur and write alt, which then swap; the boundary and
     // ghost values (not changed by the solve) are copied into alt first
     T *cur = F<T>(c->Ut), *alt = zebra ? F<T>(c->Ualt) : nullptr;
-    if (zebra) launch_copy_faces3<T>(c->g, cur, alt, c->s);
+    if (zebra) launch_copy_faces3<T>(c->g, cur, alt, c->gs, c->s);
+    else launch_gs_init(c->gs, c->s);
     int act[3] = {1, 1, 1}, sw[3] = {0, 0, 0};
     double rs[3] = {0, 0, 0};
     bool fresh = false;                        // gs_h holds the final control block
@@ -1000,13 +1017,12 @@ template <class T> static int helm_impl(tbl_ctx *c, double errorstop, int mmax, 
                 launch_helm_resid<T>(c->g, F<T>(c->Q), zebra ? cur : F<T>(c->Ut), c->gs, c->part, it == 1 ? 1 : 0,
                                      c->s);
             }
+            const bool poll = it >= 3 && (every || it % 8 == 1);
             launch_helm_fin(c->g, c->gs, c->part, it, errorstop, c->mixed ? 32.0 * 1.1920928955078125e-7 : 0.0, c->s,
-                            pre ? pre_nb : 0);
-            if (it >= 3 && (every || it % 8 == 1)) {
-                CHK(d2h(c, c->gs_h, c->gs, gs_ctrl_bytes()));
-                CHK(poll_mark(c));
+                            pre ? pre_nb : 0, poll ? pub_of(c, c->gs_h) : Pub());
+            if (poll) {
                 if (ppe_ahead) launch_ppe_rhs<T>(c->g, zebra ? cur : F<T>(c->Ut), c->pRhs, c->s, c->gs);
-                CHK(poll_spin(c));
+                CHK(pub_wait(c));
                 gs_ctrl_read(c->gs_h, act, sw, rs);
                 if (!act[0] && !act[1] && !act[2]) {
                     fresh = true;
@@ -1056,8 +1072,9 @@ template <class T> static int helm_impl(tbl_ctx *c, double errorstop, int mmax, 
         HIPCHK(c, hipGetLastError());
     }
     if (!fresh) {
-        CHK(d2h(c, c->gs_h, c->gs, gs_ctrl_bytes()));
-        CHK(poll_wait(c));
+        launch_publish(c->gs, (int)(gs_ctrl_bytes() / 8), pub_of(c, c->gs_h), c->s);
+        HIPCHK(c, hipGetLastError());
+        CHK(pub_wait(c));
         gs_ctrl_read(c->gs_h, act, sw, rs);
     }
     if (zebra && cur != F<T>(c->Ut)) std::swap(c->Ut, c->Ualt);   // the solution is in cur
@@ -1117,10 +1134,12 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
     T *V = F<T>(c->V), *W = F<T>(c->W), *scr = F<T>(c->scr), *r = F<T>(c->r);
     const long ldv = c->ldv;
     if (kmax > c->p.kmax) return fail(c, TBL_EARG, "kmax above the allocated restart length");
-    // control block, set up on the device
     const int mode = (c->p.tol_mode == TBL_TOL_TRUE) ? GM_MODE_TRUE : GM_MODE_REF;
-    launch_gm_init(c->gm, errtol, c->p.inner_tol, kmax, mmax, mode, c->s);
-    launch_zero_faces(g, c->PCorr, c->s);
+    const int poll = (N > 2000000 || c->p.precond == TBL_PC_FAST) ? 1 : 4;
+    // the second PCorr buffer of fused updates (TRUE) and unit steps
+    const bool two = c->p.precond == TBL_PC_FAST || (mode == GM_MODE_TRUE && poll == 1);
+    if (two && !c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
+    launch_gm_init(g, c->gm, errtol, c->p.inner_tol, kmax, mmax, mode, c->PCorr, two ? c->PCalt : nullptr, c->s);
     double *part_r = c->part;                  // residual partials
     double *part_z = c->part + nbr + 8;        // norm partials (and dot partials)
     const bool fuse_dot = poisson_blocks(g) <= c->npart - nbr - 8;
@@ -1132,13 +1151,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         c->pc_hist = c->pc_hist < 2 ? c->pc_hist + 1 : 2;
     }
     const int *act = &c->gm->st.active;
-    const int poll = (N > 2000000 || c->p.precond == TBL_PC_FAST) ? 1 : 4;
     bool final_res = false;                    // st.true_res is the residual of the final PCorr
-    // the second PCorr buffer of fused updates (TRUE) and unit steps
-    if (c->p.precond == TBL_PC_FAST || (mode == GM_MODE_TRUE && poll == 1)) {
-        if (!c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
-        launch_zero_faces(g, c->PCalt, c->s);
-    }
     if (mode == GM_MODE_TRUE) {
         // Flexible (right-preconditioned) GMRES: the Givens estimate is the true
         // residual, one preconditioner application per Arnoldi step, and the
@@ -1199,12 +1212,10 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                     Tscope ts(c, TBL_K_RESID, (double)N * (24.0 + 2.0 * sizeof(T)));
                     launch_resid_upd<T>(g, c->pRhs, c->PCorr, Z, c->gm, c->PCalt, v1, part_r, c->s, RU_UNIT);
                 }
-                launch_fin_unit(c->gm, part_r, (int)nbr, nullptr, 0, c->s);
+                launch_fin_unit(c->gm, part_r, (int)nbr, nullptr, 0, pub_of(c, c->gm_h), c->s);
                 HIPCHK(c, hipGetLastError());
-                CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
-                CHK(poll_mark(c));
                 if (ahead) launch_precond<T>(g, c->p.precond, c->fast, v1, scr, Z, act, c->s, FPC_HEAD);
-                CHK(poll_spin(c));
+                CHK(pub_wait(c));
                 opened = head = false;
                 if (c->gm_h->unit_ok) {
                     std::swap(c->PCorr, c->PCalt);
@@ -1226,13 +1237,13 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                     v0 = V;
                 }
                 if (!opened) {
-                    CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
+                    ask_status(c);
                     // the first Arnoldi step's first transform is queued behind the
-                    // status read-back, gated on st.active (0 exactly when the solve
-                    // has ended), so the GPU works while the host waits for the status
-                    CHK(poll_mark(c));
+                    // status, gated on st.active (0 exactly when the solve has
+                    // ended), so the GPU works while the host waits for the status
                     if (ahead) launch_precond<T>(g, c->p.precond, c->fast, V, scr, Z, act, c->s, FPC_HEAD);
-                    CHK(poll_spin(c));
+                    HIPCHK(c, hipGetLastError());
+                    CHK(pub_wait(c));
                     if (c->gm_h->outer_done) { final_res = true; break; }
                     head = ahead;
                 }
@@ -1273,14 +1284,14 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                 launch_fin_update(c->gm, part_z, (int)nbv, j, c->s);
                 HIPCHK(c, hipGetLastError());
                 if ((j + 1) % poll == 0 && j + 1 < kmax) {
-                    CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
+                    ask_status(c);
                     const bool qa = ahead_res && j == 0 && m + 1 < mmax;
-                    CHK(poll_mark(c));
                     if (qa) {
                         launch_fin_cycle(c->gm, c->s, 1);
                         launch_resid_upd<T>(g, c->pRhs, c->PCorr, Z, c->gm, c->PCalt, V, part_r, c->s, RU_GATED);
                     }
-                    CHK(poll_spin(c));
+                    HIPCHK(c, hipGetLastError());
+                    CHK(pub_wait(c));
                     if (!c->gm_h->active) {
                         one_step = (j == 0);
                         if (qa) {
@@ -1310,8 +1321,9 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
             launch_xupd<T>(Z, ldv, N, c->gm, c->PCorr, c->s);
         }
         if (!final_res) {
-            CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
-            CHK(poll_wait(c));
+            ask_status(c);
+            HIPCHK(c, hipGetLastError());
+            CHK(pub_wait(c));
         }
     }
     for (int m = 0; m < mmax && mode == GM_MODE_REF; m++) {
@@ -1332,10 +1344,9 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
             launch_resid_upd<T>(g, c->pRhs, c->PCorr, V, c->gm, c->PCalt, r, part_r, c->s, RU_UNIT);
             launch_precond<T>(g, c->p.precond, c->fast, r, scr, W, act, c->s);
             launch_norm2<T>(W, N, part_z, act, c->s);
-            launch_fin_unit(c->gm, part_r, (int)nbr, part_z, (int)nbv, c->s);
+            launch_fin_unit(c->gm, part_r, (int)nbr, part_z, (int)nbv, pub_of(c, c->gm_h), c->s);
             HIPCHK(c, hipGetLastError());
-            CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
-            CHK(poll_wait(c));
+            CHK(pub_wait(c));
             if (c->gm_h->unit_ok) std::swap(c->PCorr, c->PCalt);
             if (c->gm_h->outer_done) { final_res = true; break; }
         }
@@ -1361,8 +1372,9 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
             launch_fin_update(c->gm, part_z, (int)nbv, j, c->s);
             HIPCHK(c, hipGetLastError());
             if ((j + 1) % poll == 0 && j + 1 < kmax) {
-                CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
-                CHK(poll_wait(c));
+                ask_status(c);
+                HIPCHK(c, hipGetLastError());
+                CHK(pub_wait(c));
                 if (!c->gm_h->active) break;
             }
         }
@@ -1371,9 +1383,9 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
             Tscope ts(c, TBL_K_XUPD);
             launch_xupd<T>(V, ldv, N, c->gm, c->PCorr, c->s);
         }
+        ask_status(c);
         HIPCHK(c, hipGetLastError());
-        CHK(d2h(c, c->gm_h, &c->gm->st, sizeof(GmStatus)));
-        CHK(poll_wait(c));
+        CHK(pub_wait(c));
         if (c->gm_h->outer_done) break;
     }
     GmStatus st = *c->gm_h;
@@ -1391,10 +1403,8 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
     if (!final_res) {
         launch_resid<double>(g, c->pRhs, c->PCorr, nullptr, part_r, c->s);
         launch_fin_sum(part_r, (int)nbr, c->dd + DD_BNORM, c->s);
-        double r2 = 0.0;
-        CHK(d2h(c, &r2, c->dd + DD_BNORM, sizeof(double)));
-        CHK(poll_wait(c));
-        tr = sqrt(r2);
+        CHK(read_diag(c));
+        tr = sqrt(c->dh[DD_BNORM]);
     }
     if (cycles) *cycles = st.cycle;
     if (iters) *iters = st.total;
@@ -1439,11 +1449,19 @@ extern "C" int tbl_apply_bcs(tbl_ctx *c)
     return c->mixed ? bcs_impl<float>(c) : bcs_impl<double>(c);
 }
 
+// block partials of the divergence sum and of the mass fluxes; launch_fin_diag
+// (fin_diag) finishes them into the diagnostics record
 template <class T> static int div_impl(tbl_ctx *c)
 {
     Tscope ts(c, TBL_K_DIAG, 3.0 * (double)c->g.N * sizeof(T));      // the three velocity components
     launch_div_check<T>(c->g, F<T>(c->Ut), c->part, c->s);
-    launch_fin_sum(c->part, (int)resid_blocks(c->g), c->dd + DD_DIV, c->s);
+    HIPCHK(c, hipGetLastError());
+    return 0;
+}
+static int fin_diag(tbl_ctx *c, bool div, bool mass, bool pub)
+{
+    launch_fin_diag(c->part, div ? (int)resid_blocks(c->g) : 0, mass ? c->dd + DD_NCOUNT : nullptr, c->mass_denom, c->dd,
+                    pub ? pub_of(c, c->dh) : Pub(), c->s);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -1456,9 +1474,9 @@ extern "C" int tbl_div_check(tbl_ctx *c, double *div, double *signed_sum)
 {
     if (!c) return TBL_EARG;
     CHK(c->mixed ? div_impl<float>(c) : div_impl<double>(c));
-    double s = 0.0;
-    CHK(d2h(c, &s, c->dd + DD_DIV, sizeof(double)));
-    CHK(poll_wait(c));
+    CHK(fin_diag(c, true, false, true));
+    CHK(pub_wait(c));
+    const double s = c->dh[DD_DIV];
     if (signed_sum) *signed_sum = s;
     if (div) *div = div_metric(c, s);
     return 0;
@@ -1490,7 +1508,7 @@ extern "C" int tbl_div_check_noalloc(tbl_ctx *c, const void *Ut_dev, double *out
 template <class T> static int mass_impl(tbl_ctx *c)
 {
     Tscope ts(c, TBL_K_DIAG, 5.0 * (double)c->g.nY * c->g.nZ * sizeof(T));   // u on the five planes
-    launch_mass_flux<T>(c->g, F<T>(c->Ut), c->p.planes, c->mass_denom, c->dd + DD_MASS, c->dd + DD_NCOUNT, c->s);
+    launch_mass_flux<T>(c->g, F<T>(c->Ut), c->p.planes, c->dd + DD_NCOUNT, c->s);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -1498,9 +1516,10 @@ extern "C" int tbl_mass_flux(tbl_ctx *c, double *mass5)
 {
     if (!c) return TBL_EARG;
     CHK(c->mixed ? mass_impl<float>(c) : mass_impl<double>(c));
+    CHK(fin_diag(c, false, true, mass5 != nullptr));
     if (mass5) {
-        CHK(d2h(c, mass5, c->dd + DD_MASS, 5 * sizeof(double)));
-        CHK(poll_wait(c));
+        CHK(pub_wait(c));
+        memcpy(mass5, c->dh + DD_MASS, 5 * sizeof(double));
     }
     return 0;
 }
@@ -1546,14 +1565,10 @@ extern "C" int tbl_ke_guard(tbl_ctx *c, double *ke, int *guard)
     if (!c) return TBL_EARG;
     HIPCHK(c, hipMemsetAsync(c->guard, 0, sizeof(int), c->s));
     CHK(c->mixed ? ke_impl<float>(c) : ke_impl<double>(c));
-    double s = 0.0;
-    int gd = 0;
-    CHK(d2h(c, &s, c->dd + DD_KE, sizeof(double)));
-    CHK(d2h(c, &gd, c->guard, sizeof(int)));
-    CHK(poll_wait(c));
+    CHK(read_diag(c));
     const tbl_params &p = c->p;
-    if (ke) *ke = s / (double)(p.nX * (p.nY - 2) * (p.nZ - 2));
-    if (guard) *guard = gd;
+    if (ke) *ke = c->dh[DD_KE] / (double)(p.nX * (p.nY - 2) * (p.nZ - 2));
+    if (guard) memcpy(guard, c->dh + DD_GUARD, sizeof(int));
     return 0;
 }
 
@@ -1570,7 +1585,7 @@ extern "C" int tbl_wall_shear(tbl_ctx *c, double *tau)
     CHK(c->mixed ? tau_impl<float>(c) : tau_impl<double>(c));
     if (tau) {
         CHK(d2h(c, tau, c->tau, c->p.nX * sizeof(double)));
-        CHK(poll_wait(c));
+        HIPCHK(c, hipStreamSynchronize(c->s));
     }
     return 0;
 }
@@ -1581,7 +1596,7 @@ extern "C" int tbl_wall_shear_mean(tbl_ctx *c, double *tau_mean, double *cf, int
     if (c->p.wall_shear_window <= 0) return fail(c, TBL_ESTATE, "tbl_wall_shear_mean: wall_shear_window is 0 (off)");
     if (tau_mean) CHK(d2h(c, tau_mean, c->taumean, c->p.nX * sizeof(double)));
     if (cf) CHK(d2h(c, cf, c->cf, c->p.nX * sizeof(double)));
-    CHK(poll_wait(c));
+    HIPCHK(c, hipStreamSynchronize(c->s));
     if (nwindows) *nwindows = c->nwin;
     return 0;
 }
@@ -1633,13 +1648,19 @@ extern "C" int tbl_step(tbl_ctx *c, int nsteps, tbl_diag *diag)
             CHK(tbl_rescale(c));
             d.rescaled = 1;
         }
-        HIPCHK(c, hipMemsetAsync(c->guard, 0, sizeof(int), c->s));
+        // the kinetic energy reuses the divergence's partials, so they are
+        // finished before it; otherwise the finishing kernel is the step's last
         const bool ke_on = c->cnt > p.freq_tim_avg;
-        if (ke_on) CHK(c->mixed ? ke_impl<float>(c) : ke_impl<double>(c));
-        CHK(d2h(c, c->dh, c->dd, DD_NCOUNT * sizeof(double)));
+        CHK(fin_diag(c, true, true, !ke_on));
         int gd = 0;
-        CHK(d2h(c, &gd, c->guard, sizeof(int)));
-        CHK(poll_wait(c));
+        if (ke_on) {
+            HIPCHK(c, hipMemsetAsync(c->guard, 0, sizeof(int), c->s));
+            CHK(c->mixed ? ke_impl<float>(c) : ke_impl<double>(c));
+            CHK(read_diag(c));
+            memcpy(&gd, c->dh + DD_GUARD, sizeof(int));
+        } else {
+            CHK(pub_wait(c));
+        }
         d.div_signed = c->dh[DD_DIV];
         d.div = div_metric(c, d.div_signed);
         for (int q = 0; q < 5; q++) d.mass[q] = c->dh[DD_MASS + q];

@@ -142,6 +142,27 @@ __device__ __forceinline__ double block_sum(double v, double *sh, int t) {
     return r;
 }
 
+// Result that a kernel hands to the waiting host: the words at src go to
+// pinned host memory at dst, then the sequence word takes val (seq null: not
+// wanted).  The host spins on the sequence word (pub_wait); a copy command
+// behind the kernel, an event and its queries cost 10-20 us more, as much as
+// two or three kernels of a small grid.
+struct Pub {
+    unsigned *seq = nullptr;
+    void *dst = nullptr;
+    unsigned val = 0;
+};
+template <class S> __device__ __forceinline__ void publish(const Pub &P, const S *src)     // one thread
+{
+    static_assert(sizeof(S) % 8 == 0, "published in 8-byte words");
+    if (!P.seq) return;
+    const unsigned long long *s = reinterpret_cast<const unsigned long long *>(src);
+    unsigned long long *d = static_cast<unsigned long long *>(P.dst);
+    for (unsigned q = 0; q < sizeof(S) / 8; q++) d[q] = s[q];
+    __threadfence_system();
+    __hip_atomic_store(P.seq, P.val, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // GMRES control block, resident in device memory.  Arnoldi, Givens and the
 // stopping decisions run on the device; the host polls only `st`.
 struct GmStatus {

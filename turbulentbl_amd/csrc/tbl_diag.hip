@@ -124,7 +124,7 @@ __global__ __launch_bounds__(1024) void k_fin_div(const double *part, int nb, do
 }
 
 // ---------------------------------------------------------------- a13
-struct Planes { int p[5]; double denom; };
+struct Planes { int p[5]; };
 template <class T>
 __global__ __launch_bounds__(256) void k_mass_flux(Geo g, const T *__restrict__ Ut, Planes pl, double *__restrict__ part)
 {
@@ -146,17 +146,32 @@ __global__ __launch_bounds__(256) void k_mass_flux(Geo g, const T *__restrict__ 
     double s = block_sum<256>(a, sh, threadIdx.x);
     if (threadIdx.x == 0) part[q * MF_BLK + blockIdx.x] = s;
 }
-__global__ void k_mass_fin(const double *__restrict__ part, double denom, double *__restrict__ out)
+// last kernel of the diagnostics: the divergence sum (as k_fin_sum), the mass
+// fluxes, and the record to the host
+struct DiagRec { double w[9]; };
+__global__ __launch_bounds__(1024) void k_fin_diag(const double *part, int nb, const double *__restrict__ mpart,
+                                                  double denom, double *rec, Pub pub)
 {
-    const int q = threadIdx.x;
-    if (q >= 5) return;
+    __shared__ double sh[16];
+    if (mpart && threadIdx.x >= 64 && threadIdx.x < 69) {
+        const int q = threadIdx.x - 64;
+        double a = 0.0;
+        for (int b = 0; b < MF_BLK; b++) a += mpart[q * MF_BLK + b];
+        rec[1 + q] = a / denom;
+    }
     double a = 0.0;
-    for (int b = 0; b < MF_BLK; b++) a += part[q * MF_BLK + b];
-    out[q] = a / denom;
+#pragma unroll 8
+    for (int q = threadIdx.x; q < nb; q += 1024) a += part[q];
+    const double s = block_sum<1024>(a, sh, threadIdx.x);
+    if (threadIdx.x != 0) return;
+    if (nb > 0) rec[0] = s;
+    publish(pub, (const DiagRec *)rec);
+}
+void launch_fin_diag(const double *part, int nb, const double *mpart, double denom, double *rec, const Pub &pub, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_fin_diag, dim3(1), dim3(1024), 0, s, part, nb, mpart, denom, rec, pub);
 }
 
-// ---------------------------------------------------------------- a14
-// thread per (i,k); the span sum runs in the reference's j order
 template <class T>
 __global__ __launch_bounds__(256) void k_stats(Geo g, const T *__restrict__ Ut, double *__restrict__ sums)
 {
@@ -443,15 +458,12 @@ void launch_fin_div(const double *part, int nb, double nint, double *out2, hipSt
     hipLaunchKernelGGL(k_fin_div, dim3(1), dim3(1024), 0, s, part, nb, nint, out2);
 }
 template <class T>
-void launch_mass_flux(const Geo &g, const T *Ut, const int *planes, double denom, double *out5, double *part,
-                      hipStream_t s)
+void launch_mass_flux(const Geo &g, const T *Ut, const int *planes, double *part, hipStream_t s)
 {
     // part holds 5 * MF_BLK doubles
     Planes pl;
     for (int q = 0; q < 5; q++) pl.p[q] = planes[q];
-    pl.denom = denom;
     hipLaunchKernelGGL(k_mass_flux<T>, dim3(MF_BLK, 5), dim3(256), 0, s, g, Ut, pl, part);
-    hipLaunchKernelGGL(k_mass_fin, dim3(1), dim3(64), 0, s, (const double *)part, denom, out5);
 }
 template <class T>
 void launch_stats(const Geo &g, const T *Ut, double *sums, hipStream_t s)
@@ -494,7 +506,7 @@ void launch_tau_window(const Geo &g, int window, double *acc, double *mean, doub
 
 #define TBL_INST(T)                                                                                           \
     template void launch_div_check<T>(const Geo &, const T *, double *, hipStream_t);                         \
-    template void launch_mass_flux<T>(const Geo &, const T *, const int *, double, double *, double *, hipStream_t); \
+    template void launch_mass_flux<T>(const Geo &, const T *, const int *, double *, hipStream_t); \
     template void launch_stats<T>(const Geo &, const T *, double *, hipStream_t);                             \
     template void launch_rescale<T>(const Geo &, int, int, const T *, double *, double *, RecDev *, double *,  \
                                     int *, double *, double *, double *, double *, double *, hipStream_t);    \

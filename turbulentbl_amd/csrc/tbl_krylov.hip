@@ -85,15 +85,32 @@ __device__ __forceinline__ double fin_sum(const double *part, int nb, double *sh
 // finishing blocks of the grid-wide reductions (up to ~16k partials)
 static constexpr int FB = 1024;
 
-// control block of a new solve: zeroed, then the solve's parameters.  A
-// kernel rather than a copy: the block is 33 KB, and a copy from pageable host
-// memory holds the host until it has been staged.
-__global__ __launch_bounds__(FB) void k_gm_init(GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax,
-                                               int mode)
+// Start of a solve: the control block (the last workgroup), zeroed and given the
+// solve's parameters, and the zero faces of the PCorr buffers, dnssetbl.f90:451-460
+// (the others).  A kernel rather than a copy: the block is 33 KB, and a copy
+// from pageable host memory holds the host until it has been staged.
+__global__ __launch_bounds__(VB) void k_gm_init(Geo g, GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax,
+                                               int mode, double *PC, double *PC2)
 {
+    if (blockIdx.x + 1 < gridDim.x) {
+        const long nX = g.nX, nY = g.nY, nZ = g.nZ, fz = nX * nY, fy = nX * nZ, fx = nY * nZ;
+        long t = (long)blockIdx.x * VB + threadIdx.x, x;
+        if (t < 2 * fz) {
+            x = t % fz + (t < fz ? 0 : fz * (nZ - 1));
+        } else if ((t -= 2 * fz) < 2 * fy) {
+            const long q = t % fy;
+            x = q % nX + nX * ((t < fy ? 0 : nY - 1) + nY * (q / nX));
+        } else {
+            if ((t -= 2 * fy) >= 2 * fx) return;
+            x = (t < fx ? 0 : nX - 1) + nX * (t % fx);
+        }
+        PC[x] = 0.0;
+        if (PC2) PC2[x] = 0.0;
+        return;
+    }
     static_assert(sizeof(GmCtrl) % sizeof(double) == 0, "GmCtrl is cleared in doubles");
     double *w = reinterpret_cast<double *>(c);
-    for (unsigned q = threadIdx.x; q < sizeof(GmCtrl) / sizeof(double); q += FB) w[q] = 0.0;
+    for (unsigned q = threadIdx.x; q < sizeof(GmCtrl) / sizeof(double); q += VB) w[q] = 0.0;
     __syncthreads();
     if (threadIdx.x == 0) {
         c->errtol = errtol;
@@ -103,6 +120,19 @@ __global__ __launch_bounds__(FB) void k_gm_init(GmCtrl *c, double errtol, double
         c->mode = mode;
         c->st.sumnor = 1.0;
     }
+}
+
+__global__ __launch_bounds__(64) void k_publish(const unsigned long long *__restrict__ src, int words, Pub P)
+{
+    unsigned long long *d = static_cast<unsigned long long *>(P.dst);
+    for (int q = threadIdx.x; q < words; q += 64) d[q] = src[q];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(P.seq, P.val, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+void launch_publish(const void *src, int words, const Pub &pub, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, (const unsigned long long *)src, words, pub);
 }
 
 // Start of a cycle in true-residual mode from the residual norm res (one thread)
@@ -134,7 +164,7 @@ __device__ __forceinline__ void open_cycle(GmCtrl *c, double rho)
 // mode).  dnssetbl.f90:536-546.
 __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_r, int nb_r,
                                                  const double *part_z, int nb_z, int first,
-                                                 const double *part_b)
+                                                 const double *part_b, Pub pub)
 {
     __shared__ double sh[FB / 64];
     __shared__ double rho_s;
@@ -152,8 +182,9 @@ __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_
     st.cycle += 1;
     st.kit = 0;
     st.rho = rho;
-    if (!(rho == rho) || !(st.true_res == st.true_res)) { st.nan = 1; st.active = 0; st.outer_done = 1; return; }
-    if (c->mode == GM_MODE_REF) {
+    if (!(rho == rho) || !(st.true_res == st.true_res)) {
+        st.nan = 1; st.active = 0; st.outer_done = 1;
+    } else if (c->mode == GM_MODE_REF) {
         if (first) st.sumnor = rho;
         st.sumav = rho / st.sumnor;
         const bool go = (st.sumav > c->errtol) && rho > 0.0;
@@ -162,6 +193,7 @@ __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_
     } else {
         start_true(c, rho);
     }
+    publish(pub, &st);
 }
 
 // A cycle whose preconditioner inverts A nearly exactly needs no Arnoldi step:
@@ -176,14 +208,17 @@ __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_
 // Otherwise the cycle stays open and the host runs its Arnoldi steps from
 // z_0 as if nothing had been tried.
 __global__ __launch_bounds__(FB) void k_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z,
-                                                int nb_z)
+                                                int nb_z, Pub pub)
 {
     __shared__ double sh[FB / 64];
     __shared__ double res_s;
     __shared__ int ok_s;
     GmStatus &st = c->st;
     if (!st.active) {
-        if (threadIdx.x == 0) st.unit_ok = 0;
+        if (threadIdx.x == 0) {
+            st.unit_ok = 0;
+            publish(pub, &st);
+        }
         return;
     }
     const bool ref = c->mode == GM_MODE_REF;
@@ -204,6 +239,7 @@ __global__ __launch_bounds__(FB) void k_fin_unit(GmCtrl *c, const double *part_r
         }
         if (ok) { st.total += 1; st.kit = ref ? 1 : 0; st.rho = ref ? rho : res; st.true_res = res; }
         st.unit_ok = ok ? 1 : 0;
+        publish(pub, &st);
         ok_s = ok && !ref;
         res_s = res;
     }
@@ -439,17 +475,20 @@ void launch_norm2(const T *x, long N, double *part, const int *active, hipStream
     hipLaunchKernelGGL(k_norm2<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, x, N, part, active);
 }
 void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
-                      const double *part_b)
+                      const double *part_b, const Pub &pub)
 {
-    hipLaunchKernelGGL(k_fin_start, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, first, part_b);
+    hipLaunchKernelGGL(k_fin_start, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, first, part_b, pub);
 }
-void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, hipStream_t s)
+void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, const Pub &pub, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fin_unit, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z);
+    hipLaunchKernelGGL(k_fin_unit, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, pub);
 }
-void launch_gm_init(GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax, int mode, hipStream_t s)
+void launch_gm_init(const Geo &g, GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax, int mode, double *PC,
+                    double *PC2, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_gm_init, dim3(1), dim3(FB), 0, s, c, errtol, inner_tol, kmax, mmax, mode);
+    const long faces = 2 * ((long)g.nX * g.nY + (long)g.nX * g.nZ + (long)g.nY * g.nZ);
+    hipLaunchKernelGGL(k_gm_init, dim3((unsigned)((faces + VB - 1) / VB + 1)), dim3(VB), 0, s, g, c, errtol, inner_tol, kmax,
+                       mmax, mode, PC, PC2);
 }
 template <class T>
 void launch_dots(const T *V, long ldv, int j, long N, const GmCtrl *c, double *part, hipStream_t s)

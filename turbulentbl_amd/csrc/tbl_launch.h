@@ -19,7 +19,8 @@ template <class T> void launch_momentum_rhs(const Geo &g, const T *Ut, const T *
                                             double *hpart = nullptr);
 template <class T> void launch_helm_resid(const Geo &g, const T *Q, const T *Ut, const void *ctrl, double *part, int first, hipStream_t s);
 void launch_helm_fin(const Geo &g, void *ctrl, const double *part, int it, double errorstop, double floor_coef, hipStream_t s,
-                     int nb = 0);
+                     int nb = 0, const Pub &pub = Pub());
+void launch_gs_init(void *ctrl, hipStream_t s);          // all components active, sums zero
 template <class T> void launch_helm_sweep(const Geo &g, const T *Q, T *Ut, const void *ctrl, int colour, hipStream_t s);
 template <class T> void launch_helm_zline(const Geo &g, const T *Q, T *Ut, const T *zf, const void *ctrl, int colour, hipStream_t s);
 // one pass of the z-line zebra sweep: x neighbours from cur, span rows from
@@ -27,7 +28,8 @@ template <class T> void launch_helm_zline(const Geo &g, const T *Q, T *Ut, const
 template <class T> void launch_helm_zebra(const Geo &g, const T *Q, const T *cur, const T *ysrc, T *dst, const T *zf,
                                           const void *ctrl, int colour, hipStream_t s);
 // boundary / ghost values of the three velocity components, src -> dst
-template <class T> void launch_copy_faces3(const Geo &g, const T *src, T *dst, hipStream_t s);
+// (and the Gauss-Seidel control block of a new solve, as launch_gs_init)
+template <class T> void launch_copy_faces3(const Geo &g, const T *src, T *dst, void *ctrl, hipStream_t s);
 // per-slab lexicographic Gauss-Seidel sweep (snapshot of the slabs' ghost
 // planes into halo, then the sweep); threads a slab kernel needs, 0 if the
 // slabs are too thick for one workgroup
@@ -35,7 +37,6 @@ template <class T> void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *halo
                                         hipStream_t s);
 int slab_threads(const Geo &g, int nkmax);
 size_t gs_ctrl_bytes();
-void gs_ctrl_init(void *host, int active_mask);
 void gs_ctrl_read(const void *host, int *active, int *sweeps, double *res);
 // gate (optional): the Gauss-Seidel control block; the launch does nothing
 // while any of its components is active
@@ -98,11 +99,15 @@ void launch_fill(double *x, double v, long n, hipStream_t s);
 template <class T> void launch_norm2(const T *x, long N, double *part, const int *active, hipStream_t s);
 // part_b (optional): nb_r block partials of ||pRhs||^2 (start of a true-residual solve)
 void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
-                      const double *part_b = nullptr);
+                      const double *part_b = nullptr, const Pub &pub = Pub());
 // judges the tentative unit step: residual partials part_r, and the block
 // partials of its preconditioned residual (part_z, reference's stopping rule)
-void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, hipStream_t s);
-void launch_gm_init(GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax, int mode, hipStream_t s);
+void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, const Pub &pub, hipStream_t s);
+// start of a pressure solve: the control block, and zero faces of PC (and of PC2)
+void launch_gm_init(const Geo &g, GmCtrl *c, double errtol, double inner_tol, int kmax, int mmax, int mode, double *PC,
+                    double *PC2, hipStream_t s);
+// words 8-byte words at src to the host
+void launch_publish(const void *src, int words, const Pub &pub, hipStream_t s);
 template <class T> void launch_dots(const T *V, long ldv, int j, long N, const GmCtrl *c, double *part, hipStream_t s);
 void launch_fin_dots(GmCtrl *c, const double *part, int nb, int j, hipStream_t s);
 template <class T> void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s);
@@ -121,8 +126,10 @@ void launch_fin_sum(const double *part, int nb, double *out, hipStream_t s);
 // out2[0] = |sum of part| / nint, out2[1] = the sum
 void launch_fin_div(const double *part, int nb, double nint, double *out2, hipStream_t s);
 #define MF_BLK 64   // mass-flux partial blocks per plane
-template <class T> void launch_mass_flux(const Geo &g, const T *Ut, const int *planes, double denom, double *out5,
-                                         double *part, hipStream_t s);
+template <class T> void launch_mass_flux(const Geo &g, const T *Ut, const int *planes, double *part, hipStream_t s);
+// rec[0] = sum of the nb divergence partials (nb > 0), rec[1..5] = mass flux
+// (mpart given); publishes the nine words of rec
+void launch_fin_diag(const double *part, int nb, const double *mpart, double denom, double *rec, const Pub &pub, hipStream_t s);
 template <class T> void launch_stats(const Geo &g, const T *Ut, double *sums, hipStream_t s);
 template <class T> void launch_rescale(const Geo &g, int i_rec0, int nsamples, const T *Ut, double *sums,
                                        double *avg, RecDev *rec, double *Wt, int *newk, double *bltkns,

@@ -592,36 +592,62 @@ __global__ __launch_bounds__(RT_T) void k_helm_resid(Geo g, const T *__restrict_
 // adds: stop once the L1 residual is at the roundoff level of the stored
 // field, floor_coef * ||Q||_1, which the reference's 1e-6 relative target
 // cannot go below in single precision.
+// One block; the sums of the three components (and, on the first pass, of |Q|)
+// are formed together: per thread in fixed strided order, then the fixed order
+// of block_sum.  Publishes the control block.
 __global__ __launch_bounds__(1024) void k_helm_fin(GsCtrl *ctrl, const double *__restrict__ part, int nb, int it,
-                                                  double errorstop, double floor_coef)
+                                                  double errorstop, double floor_coef, Pub pub)
 {
-    __shared__ double sh[16];
+    __shared__ double sh[6][16];
     const double tiny = (double)1e-12f;    // REAL(4) literal, dnssetbl.f90:392
+    const int t = threadIdx.x;
+    // an ended component's old partials are summed too and not used: a test
+    // around the loads would keep them from overlapping
+    double a[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int q = t; q < nb; q += 1024)
+#pragma unroll
+        for (int p = 0; p < 3; p++) a[p] += part[(long)p * nb + q];
+    if (it == 1) {
+#pragma unroll 4
+        for (int q = t; q < nb; q += 1024)
+#pragma unroll
+            for (int p = 3; p < 6; p++) a[p] += part[(long)p * nb + q];
+    }
+#pragma unroll
+    for (int p = 0; p < 6; p++) {
+        const double w = wave_sum(a[p]);
+        if ((t & 63) == 0) sh[p][t >> 6] = w;
+    }
+    __syncthreads();
+    if (t < 3 && ctrl->active[t]) {
+        double res = 0.0, qn = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) { res += sh[t][q]; qn += sh[3 + t][q]; }
+        if (it == 1) { ctrl->sumnor[t] = res; ctrl->qnorm[t] = qn; }
+        ctrl->res[t] = res;
+        const double sumav = res / ctrl->sumnor[t];
+        if (sumav < errorstop || res < tiny || (floor_coef > 0.0 && res <= floor_coef * ctrl->qnorm[t])) {
+            ctrl->active[t] = 0;
+            ctrl->sweeps[t] = it - 1;
+        }
+    }
+    __syncthreads();
+    if (t == 0) publish(pub, ctrl);
+}
+// control block of a new solve (one thread)
+__device__ __forceinline__ void gs_start(GsCtrl *c)
+{
     for (int p = 0; p < 3; p++) {
-        if (!ctrl->active[p]) continue;
-        double a = 0.0;
-        // fixed per-thread strided order, then fixed block reduction: deterministic
-#pragma unroll 8
-        for (int q = threadIdx.x; q < nb; q += 1024) a += part[(long)p * nb + q];
-        double res = block_sum<1024>(a, sh, threadIdx.x);
-        double qn = 0.0;
-        if (it == 1) {
-            double aq = 0.0;
-            for (int q = threadIdx.x; q < nb; q += 1024) aq += part[(long)(3 + p) * nb + q];
-            qn = block_sum<1024>(aq, sh, threadIdx.x);
-        }
-        if (threadIdx.x == 0) {
-            if (it == 1) { ctrl->sumnor[p] = res; ctrl->qnorm[p] = qn; }
-            ctrl->res[p] = res;
-            double sumav = res / ctrl->sumnor[p];
-            if (sumav < errorstop || res < tiny || (floor_coef > 0.0 && res <= floor_coef * ctrl->qnorm[p])) {
-                ctrl->active[p] = 0;
-                ctrl->sweeps[p] = it - 1;
-            }
-        }
-        __syncthreads();
+        c->sumnor[p] = 0; c->res[p] = 0; c->qnorm[p] = 0;
+        c->active[p] = 1; c->sweeps[p] = 0;
     }
 }
+__global__ void k_gs_init(GsCtrl *c)
+{
+    if (threadIdx.x == 0) gs_start(c);
+}
+void launch_gs_init(void *ctrl, hipStream_t s) { hipLaunchKernelGGL(k_gs_init, dim3(1), dim3(64), 0, s, (GsCtrl *)ctrl); }
 
 // one colour of a red-black sweep; thread per same-colour node along i
 template <class T>
@@ -968,8 +994,9 @@ __attribute__((amdgpu_waves_per_eu((sizeof(T) == 4 && LC == 16) ? 6 : 1))) void 
 // the boundary and ghost values (i = 0, nX-1 columns, j = 0, nY-1 rows,
 // k = 0, nZ-1 planes) of the three velocity components, src -> dst
 template <class T>
-__global__ void k_copy_faces3(Geo g, const T *__restrict__ src, T *__restrict__ dst)
+__global__ void k_copy_faces3(Geo g, const T *__restrict__ src, T *__restrict__ dst, GsCtrl *ctrl)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) gs_start(ctrl);
     const long nX = g.nX, nY = g.nY, nZ = g.nZ, N = g.N;
     const long fz = nX * nY, fy = nX * nZ, fx = nY * nZ, per = 2 * (fz + fy + fx);
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1284,30 +1311,33 @@ __global__ void k_zero_faces(Geo g, T *x)
 
 // ----------------------------------------------------------------------------
 // a10: PCorr extrapolation (dnssetbl.f90:697-708), then pressure update and
-// projection (:711-726).  Three face kernels keep the reference's order:
-// wall-normal faces, span copies, inflow/outflow faces.
+// projection (:711-726).  The reference sets the wall-normal faces, copies the
+// span ghosts, then sets the inflow and outflow faces.  k_pc_zspan does the
+// first two: the value of an edge row of a wall-normal face goes to its ghost
+// by the thread that formed it.  (The third in k_project, by the threads of the
+// cells next to those faces, made that kernel a third slower.)
 // ----------------------------------------------------------------------------
-__global__ void k_pc_zfaces(Geo g, double *PC)
+__global__ void k_pc_zspan(Geo g, double *PC)
 {
-    const int nX = g.nX, nY = g.nY, nZ = g.nZ;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y + 1;
-    if (i >= nX || j > nY - 2) return;
-    const long s = g.sZ, b = (long)i + (long)nX * j;
-    PC[b] = ((4.0 * PC[b + s]) - PC[b + 2 * s]) / 3.0;
-    const long t = b + s * (nZ - 1);
-    PC[t] = (5.0 * PC[t - s] + (-4.0 * PC[t - 2 * s] + PC[t - 3 * s])) / 2.0;
+    const long nX = g.nX, nY = g.nY, nZ = g.nZ, s = g.sZ, nz = nX * (nY - 2);
+    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nz) {                                                // wall-normal faces at (i, j)
+        const long i = t % nX, j = t / nX + 1, b = i + nX * j, e = b + s * (nZ - 1);
+        const double lo = ((4.0 * PC[b + s]) - PC[b + 2 * s]) / 3.0;
+        const double hi = (5.0 * PC[e - s] + (-4.0 * PC[e - 2 * s] + PC[e - 3 * s])) / 2.0;
+        PC[b] = lo;
+        PC[e] = hi;
+        if (j == 1) { PC[b + nX * (nY - 2)] = lo; PC[e + nX * (nY - 2)] = hi; }
+        if (j == nY - 2) { PC[i] = lo; PC[i + s * (nZ - 1)] = hi; }
+        return;
+    }
+    t -= nz;                                                     // span ghosts at (i, k)
+    if (t >= nX * (nZ - 2)) return;
+    const long b = t % nX + s * (t / nX + 1);
+    PC[b] = PC[b + nX * (nY - 2)];
+    PC[b + nX * (nY - 1)] = PC[b + nX];
 }
-__global__ void k_pc_span(Geo g, double *PC)
-{
-    const int nX = g.nX, nY = g.nY;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (i >= nX) return;
-    const long b = (long)i + (long)g.sZ * k;
-    PC[b] = PC[b + (long)nX * (nY - 2)];
-    PC[b + (long)nX * (nY - 1)] = PC[b + (long)nX];
-}
+
 __global__ void k_pc_xfaces(Geo g, double *PC)
 {
     const int nX = g.nX, nY = g.nY, nZ = g.nZ;
@@ -1344,62 +1374,62 @@ __global__ __launch_bounds__(256) void k_project(Geo g, const double *__restrict
 // ----------------------------------------------------------------------------
 // a11: velocity and pressure boundary conditions (dnssetbl.f90:728-797)
 // ----------------------------------------------------------------------------
-// wall (k=1: no slip, w = wall_w control hook) and top (k=nZ: 2nd-order zero gradient)
+// The reference sets wall and top, outflow and span ghosts one after the
+// other, for the velocity and then for the pressure.  Each of the two groups is
+// one launch: a thread forms the value of its own boundary point from interior
+// and inflow points only (a point of two groups from the first group's formula
+// again), and the value of an edge row goes to its ghost as well, so no thread
+// reads what another writes.  A launch of these few points costs its latency:
+// at 64x32x48 six of them took 17 us a step and the gaps between them, these
+// two 10.5 us.
 template <class T>
-__global__ void k_bc_vel_z(Geo g, T *Ut, const double *wall_w)
+__global__ void k_bc_vel(Geo g, T *Ut, const double *__restrict__ wall_w)
 {
-    const int nX = g.nX, nY = g.nY, nZ = g.nZ;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y + 1;
-    if (i >= nX || j > nY - 2) return;
-    const long s = g.sZ, b = (long)i + (long)nX * j, top = b + s * (nZ - 1);
+    const long nX = g.nX, nY = g.nY, nZ = g.nZ, s = g.sZ;
+    const long nz = nX * (nY - 2), nx = (nY - 2) * (nZ - 2), ny = (nX - 1) * (nZ - 2);
+    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nz) {
+        // wall (no slip, w = wall_w control hook) and top (2nd-order zero
+        // gradient) at (i, j); i = nX-1 extrapolates their values (outflow)
+        const long i = t % nX, j = t / nX + 1, b = i + nX * j, e = b + s * (nZ - 1);
+        for (int p = 0; p < 3; p++) {
+            T *u = Ut + (long)p * g.N;
+            auto wall = [&](long q) { return (p == 2 && wall_w) ? (T)wall_w[q] : T(0.0); };
+            auto top = [&](long q) { return (T(4.0) * u[q - s] - u[q - 2 * s]) / T(3.0); };
+            const bool out = i == nX - 1;
+            const T lo = out ? (T(4.0) * wall(b - 1) - wall(b - 2)) / T(3.0) : wall(b);
+            const T hi = out ? (T(4.0) * top(e - 1) - top(e - 2)) / T(3.0) : top(e);
+            u[b] = lo;
+            u[e] = hi;
+            if (j == 1) { u[b + nX * (nY - 2)] = lo; u[e + nX * (nY - 2)] = hi; }
+            if (j == nY - 2) { u[i] = lo; u[i + s * (nZ - 1)] = hi; }
+        }
+        return;
+    }
+    if ((t -= nz) < nx) {                                        // outflow at (j, k)
+        const long j = t % (nY - 2) + 1, r = s * (t / (nY - 2) + 1) + nX - 1, e = r + nX * j;
+        for (int p = 0; p < 3; p++) {
+            T *u = Ut + (long)p * g.N;
+            const T v = (T(4.0) * u[e - 1] - u[e - 2]) / T(3.0);
+            u[e] = v;
+            if (j == 1) u[r + nX * (nY - 1)] = v;
+            if (j == nY - 2) u[r] = v;
+        }
+        return;
+    }
+    if ((t -= nx) >= ny) return;                                 // span ghosts at (i < nX-1, k)
+    const long b = t % (nX - 1) + s * (t / (nX - 1) + 1);
     for (int p = 0; p < 3; p++) {
         T *u = Ut + (long)p * g.N;
-        u[b] = (p == 2 && wall_w) ? (T)wall_w[b] : T(0.0);
-    }
-    for (int p = 0; p < 3; p++) {
-        T *u = Ut + (long)p * g.N;
-        u[top] = (T(4.0) * u[top - s] - u[top - 2 * s]) / T(3.0);
+        u[b] = u[b + nX * (nY - 2)];
+        u[b + nX * (nY - 1)] = u[b + nX];
     }
 }
-// outflow (i=nX) for every k, after the wall/top values are set
+// bottom pressure (from wall-normal momentum) and top pressure, interior i and j
 template <class T>
-__global__ void k_bc_vel_out(Geo g, T *Ut)
+__device__ __forceinline__ void bc_press_z(const Geo &g, const T *__restrict__ Ut, const T *Press, long b, T &lo, T &hi)
 {
-    const int nX = g.nX, nY = g.nY, nZ = g.nZ;
-    const int j = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int k = blockIdx.y;
-    if (j > nY - 2 || k >= nZ) return;
-    const long e = (long)nX - 1 + (long)nX * ((long)j + (long)nY * k);
-    for (int p = 0; p < 3; p++) {
-        T *u = Ut + (long)p * g.N;
-        u[e] = (T(4.0) * u[e - 1] - u[e - 2]) / T(3.0);
-    }
-}
-// span periodic ghosts j=1 <- nY-1, j=nY <- 2 for ncomp components
-template <class T>
-__global__ void k_span_copy(Geo g, T *f, int ncomp)
-{
-    const int nX = g.nX, nY = g.nY;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (i >= nX) return;
-    for (int p = 0; p < ncomp; p++) {
-        T *u = f + (long)p * g.N;
-        const long b = (long)i + (long)g.sZ * k;
-        u[b] = u[b + (long)nX * (nY - 2)];
-        u[b + (long)nX * (nY - 1)] = u[b + (long)nX];
-    }
-}
-// bottom (from wall-normal momentum) and top pressure, interior i and j
-template <class T>
-__global__ void k_bc_press_z(Geo g, const T *__restrict__ Ut, T *__restrict__ Press)
-{
-    const int nX = g.nX, nY = g.nY, nZ = g.nZ;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y + 1;
-    if (i > nX - 2 || j > nY - 2) return;
-    const long s = g.sZ, b = (long)i + (long)nX * j;
+    const long s = g.sZ, nX = g.nX;
     const T *W = Ut + 2 * g.N;
     const double dx = g.dx, dy = g.dy, df1 = g.df1, df2 = g.df2, Re = g.Re;
     const double w1 = W[b], w2 = W[b + s], w3 = W[b + 2 * s];
@@ -1408,26 +1438,23 @@ __global__ void k_bc_press_z(Geo g, const T *__restrict__ Ut, T *__restrict__ Pr
     const double rt2 = ((double)W[b - nX] - 2.0 * w1 + (double)W[b + nX]) / (dy * dy);
     const double rt3 = (2.0 * df1 * w3 - 2.0 * df2 * w2 + 2.0 * (df2 - df1) * w1) / (df1 * (df2 * df2) - (df2 * (df1 * df1)));
     const double rt12 = -rt11 + (rt1 + rt2 + rt3) / Re;
-    Press[b] = (T)((double)Press[b + s] - rt12 * df1);
-    const long t = b + s * (nZ - 1);
+    lo = (T)((double)Press[b + s] - rt12 * df1);
+    const long t = b + s * (g.nZ - 1);
     const double r1 = (11.0 * (double)W[t] - 18.0 * (double)W[t - s] + 9.0 * (double)W[t - 2 * s] - 2.0 * (double)W[t - 3 * s]) / (6.0 * g.dXi);
-    const double r2 = (r1 * g.JacInv[nZ - 1]);
-    Press[t] = (T)(r2 / Re);
+    const double r2 = (r1 * g.JacInv[g.nZ - 1]);
+    hi = (T)(r2 / Re);
 }
-// outflow and inflow pressure, k = 2..nZ-1 (inflow from streamwise momentum)
+// inflow (from streamwise momentum) and outflow pressure of row c = (0, j, k), k = 2..nZ-1
 template <class T>
-__global__ void k_bc_press_x(Geo g, const T *__restrict__ Ut, const T *__restrict__ Utold, T *__restrict__ Press)
+__device__ __forceinline__ void bc_press_x(const Geo &g, const T *__restrict__ Ut, const T *__restrict__ Utold,
+                                           const T *Press, long c, int k, T &in, T &out)
 {
-    const int nX = g.nX, nY = g.nY, nZ = g.nZ;
-    const int j = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int k = blockIdx.y + 1;
-    if (j > nY - 2 || k > nZ - 2) return;
+    const int nX = g.nX, nZ = g.nZ;
     const long N = g.N, sk = g.sZ;
-    const long c = (long)nX * ((long)j + (long)nY * k);
     const T *U = Ut, *V = Ut + N, *W = Ut + 2 * N;
     const double dx = g.dx, dy = g.dy, dXi = g.dXi, Re = g.Re, dt = g.dt;
     const long e = c + nX - 1;
-    Press[e] = (T)((3.0 * (double)U[e] - 4.0 * (double)U[e - 1] + (double)U[e - 2]) / (2.0 * dx * Re));
+    out = (T)((3.0 * (double)U[e] - 4.0 * (double)U[e - 1] + (double)U[e - 2]) / (2.0 * dx * Re));
     const double u1 = U[c];
     const double rt1 = u1 * (((double)U[c + 1] - u1) / (dx));
     const double rt2 = (double)V[c] * (((double)U[c + nX] - (double)U[c - nX]) / (2.0 * dy));
@@ -1448,7 +1475,40 @@ __global__ void k_bc_press_x(Geo g, const T *__restrict__ Ut, const T *__restric
     const double Ji = g.JacInv[k];
     rt6 = rt6 * (Ji * Ji) - g.Jac2[k] * rt11 * (Ji * Ji * Ji);
     const double rt12 = (u1 - (double)Utold[c]) / dt;
-    Press[c] = (T)(((2 * dx * ((rt12 + rt1 + rt2 + rt3 * Ji) - ((rt4 + rt5 + rt6) / Re))) - (double)Press[c + 2] + (4 * (double)Press[c + 1])) / 3.0);
+    in = (T)(((2 * dx * ((rt12 + rt1 + rt2 + rt3 * Ji) - ((rt4 + rt5 + rt6) / Re))) - (double)Press[c + 2] + (4 * (double)Press[c + 1])) / 3.0);
+}
+template <class T>
+__global__ void k_bc_press(Geo g, const T *__restrict__ Ut, const T *__restrict__ Utold, T *Press)
+{
+    const long nX = g.nX, nY = g.nY, nZ = g.nZ, s = g.sZ;
+    const long nz = (nX - 2) * (nY - 2), nx = (nY - 2) * (nZ - 2), ny = nX * nZ;
+    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nz) {                                                // bottom and top at (i, j)
+        const long i = t % (nX - 2) + 1, j = t / (nX - 2) + 1, b = i + nX * j, e = b + s * (nZ - 1);
+        T lo, hi;
+        bc_press_z<T>(g, Ut, Press, b, lo, hi);
+        Press[b] = lo;
+        Press[e] = hi;
+        if (j == 1) { Press[b + nX * (nY - 2)] = lo; Press[e + nX * (nY - 2)] = hi; }
+        if (j == nY - 2) { Press[i] = lo; Press[i + s * (nZ - 1)] = hi; }
+        return;
+    }
+    if ((t -= nz) < nx) {                                        // inflow and outflow at (j, k)
+        const long j = t % (nY - 2) + 1, k = t / (nY - 2) + 1, r = s * k, c = r + nX * j;
+        T in, out;
+        bc_press_x<T>(g, Ut, Utold, Press, c, (int)k, in, out);
+        Press[c] = in;
+        Press[c + nX - 1] = out;
+        if (j == 1) { Press[r + nX * (nY - 1)] = in; Press[r + nX * (nY - 1) + nX - 1] = out; }
+        if (j == nY - 2) { Press[r] = in; Press[r + nX - 1] = out; }
+        return;
+    }
+    if ((t -= nx) >= ny) return;                                 // span ghosts of the other (i, k): both inside, or both edges
+    const long i = t % nX, k = t / nX, b = i + s * k;
+    const bool ei = i == 0 || i == nX - 1, ek = k == 0 || k == nZ - 1;
+    if (ei != ek) return;
+    Press[b] = Press[b + nX * (nY - 2)];
+    Press[b + nX * (nY - 1)] = Press[b + nX];
 }
 
 // Utold(1,:,:,1) = Ut(1,:,:,1): the part of Utold = Ut (dnssetbl.f90:257)
@@ -1609,10 +1669,10 @@ void launch_helm_resid(const Geo &g, const T *Q, const T *Ut, const void *ctrl, 
     hipLaunchKernelGGL(k_helm_resid<T>, grid, dim3(RT_T), 0, s, g, Q, Ut, (const GsCtrl *)ctrl, part, first, kc);
 }
 void launch_helm_fin(const Geo &g, void *ctrl, const double *part, int it, double errorstop, double floor_coef,
-                     hipStream_t s, int nb)
+                     hipStream_t s, int nb, const Pub &pub)
 {
     hipLaunchKernelGGL(k_helm_fin, dim3(1), dim3(1024), 0, s, (GsCtrl *)ctrl, part, nb > 0 ? nb : (int)resid_blocks(g),
-                       it, errorstop, floor_coef);
+                       it, errorstop, floor_coef, pub);
 }
 template <class T>
 void launch_helm_sweep(const Geo &g, const T *Q, T *Ut, const void *ctrl, int colour, hipStream_t s)
@@ -1658,20 +1718,12 @@ void launch_helm_zebra(const Geo &g, const T *Q, const T *cur, const T *ysrc, T 
                            (const GsCtrl *)ctrl, colour, C, nbx, nblk, pw);
 }
 template <class T>
-void launch_copy_faces3(const Geo &g, const T *src, T *dst, hipStream_t s)
+void launch_copy_faces3(const Geo &g, const T *src, T *dst, void *ctrl, hipStream_t s)
 {
     const long per = 2 * ((long)g.nX * g.nY + (long)g.nX * g.nZ + (long)g.nY * g.nZ);
-    hipLaunchKernelGGL(k_copy_faces3<T>, dim3((unsigned)((3 * per + 255) / 256)), dim3(256), 0, s, g, src, dst);
+    hipLaunchKernelGGL(k_copy_faces3<T>, dim3((unsigned)((3 * per + 255) / 256)), dim3(256), 0, s, g, src, dst, (GsCtrl *)ctrl);
 }
 size_t gs_ctrl_bytes() { return sizeof(GsCtrl); }
-void gs_ctrl_init(void *host, int nactive_mask)
-{
-    GsCtrl *c = (GsCtrl *)host;
-    for (int p = 0; p < 3; p++) {
-        c->sumnor[p] = 0; c->res[p] = 0; c->qnorm[p] = 0;
-        c->active[p] = (nactive_mask >> p) & 1; c->sweeps[p] = 0;
-    }
-}
 void gs_ctrl_read(const void *host, int *active, int *sweeps, double *res)
 {
     const GsCtrl *c = (const GsCtrl *)host;
@@ -2052,23 +2104,20 @@ template void launch_zero_faces<float>(const Geo &, float *, hipStream_t);
 template <class T>
 void launch_project(const Geo &g, double *PC, T *Press, T *Ut, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_pc_zfaces, dim3((g.nX + 255) / 256, g.nY - 2), dim3(256), 0, s, g, PC);
-    hipLaunchKernelGGL(k_pc_span, dim3((g.nX + 255) / 256, g.nZ), dim3(256), 0, s, g, PC);
+    const long n = (long)g.nX * (g.nY - 2) + (long)g.nX * (g.nZ - 2);
+    hipLaunchKernelGGL(k_pc_zspan, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, PC);
     hipLaunchKernelGGL(k_pc_xfaces, dim3((g.nY - 2 + 255) / 256, g.nZ), dim3(256), 0, s, g, PC);
     hipLaunchKernelGGL(k_project<T>, tiles3(g), dim3(256), 0, s, g, (const double *)PC, Press, Ut);
 }
-
 template <class T>
 void launch_bcs(const Geo &g, T *Ut, const T *Utold, T *Press, const double *wall_w, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_bc_vel_z<T>, dim3((g.nX + 255) / 256, g.nY - 2), dim3(256), 0, s, g, Ut, wall_w);
-    hipLaunchKernelGGL(k_bc_vel_out<T>, dim3((g.nY - 2 + 255) / 256, g.nZ), dim3(256), 0, s, g, Ut);
-    hipLaunchKernelGGL(k_span_copy<T>, dim3((g.nX + 255) / 256, g.nZ), dim3(256), 0, s, g, Ut, 3);
-    hipLaunchKernelGGL(k_bc_press_z<T>, dim3((g.nX - 2 + 255) / 256, g.nY - 2), dim3(256), 0, s, g, (const T *)Ut, Press);
-    hipLaunchKernelGGL(k_bc_press_x<T>, dim3((g.nY - 2 + 255) / 256, g.nZ - 2), dim3(256), 0, s, g, (const T *)Ut, Utold, Press);
-    hipLaunchKernelGGL(k_span_copy<T>, dim3((g.nX + 255) / 256, g.nZ), dim3(256), 0, s, g, Press, 1);
+    const long nX = g.nX, nY = g.nY, nZ = g.nZ;
+    const long nv = nX * (nY - 2) + (nY - 2) * (nZ - 2) + (nX - 1) * (nZ - 2);
+    const long np = (nX - 2) * (nY - 2) + (nY - 2) * (nZ - 2) + nX * nZ;
+    hipLaunchKernelGGL(k_bc_vel<T>, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s, g, Ut, wall_w);
+    hipLaunchKernelGGL(k_bc_press<T>, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s, g, (const T *)Ut, Utold, Press);
 }
-
 template <class T>
 void launch_recycle(const Geo &g, T *Ut, int i_rec0, double eps, const double *lamda, const double *avg,
                     const double *Wt, const int *newk, const double *Ume, const double *uf, hipStream_t s)
@@ -2085,7 +2134,7 @@ void launch_recycle(const Geo &g, T *Ut, int i_rec0, double eps, const double *l
     template void launch_helm_zline<T>(const Geo &, const T *, T *, const T *, const void *, int, hipStream_t); \
     template void launch_helm_zebra<T>(const Geo &, const T *, const T *, const T *, T *, const T *, const void *, int, \
                                        hipStream_t);                                                                    \
-    template void launch_copy_faces3<T>(const Geo &, const T *, T *, hipStream_t);                                     \
+    template void launch_copy_faces3<T>(const Geo &, const T *, T *, void *, hipStream_t);                                     \
     template void launch_helm_lex<T>(const Geo &, const T *, T *, T *, const void *, int, hipStream_t);                \
     template void launch_ppe_rhs<T>(const Geo &, const T *, double *, hipStream_t, const void *);          \
     template unsigned launch_poisson<T>(const Geo &, const T *, T *, const int *, const double *, hipStream_t, \
