@@ -96,3 +96,22 @@ def test_adjoint_momentum_tiles(tbl, grid):
                 Jp = wall_shear_objective(base + eps * d, sv, reset, 3, i0, i1, freeze=True)
                 Jm = wall_shear_objective(base - eps * d, sv, reset, 3, i0, i1, freeze=True)
             assert abs(float((Jp - Jm) / (2 * eps)) - ad) <= 1e-5 * abs(ad)
+
+
+# below one chunk of the pinned ring, exactly one, one and a little, more chunks
+# than slots; on both sides of the sizes that take a plain copy
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("grid", [(8, 8, 8), (64, 64, 64), (67, 64, 62), (131, 130, 129)])
+def test_field_transfers(tbl, grid, precision):
+    """what goes to the device comes back, FP32 fields rounded once"""
+    rng = np.random.default_rng(3)
+    held = np.float32 if precision == "mixed" else np.float64
+    with tbl.Solver(*grid, precision=precision, kmax=2, i_rec=4, planes=(2, 3, 4, 5, 6)) as sv:
+        U, P, PC = sv.zeros(3), sv.zeros(), sv.zeros()
+        for a in (U, P, PC):
+            a[...] = rng.standard_normal(a.shape)
+        for _ in range(2):
+            sv.upload(U, P, PC)
+            got = sv.download()
+        assert np.array_equal(got[0], U.astype(held)) and np.array_equal(got[1], P.astype(held))
+        assert np.array_equal(got[2], PC)
