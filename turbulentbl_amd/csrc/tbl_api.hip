@@ -432,7 +432,7 @@ static int create_impl(tbl_ctx *c)
     // (kmax+1) groups of vec_blocks(N) each
     const size_t nbr = resid_blocks(c->g), nbv = vec_blocks(N);
     c->npart = 6 * nbr + 8 + (size_t)(p.kmax + 2) * (nbv + 8);
-    c->npart = std::max(c->npart, nbr + 8 + (size_t)poisson_blocks(c->g));   // fused first dot fits
+    c->npart = std::max(c->npart, nbr + 8 + (size_t)poisson_blocks(c->g, c->mixed));   // fused first dot fits
     c->npart = std::max(c->npart, 6 * (size_t)rhs_blocks(c->g, c->mixed));             // fused first residual pass fits
     CHK(dalloc(c, &c->part, c->npart * sizeof(double)));
     CHK(dalloc(c, &c->gm, sizeof(GmCtrl)));
@@ -1266,12 +1266,13 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
     const int mode = (c->p.tol_mode == TBL_TOL_TRUE) ? GM_MODE_TRUE : GM_MODE_REF;
     const int poll = (N > 2000000 || c->p.precond == TBL_PC_FAST) ? 1 : 4;
     // the second PCorr buffer of fused updates (TRUE) and unit steps
-    const bool two = c->p.precond == TBL_PC_FAST || (mode == GM_MODE_TRUE && poll == 1);
+    const bool unit_steps = c->p.precond == TBL_PC_FAST && sizeof(T) == sizeof(double);
+    const bool two = unit_steps || (mode == GM_MODE_TRUE && poll == 1);
     if (two && !c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
     launch_gm_init(g, c->gm, errtol, c->p.inner_tol, kmax, mmax, mode, c->PCorr, two ? c->PCalt : nullptr, c->s);
     double *part_r = c->part;                  // residual partials
     double *part_z = c->part + nbr + 8;        // norm partials (and dot partials)
-    const bool fuse_dot = poisson_blocks(g) <= c->npart - nbr - 8;
+    const bool fuse_dot = poisson_blocks(g, c->mixed) <= c->npart - nbr - 8;
     if (c->p.pc_extrap) {
         // initial guess 2 PCorr(n-1) - PCorr(n-2); the face values are zeroed below
         if (!c->PCprev) CHK(dalloc(c, &c->PCprev, (size_t)N * sizeof(double)));
@@ -1300,16 +1301,25 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         // behind that step's status read-back, gated on the cycle having ended
         // (off while the residual class is timed)
         const bool ahead_res = fuse_upd && !(c->tmask & (1u << TBL_K_RESID));
+        // the first Arnoldi step is the last of its cycle with the fast
+        // preconditioner: its vector is only measured, and formed when the
+        // status asks for a second step (1024x256x192 mixed 98 -> 77 us)
+        const bool norm_only = c->p.precond == TBL_PC_FAST && kmax > 1 && poll == 1;
         bool pend = false;
         bool queued = false;                   // the cycle's residual pass ran behind the last read-back
-        // unit steps (k_fin_unit) while they are accepted: the fast
+        // unit steps (k_fin_unit) while they are accepted, in FP64: the fast
         // preconditioner inverts A to its storage type's rounding, so a cycle
         // is z_0 = M^{-1} r, the residual of PCorr + z_0 and one read-back; the
         // operator apply, the dot product and the orthogonalisation pass of
         // the Arnoldi step are not run, nor the read-back at the solve's start.
         // The step's residual goes to the other of two vectors (v0, v1), so
-        // that a refused step leaves v_0 for the Arnoldi steps
-        bool unit = c->p.precond == TBL_PC_FAST;
+        // that a refused step leaves v_0 for the Arnoldi steps.
+        // Mixed contexts run the Arnoldi step: its coefficient differs from 1
+        // in the seventh digit there, and a PCorr that differs at all moves
+        // some value of the FP32 fields by a rounding, which grows to what
+        // FP32 leaves open (the pressure of 333x94x131 after 40 steps: 4e-6,
+        // and 1e-3 at a point where a switch of the convection tripped).
+        bool unit = unit_steps;
         bool opened = false;                   // the last unit step opened this cycle
         bool head = false;                     // its first transform ran behind the last read-back
         T *v0 = V, *v1 = r;
@@ -1407,8 +1417,8 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                     launch_fin_dots(c->gm, part_z, (int)nbv, j, c->s);
                 }
                 {
-                    Tscope ts(c, TBL_K_UPDATE, (j + 3.0) * (double)N * sizeof(T));
-                    launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s);
+                    Tscope ts(c, TBL_K_UPDATE, (j + (norm_only && j == 0 ? 2.0 : 3.0)) * (double)N * sizeof(T));
+                    launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s, !(norm_only && j == 0));
                 }
                 launch_fin_update(c->gm, part_z, (int)nbv, j, c->s);
                 HIPCHK(c, hipGetLastError());
@@ -1429,6 +1439,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                         }
                         break;
                     }
+                    if (norm_only && j == 0) launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s);
                 }
             }
             if (!queued) {                     // (queued: fin_cycle and PCorr += y z0 have run)
@@ -1467,7 +1478,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         launch_norm2<T>(V, N, part_z, nullptr, c->s);
         launch_fin_start(c->gm, part_r, (int)nbr, part_z, (int)nbv, m == 0 ? 1 : 0, c->s);
         HIPCHK(c, hipGetLastError());
-        if (m == 0 && c->p.precond == TBL_PC_FAST) {
+        if (m == 0 && unit_steps) {
             // unit step (k_fin_unit): the preconditioned residual of PCorr + V_0
             // (into W; r holds the residual) ends the solve, or is dropped
             launch_resid_upd<T>(g, c->pRhs, c->PCorr, V, c->gm, c->PCalt, r, part_r, c->s, RU_UNIT);

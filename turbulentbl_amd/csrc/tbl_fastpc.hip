@@ -761,11 +761,12 @@ void k_line_solve(Geo g, T *__restrict__ d, const double *__restrict__ ly,
         red(AL, BL, CL, DL, fA, rF, fC, fD, hu ? uA : T(0), hu ? uR : T(1), hu ? uC : T(0), hu ? uD : T(0));
     }
     // Each level squares the couplings (relative to the diagonal), and most
-    // lines have a diagonal far above 2 |ow|: once no coupling of the line
-    // reaches LS_TINY, what it could still move is 2^-40 (FP32) or 2^-80
-    // (FP64) of the line's largest value, below what the transforms round off,
-    // and the remaining levels are not run.
-    constexpr T LS_TINY = sizeof(T) == 4 ? T(0x1p-40) : T(0x1p-80);
+    // lines have a diagonal far above 2 |ow|: a level changes nothing once no
+    // coupling of the line is left, and the remaining ones are not run.  FP32
+    // couplings underflow to zero a level or two on, and the result is that of
+    // all levels bit for bit; in FP64 they count as gone at 2^-80 of the
+    // diagonal, where they could still move 2^-80 of the line's largest value.
+    constexpr T LS_TINY = sizeof(T) == 4 ? T(0) : T(0x1p-80);
     for (int h = 1; h < 64; h <<= 1) {
         const T big = LS_TINY * fabs(BF), bil = LS_TINY * fabs(BL);
         if (!__any(fabs(AF) > big || fabs(CF) > big || fabs(AL) > bil || fabs(CL) > bil)) break;

@@ -313,8 +313,9 @@ __global__ __launch_bounds__(VB) void k_fin_dots(GmCtrl *c, const double *part, 
     }
 }
 
-// z -= sum_i coef_i V_i (double arithmetic), partials of ||z||^2
-template <class T>
+// z -= sum_i coef_i V_i (double arithmetic), partials of ||z||^2; STORE false
+// leaves z as it was (the same norm: of the values rounded as stored)
+template <class T, bool STORE>
 __global__ __launch_bounds__(VB) void k_update(const T *__restrict__ V, long ldv, int j, long N,
                                               GmCtrl *__restrict__ c, double *__restrict__ part)
 {
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(VB) void k_update(const T *__restrict__ V, long ldv
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const T st = (T)s[u];
-            z[e + u * VB] = st;
+            if (STORE) z[e + u * VB] = st;
             const double sd = st;
             a += sd * sd;
         }
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(VB) void k_update(const T *__restrict__ V, long ldv
         double s = z[e];
         for (int i = 0; i <= j; i++) s -= co[i] * (double)V[(long)i * ldv + e];
         const T st = (T)s;
-        z[e] = st;
+        if (STORE) z[e] = st;
         const double sd = st;
         a += sd * sd;
     }
@@ -500,9 +501,13 @@ void launch_fin_dots(GmCtrl *c, const double *part, int nb, int j, hipStream_t s
     hipLaunchKernelGGL(k_fin_dots, dim3(1), dim3(VB), 0, s, c, part, nb, j);
 }
 template <class T>
-void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s)
+void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s, bool store)
 {
-    hipLaunchKernelGGL(k_update<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, j, N, c, part);
+    if (!store) {
+        hipLaunchKernelGGL((k_update<T, false>), dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, j, N, c, part);
+        return;
+    }
+    hipLaunchKernelGGL((k_update<T, true>), dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, j, N, c, part);
 }
 void launch_fin_update(GmCtrl *c, const double *part, int nb, int j, hipStream_t s)
 {
@@ -520,7 +525,7 @@ void launch_xupd(const T *V, long ldv, long N, const GmCtrl *c, double *PC, hipS
 #define TBL_INST(T)                                                                                 \
     template void launch_norm2<T>(const T *, long, double *, const int *, hipStream_t);             \
     template void launch_dots<T>(const T *, long, int, long, const GmCtrl *, double *, hipStream_t); \
-    template void launch_update<T>(const T *, long, int, long, GmCtrl *, double *, hipStream_t);    \
+    template void launch_update<T>(const T *, long, int, long, GmCtrl *, double *, hipStream_t, bool); \
     template void launch_xupd<T>(const T *, long, long, const GmCtrl *, double *, hipStream_t);
 TBL_INST(double)
 TBL_INST(float)

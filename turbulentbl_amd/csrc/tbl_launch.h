@@ -41,7 +41,7 @@ void gs_ctrl_read(const void *host, int *active, int *sweeps, double *res);
 // gate (optional): the Gauss-Seidel control block; the launch does nothing
 // while any of its components is active
 template <class T> void launch_ppe_rhs(const Geo &g, const T *Ut, double *pRhs, hipStream_t s, const void *gate = nullptr);
-unsigned poisson_blocks(const Geo &g);   // partials written by launch_poisson with part
+unsigned poisson_blocks(const Geo &g, bool single);   // partials written by launch_poisson with part
 // out = A x (scaled); with part: also the block partials of <out, v0> (returns the block count)
 template <class T>
 unsigned launch_poisson(const Geo &g, const T *x, T *out, const int *active, const double *scale, hipStream_t s,
@@ -110,7 +110,9 @@ void launch_gm_init(const Geo &g, GmCtrl *c, double errtol, double inner_tol, in
 void launch_publish(const void *src, int words, const Pub &pub, hipStream_t s);
 template <class T> void launch_dots(const T *V, long ldv, int j, long N, const GmCtrl *c, double *part, hipStream_t s);
 void launch_fin_dots(GmCtrl *c, const double *part, int nb, int j, hipStream_t s);
-template <class T> void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s);
+// store false: the norm of the new vector only, the vector is left as it was
+template <class T> void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s,
+                                      bool store = true);
 void launch_fin_update(GmCtrl *c, const double *part, int nb, int j, hipStream_t s);
 // gated: does nothing while the cycle is active (queued ahead of a host poll)
 void launch_fin_cycle(GmCtrl *c, hipStream_t s, int gated = 0);

@@ -1741,22 +1741,25 @@ void launch_ppe_rhs(const Geo &g, const T *Ut, double *pRhs, hipStream_t s, cons
 #endif
 // planes per thread: POISSON_KC, fewer where that leaves less than 2048 blocks
 // (256 CUs x 8 resident blocks): a plane costs a thread one load latency.
-// 64x32x48 17 -> 6 us, 256x64x96 21 -> 15 us
-static int poisson_chunk(const Geo &g)
+// 64x32x48 17 -> 6 us, 256x64x96 21 -> 15 us.  FP32 keeps POISSON_KC: the
+// order of the dot product's partials follows the chunks, and a coefficient
+// that differs in its last digit moves FP32 fields by roundings.
+static int poisson_chunk(const Geo &g, bool single)
 {
+    if (single) return POISSON_KC;
     const long tiles = (long)((g.nX - 1 + 63) / 64) * ((g.nY - 2 + 3) / 4);
     return (int)std::max(1L, std::min((long)POISSON_KC, (g.nZ - 2) * tiles / 2048));
 }
-unsigned poisson_blocks(const Geo &g)
+unsigned poisson_blocks(const Geo &g, bool single)
 {
-    const int kc = poisson_chunk(g);
+    const int kc = poisson_chunk(g, single);
     return (unsigned)(((g.nX - 1 + 63) / 64) * ((g.nY - 2 + 3) / 4) * ((g.nZ - 2 + kc - 1) / kc));
 }
 template <class T>
 unsigned launch_poisson(const Geo &g, const T *x, T *out, const int *active, const double *scale, hipStream_t s,
                         const T *v0, double *part)
 {
-    const int kchunk = poisson_chunk(g);
+    const int kchunk = poisson_chunk(g, sizeof(T) == 4);
     unsigned nbx = (g.nX - 1 + 63) / 64, nby = (g.nY - 2 + 3) / 4, nbz = (g.nZ - 2 + kchunk - 1) / kchunk;
     hipLaunchKernelGGL(k_poisson<T>, dim3(nbx * nby * nbz), dim3(256), 0, s, g, x, out, active, scale, v0, part, kchunk,
                        nbx, nby, nbz);
