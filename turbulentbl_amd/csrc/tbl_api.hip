@@ -430,7 +430,7 @@ static int create_impl(tbl_ctx *c)
     // partials: [0, 6*nbr+8) for tile reductions (Gauss-Seidel uses 6 per tile);
     // GMRES puts the residual partials at 0 and the vector partials at nbr+8,
     // (kmax+1) groups of vec_blocks(N) each
-    const size_t nbr = resid_blocks(c->g), nbv = vec_blocks(N);
+    const size_t nbr = resid_blocks(c->g), nbv = vec_blocks(N, c->mixed);
     c->npart = 6 * nbr + 8 + (size_t)(p.kmax + 2) * (nbv + 8);
     c->npart = std::max(c->npart, nbr + 8 + (size_t)poisson_blocks(c->g, c->mixed));   // fused first dot fits
     c->npart = std::max(c->npart, 6 * (size_t)rhs_blocks(c->g, c->mixed));             // fused first residual pass fits
@@ -1259,7 +1259,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
 {
     const Geo &g = c->g;
     const long N = g.N;
-    const unsigned nbv = vec_blocks(N), nbr = resid_blocks(g);
+    const unsigned nbv = vec_blocks(N, sizeof(T) == sizeof(float)), nbr = resid_blocks(g);
     T *V = F<T>(c->V), *W = F<T>(c->W), *scr = F<T>(c->scr), *r = F<T>(c->r);
     const long ldv = c->ldv;
     if (kmax > c->p.kmax) return fail(c, TBL_EARG, "kmax above the allocated restart length");

@@ -24,9 +24,15 @@ namespace tbl {
 static constexpr int VB = 256;     // threads per block of the vector kernels
 static constexpr int DG = 8;       // dot products per streaming pass
 
-unsigned vec_blocks(long N)
+// blocks of the vector kernels: 1024 values each in FP64 (four a thread), so
+// that a small grid still gives every CU its share, at most 4096 (90x80x50, up
+// to 50 Krylov vectors, 352 blocks instead of 88: k_dots 76 -> 33 us with the
+// grouped block sums, k_update 23 -> 16 us).  FP32 keeps 4096 values: the order of a norm's
+// partials follows the blocks, and mixed solves keep their bits.
+unsigned vec_blocks(long N, bool single)
 {
-    long nb = (N + 4095) / 4096;
+    const long per = single ? 4096 : 1024;
+    long nb = (N + per - 1) / per;
     if (nb > 4096) nb = 4096;
     if (nb < 1) nb = 1;
     return (unsigned)nb;
@@ -70,7 +76,7 @@ __global__ __launch_bounds__(VB) void k_fill(double *__restrict__ x, double v, l
 }
 void launch_fill(double *x, double v, long n, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fill, dim3(vec_blocks(n)), dim3(VB), 0, s, x, v, n);
+    hipLaunchKernelGGL(k_fill, dim3(vec_blocks(n, false)), dim3(VB), 0, s, x, v, n);
 }
 
 // deterministic sum of nb partials by one block of NT threads
@@ -252,7 +258,7 @@ template <class T>
 __global__ __launch_bounds__(VB) void k_dots(const T *__restrict__ V, long ldv, int j, long N,
                                             const GmCtrl *__restrict__ c, double *__restrict__ part)
 {
-    __shared__ double sh[VB / 64];
+    __shared__ double sh[2][DG][VB / 64];
     if (!c->st.active) return;
     const T *__restrict__ z = V + (long)(j + 1) * ldv;
     long b0, b1;
@@ -288,28 +294,36 @@ __global__ __launch_bounds__(VB) void k_dots(const T *__restrict__ V, long ldv, 
             for (int q = 0; q < DG; q++)
                 if (q < ng) acc[q] += (double)V[(long)(i0 + q) * ldv + e] * zv;
         }
+        // the group's block sums together, each in block_sum's order
+        const int par = (i0 / DG) & 1;
 #pragma unroll
         for (int q = 0; q < DG; q++) {
-            if (q < ng) {
-                double s = block_sum<VB>(acc[q], sh, threadIdx.x);
-                if (threadIdx.x == 0) part[(long)(i0 + q) * nb + blockIdx.x] = s;
-            }
+            const double s = wave_sum(acc[q]);
+            if ((threadIdx.x & 63) == 0) sh[par][q][threadIdx.x >> 6] = s;
+        }
+        __syncthreads();
+        if (threadIdx.x < ng) {
+            double s = 0.0;
+#pragma unroll
+            for (int w = 0; w < VB / 64; w++) s += sh[par][threadIdx.x][w];
+            part[(long)(i0 + threadIdx.x) * nb + blockIdx.x] = s;
         }
     }
 }
 
 // z = M^{-1} A v_j with v_j normalised (the Poisson apply scales by sigma_j), so
 // h(i,j) = <v_i, z> = sigma_i d_i and z - sum h(i,j) v_i = z - sum sigma_i^2 d_i V_i
+// Block i forms the i-th product (one block in turn for all: 27 -> 4.8 us an
+// Arnoldi step at up to 50 vectors).
 __global__ __launch_bounds__(VB) void k_fin_dots(GmCtrl *c, const double *part, int nb, int j)
 {
     __shared__ double sh[VB / 64];
     if (!c->st.active) return;
-    for (int i = 0; i <= j; i++) {
-        double d = fin_sum(part + (long)i * nb, nb, sh);
-        if (threadIdx.x == 0) {
-            GM_H(c, i, j) = c->sigma[i] * d;
-            c->coef[i] = c->sigma[i] * c->sigma[i] * d;
-        }
+    const int i = blockIdx.x;
+    const double d = fin_sum(part + (long)i * nb, nb, sh);
+    if (threadIdx.x == 0) {
+        GM_H(c, i, j) = c->sigma[i] * d;
+        c->coef[i] = c->sigma[i] * c->sigma[i] * d;
     }
 }
 
@@ -473,7 +487,7 @@ __global__ __launch_bounds__(VB) void k_xupd(const T *__restrict__ V, long ldv, 
 template <class T>
 void launch_norm2(const T *x, long N, double *part, const int *active, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_norm2<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, x, N, part, active);
+    hipLaunchKernelGGL(k_norm2<T>, dim3(vec_blocks(N, sizeof(T) == 4)), dim3(VB), 0, s, x, N, part, active);
 }
 void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
                       const double *part_b, const Pub &pub)
@@ -494,20 +508,20 @@ void launch_gm_init(const Geo &g, GmCtrl *c, double errtol, double inner_tol, in
 template <class T>
 void launch_dots(const T *V, long ldv, int j, long N, const GmCtrl *c, double *part, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_dots<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, j, N, c, part);
+    hipLaunchKernelGGL(k_dots<T>, dim3(vec_blocks(N, sizeof(T) == 4)), dim3(VB), 0, s, V, ldv, j, N, c, part);
 }
 void launch_fin_dots(GmCtrl *c, const double *part, int nb, int j, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fin_dots, dim3(1), dim3(VB), 0, s, c, part, nb, j);
+    hipLaunchKernelGGL(k_fin_dots, dim3(j + 1), dim3(VB), 0, s, c, part, nb, j);
 }
 template <class T>
 void launch_update(const T *V, long ldv, int j, long N, GmCtrl *c, double *part, hipStream_t s, bool store)
 {
     if (!store) {
-        hipLaunchKernelGGL((k_update<T, false>), dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, j, N, c, part);
+        hipLaunchKernelGGL((k_update<T, false>), dim3(vec_blocks(N, sizeof(T) == 4)), dim3(VB), 0, s, V, ldv, j, N, c, part);
         return;
     }
-    hipLaunchKernelGGL((k_update<T, true>), dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, j, N, c, part);
+    hipLaunchKernelGGL((k_update<T, true>), dim3(vec_blocks(N, sizeof(T) == 4)), dim3(VB), 0, s, V, ldv, j, N, c, part);
 }
 void launch_fin_update(GmCtrl *c, const double *part, int nb, int j, hipStream_t s)
 {
@@ -520,7 +534,7 @@ void launch_fin_cycle(GmCtrl *c, hipStream_t s, int gated)
 template <class T>
 void launch_xupd(const T *V, long ldv, long N, const GmCtrl *c, double *PC, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_xupd<T>, dim3(vec_blocks(N)), dim3(VB), 0, s, V, ldv, N, c, PC);
+    hipLaunchKernelGGL(k_xupd<T>, dim3(vec_blocks(N, sizeof(T) == 4)), dim3(VB), 0, s, V, ldv, N, c, PC);
 }
 #define TBL_INST(T)                                                                                 \
     template void launch_norm2<T>(const T *, long, double *, const int *, hipStream_t);             \

@@ -93,7 +93,7 @@ int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s);
 bool solve_batched(const Geo &g, bool single);
 
 // Krylov kernels (tbl_krylov.hip)
-unsigned vec_blocks(long N);
+unsigned vec_blocks(long N, bool single);
 // x[0..n) = v (a kernel, not a memset: safe inside captured graphs)
 void launch_fill(double *x, double v, long n, hipStream_t s);
 template <class T> void launch_norm2(const T *x, long N, double *part, const int *active, hipStream_t s);
