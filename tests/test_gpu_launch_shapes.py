@@ -3,6 +3,7 @@ grids on both sides of each rule and with remainders, against the oracle."""
 import numpy as np
 import pytest
 
+from oracle import orc
 from tests.case_util import gpu_from_case, make_case, ulps
 
 pytestmark = pytest.mark.gpu
@@ -115,3 +116,32 @@ def test_field_transfers(tbl, grid, precision):
             got = sv.download()
         assert np.array_equal(got[0], U.astype(held)) and np.array_equal(got[1], P.astype(held))
         assert np.array_equal(got[2], PC)
+
+
+# slab sweeps: one, two and partly filled row blocks; 1, 1, 2, 5, 6, 8 and 32 lines
+# a thread; slabs of unequal thickness, partly filled chunks.  FP32 against the
+# FP64 oracle: a chain of at most 260 points, four roundings each, 6e-8 relative
+# to the largest value
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("grid,P", [((9, 8, 13), 4), ((70, 66, 13), 2), ((12, 68, 39), 3), ((20, 130, 57), 3),
+                                    ((67, 66, 44), 1), ((9, 130, 66), 1), ((8, 130, 130), 1)])
+def test_slab_sweeps(tbl, grid, P, precision):
+    g, s = make_case(grid, seed=2, P=P)
+    _, Q = g.momentum_rhs(s.Ut, s.Press)
+    x = g.zeros()
+    x[1:-1, 1:-1, 1:-1] = np.random.default_rng(5).standard_normal((g.nX - 2, g.nY - 2, g.nZ - 2))
+    with gpu_from_case(g, s, precision=precision, helm_mode=tbl.TBL_HELM_LEX_SLAB, precond=tbl.TBL_PC_SSOR_BLOCK,
+                       slabs=P) as sv:
+        sv.set_field(tbl.F_Q, Q)
+        y = sv.apply_operator(1, x)
+        sw, _ = sv.diffusion_solve(1e-30, 2)
+        Ut = sv.get_field(tbl.F_UT)
+    Uo = s.Ut.copy(order="F")
+    swo, _ = g.diffusion_solve(Q, Uo, order=orc.GS_LEX_BLOCK, errorstop=1e-30, mmax=2)
+    yo = g.precond_apply(x, orc.PC_SSOR_BLOCK)
+    assert list(sw) == list(swo)
+    if precision == "fp64":
+        assert np.array_equal(Ut, Uo) and np.array_equal(y[I], yo[I])
+    else:
+        assert np.abs(Ut - Uo).max() <= 1e-4 * np.abs(Uo).max()
+        assert np.abs(y[I] - yo[I]).max() <= 1e-4 * np.abs(yo[I]).max()

@@ -47,7 +47,6 @@ struct tbl_ctx {
     void *Ut = nullptr, *Utold = nullptr, *Q = nullptr, *Press = nullptr;
     void *Ualt = nullptr;                // second velocity buffer of the zebra sweep (Ut and Ualt swap)
     int *slab = nullptr;                 // per-slab orderings: 0-based first/last interior plane per slab
-    void *halo = nullptr;                // per-slab Gauss-Seidel: ghost-plane snapshots (3 x 2 slabs planes)
     double *PCorr = nullptr, *pRhs = nullptr;
     double *PCprev = nullptr;            // PCorr of the step before (extrapolated initial guess)
     double *PCalt = nullptr;             // second PCorr buffer: the fused update + residual writes it
@@ -311,11 +310,11 @@ static int create_impl(tbl_ctx *c)
     c->ldv = (N + 63) & ~63L;
     CHK(dalloc(c, &c->V, (size_t)(p.kmax + 1) * c->ldv * c->es));
     CHK(dalloc(c, &c->W, N * c->es));
-    CHK(dalloc(c, &c->scr, N * c->es));
     CHK(dalloc(c, &c->r, N * c->es));
     if (p.tol_mode == TBL_TOL_TRUE) CHK(dalloc(c, &c->Z, (size_t)p.kmax * c->ldv * c->es));
     if (p.helm_mode == TBL_HELM_ZEBRA) CHK(dalloc(c, &c->Ualt, 3 * N * c->es));
     c->g.nslab = 0; c->g.nkmax = 0; c->g.slab = nullptr;
+    size_t nscr = N;
     if (p.helm_mode == TBL_HELM_LEX_SLAB || p.precond == TBL_PC_SSOR_BLOCK) {
         // the reference's slab bounds (dnssetbl.f90:76-92): nZ/P planes per
         // rank, the remainder to the high ranks; the first and last rank
@@ -346,8 +345,9 @@ static int create_impl(tbl_ctx *c)
         CHK(dalloc(c, &c->slab, sizeof(int) * 2 * P));
         HIPCHK(c, hipMemcpyAsync(c->slab, sl.data(), sizeof(int) * 2 * P, hipMemcpyHostToDevice, c->s));
         c->g.slab = c->slab;
-        if (p.helm_mode == TBL_HELM_LEX_SLAB) CHK(dalloc(c, &c->halo, 3 * 2 * (size_t)P * c->g.sZ * c->es));
+        nscr = std::max((size_t)N, slab_scratch(c->g, p.helm_mode == TBL_HELM_LEX_SLAB));
     }
+    CHK(dalloc(c, &c->scr, nscr * c->es));
     if (p.helm_mode == TBL_HELM_ZLINE_RB || p.helm_mode == TBL_HELM_ZEBRA) {
         // elimination factors of the partitioned wall-normal line solve (the
         // line matrix a = -h Ab, b = 1 - h Ap, c = -h At is the same for every
@@ -537,7 +537,7 @@ extern "C" int tbl_destroy(tbl_ctx *c)
     void *dev[] = {c->mesh, c->Ut, c->Ualt, c->Utold, c->Q, c->Press, c->PCorr, c->pRhs, c->V, c->W, c->scr, c->r, c->Z,
                    c->part, c->gm, c->gs, c->sums, c->avg, c->Wt, c->Ume, c->uf, c->bltkns, c->dstar,
                    c->theta, c->tau, c->tausum, c->taumean, c->cf, c->wall_w, c->scan, c->newk, c->rec, c->dd, c->zf, c->br, c->PCprev,
-                   c->PCalt, c->slab, c->halo, c->r3};
+                   c->PCalt, c->slab, c->r3};
     for (void *d : dev)
         if (d) hipFree(d);
     if (c->fast) fastpc_destroy(c->fast);
@@ -1187,7 +1187,7 @@ template <class T> static int helm_impl(tbl_ctx *c, double errorstop, int mmax, 
             // neighbours come from registers, LDS and cache): 3 N values per
             // active component
             Tscope ts(c, TBL_K_HELM, 3.0 * (act[0] + act[1] + act[2]) * (double)c->g.N * sizeof(T));
-            launch_helm_lex<T>(c->g, F<T>(c->Q), F<T>(c->Ut), F<T>(c->halo), c->gs, c->g.nkmax, c->s);
+            launch_helm_lex<T>(c->g, F<T>(c->Q), F<T>(c->Ut), F<T>(c->scr), c->gs, c->s);
             HIPCHK(c, hipGetLastError());
             continue;
         }

@@ -30,11 +30,11 @@ template <class T> void launch_helm_zebra(const Geo &g, const T *Q, const T *cur
 // boundary / ghost values of the three velocity components, src -> dst
 // (and the Gauss-Seidel control block of a new solve, as launch_gs_init)
 template <class T> void launch_copy_faces3(const Geo &g, const T *src, T *dst, void *ctrl, hipStream_t s);
-// per-slab lexicographic Gauss-Seidel sweep (snapshot of the slabs' ghost
-// planes into halo, then the sweep); threads a slab kernel needs, 0 if the
-// slabs are too thick for one workgroup
-template <class T> void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *halo, const void *ctrl, int nkmax,
-                                        hipStream_t s);
+// per-slab lexicographic Gauss-Seidel sweep; threads a slab kernel needs, 0 if
+// the slabs are too thick for one workgroup; values of scr that the sweep
+// (lex) or the block SSOR needs
+template <class T> void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *scr, const void *ctrl, hipStream_t s);
+size_t slab_scratch(const Geo &g, bool lex);
 int slab_threads(const Geo &g, int nkmax);
 size_t gs_ctrl_bytes();
 void gs_ctrl_read(const void *host, int *active, int *sweeps, double *res);

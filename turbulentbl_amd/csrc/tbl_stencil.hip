@@ -1800,283 +1800,500 @@ void launch_resid_upd(const Geo &g, const double *pRhs, const double *PC, const 
 // (i-1,j,k), (i,j-1,k) and (i,j,k-1) and the old values of the other
 // neighbours; with the periodic span wrap, row j = 1 reads the old value of
 // row nY-2 and row nY-2 the new value of row 1.  Both sweeps run as a
-// wavefront over the lines: in step t line (j, k) updates its block
-// t - j - k.  Every new neighbour of a point then lies in the same block
-// before it or in a block updated in an earlier step, and every old
-// neighbour in a block of a later step (the wrap's new row 1 ny - 1 steps
-// earlier), so the values read are exactly the lexicographic loop's and the
-// results are the reference's, bit for bit.
+// wavefront over the lines: in step t line (j, k) updates its point
+// t - j - k.  Every new neighbour of a point is then the value its line formed
+// one step earlier (the wrap's new row 1: ny - 1 steps earlier), and every old
+// neighbour is updated in a later step, so the values read are exactly the
+// lexicographic loop's and the results are the reference's, bit for bit.
 // One workgroup per slab (and velocity component).  Thread (jj, kc) owns span
 // row jj and chunk kc of KL consecutive wall-normal lines of the slab (rows
-// padded to whole wavefronts); one barrier per step.
-//  * Gauss-Seidel: blocks of SL_B points (SL_B/2 in FP64), neighbour values
-//    from memory (a value another thread wrote in an earlier step is visible
-//    after that step's barrier); ceil((nX-2)/SL_B) + (nY-3) + planes steps
-//    per sweep.
-//  * block SSOR: one point per block, the i-1 and k-1 neighbours in
-//    registers (LDS across chunks), the j-1 neighbour from the previous lane
-//    by wave shuffle (LDS across wavefronts); (nX-2) + (nY-3) + planes steps
-//    per sweep.
+// padded to whole wavefronts); (nX-2) + (nY-3) + planes steps per sweep, one
+// barrier each.  The i-1 and k-1 neighbours are in registers (LDS across
+// chunks), the j-1 neighbour comes from the previous lane (LDS across
+// wavefronts).
+//
+// The points of a step lie on a diagonal of the slab: read in place, a
+// wavefront's load touches 64 cache lines, and the L1's one line a clock
+// bounds the step.  The sweeps therefore work on a skewed copy S in the order
+// of the steps: row i + jj + kk + 1 of S holds column i of line (jj, kk), line
+// kk and row jj at (kk + 1) nyp + jj, with the ghost planes of the slab at
+// kk = -1 and nk (the copy is also the snapshot of the neighbouring slabs'
+// values).  A step reads and writes whole rows of S, at addresses that are one
+// uniform base a step and an offset kept per line.  The copies in and out are
+// launches of their own over the whole chip, transposed through LDS.
+// What bounds a step is its chain of LDS reads, arithmetic, LDS writes and
+// barrier (0.33 us).  90x80x50 in 5 slabs, FP64, copies included: SSOR
+// 371 -> 135 us an application, Gauss-Seidel 580 -> 190 us a sweep; 1024x256x192 in
+// 8: a sweep 34.9 -> 8.8 ms; 64x130x130 in one: 10.9 -> 4.8 ms.
+// Values that a line forms before its first and after its last column, and
+// lines beyond the slab's last plane, go to places of S that nothing reads (the
+// outflow face and the upper ghost plane are read a step before).
 // ----------------------------------------------------------------------------
-#define SL_MAXT 1024
-#define SL_MAXW (SL_MAXT / 64)
-#define SL_B 8
-// threads of a slab workgroup with KL lines per thread: up to 1024 for
-// KL <= 8, 512 above
-#define SL_BOUND(KL) ((KL) <= 8 ? SL_MAXT : SL_MAXT / 2)
 // launch shape of a slab kernel: KL lines per thread, nkc chunks, rows
-// padded to nyp; 0 if the slabs need more threads than one workgroup has
+// padded to nyp; 0 if the slabs need more threads than one workgroup has.
+// A step is a chain of LDS reads, arithmetic, LDS writes and a barrier, which
+// more wavefronts on a SIMD overlap: one or two lines and up to 1024 threads
+// where that holds the slab (10 planes of 128 padded rows, a whole step of the
+// solver: 13.6 ms with 2 lines a thread, 14.9 with 3, 15.4 with 5).  Beyond, 512
+// threads and 5 or 6 lines, for the registers that hold operands loaded ahead
+// (10 planes of 256 rows: 1.45 ms a sweep with 5 lines, 1.57 with 3 and 1024
+// threads), then 8 lines, and 32 for the thickest slabs.
 static int slab_shape(const Geo &g, int nkmax, int &KL, int &nkc, int &nyp)
 {
+    static const int lines[] = {1, 2, 5, 6, 8, 32}, most[] = {1024, 1024, 512, 512, 1024, 512};
     nyp = (g.nY - 2 + 63) / 64 * 64;
-    for (KL = 4; KL <= 32; KL *= 2) {
+    for (int q = 0; q < 6; q++) {
+        KL = lines[q];
         nkc = (nkmax + KL - 1) / KL;
-        if (nyp * nkc <= SL_BOUND(KL)) return nyp * nkc;
+        if (nyp * nkc <= most[q]) return nyp * nkc;
     }
     return 0;
 }
-
-// snapshot of the ghost planes of every slab before a sweep; layout
-// [component][slab][below, above] x (nX nY)
-template <class T>
-__global__ void k_slab_halo(Geo g, const T *__restrict__ Ut, T *__restrict__ halo, const GsCtrl *__restrict__ ctrl)
+int slab_threads(const Geo &g, int nkmax)
 {
-    const int p = blockIdx.z, hs = blockIdx.y, r = hs >> 1;
-    if (!ctrl->active[p]) return;
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= g.sZ) return;
-    const int k = (hs & 1) ? g.slab[2 * r + 1] + 1 : g.slab[2 * r] - 1;
-    halo[((long)p * 2 * g.nslab + hs) * g.sZ + e] = Ut[(long)p * g.N + (long)k * g.sZ + e];
+    int KL, nkc, nyp;
+    return slab_shape(g, nkmax, KL, nkc, nyp);
 }
 
-template <class T, int KL>
-__global__ __launch_bounds__(SL_BOUND(KL)) void k_helm_lex(Geo g, const T *__restrict__ Qall, T *Uall,
-                                                           const T *__restrict__ halo, const GsCtrl *__restrict__ ctrl,
-                                                           int nkc, int nyp)
+// the skewed copy: span rows padded, row length, rows; values of a slab and of
+// a field
+struct Skew {
+    int nyp, len, rows;
+    long ss, fs;
+};
+static Skew skew_of(const Geo &g)
+{
+    int KL, nkc;
+    Skew sk;
+    slab_shape(g, g.nkmax, KL, nkc, sk.nyp);
+    sk.len = sk.nyp * (nkc * KL + 2);
+    sk.rows = (g.nX - 1) + (g.nY - 3) + g.nkmax + 2;
+    sk.ss = (long)sk.rows * sk.len;
+    sk.fs = sk.ss * g.nslab;
+    return sk;
+}
+size_t slab_scratch(const Geo &g, bool lex) { return (size_t)skew_of(g).fs * (lex ? 6 : 1); }
+
+// Copies into (IN) and out of S.  Block (64 rows of S, 64 span rows and plane
+// of the slab, slab and field); field f < 3 is u + f N, with the slab's ghost
+// planes, f >= 3 is q + (f - 3) N, without.  Out: interior columns only.
+template <class T, bool IN>
+__global__ __launch_bounds__(256) void k_skew(Geo g, Skew sk, const T *__restrict__ u, const T *__restrict__ q,
+                                              T *__restrict__ S, T *__restrict__ dst, const int *__restrict__ act, int ghosts)
+{
+    const int r = blockIdx.z % g.nslab, f = blockIdx.z / g.nslab;
+    if (act && !act[f % 3]) return;
+    const int W = sk.nyp / 64, wb = blockIdx.y % W, gh = f < 3 ? ghosts : 0;
+    const int kk = (int)(blockIdx.y / W) - gh, k = g.slab[2 * r] + kk;
+    if (k > g.slab[2 * r + 1] + gh) return;
+    __shared__ T sh[64][65];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // row m of the tile: column c0 + m - jr of span row jr
+    const int c0 = 64 * blockIdx.x, rows = min(g.nY - 2 - 64 * wb, 64), ncol = g.nX + 63;
+    T *Sb = S + f * sk.fs + r * sk.ss + (long)(c0 + 64 * wb + kk + 1) * sk.len + (kk + 1) * sk.nyp + 64 * wb;
+    const long f0 = (long)k * g.sZ + (long)(64 * wb + 1) * g.nX;
+    if constexpr (IN) {
+        const T *src = (f < 3 ? u + (long)f * g.N : q + (long)(f - 3) * g.N) + f0;
+        for (int jr = w; jr < rows; jr += 4) {
+            const int i = c0 + lane - jr;
+            if (i >= 0 && i < g.nX) sh[jr][lane] = src[(long)jr * g.nX + i];
+        }
+        __syncthreads();
+        for (int m = w; m < 64; m += 4) {
+            const int i = c0 + m - lane;
+            if (i >= 0 && i < g.nX && lane < rows) Sb[(long)m * sk.len + lane] = sh[lane][m];
+        }
+    } else {
+        for (int m = w; m < 64; m += 4) {
+            const int i = c0 + m - lane;
+            if (i >= 0 && i < g.nX && lane < rows) sh[lane][m] = Sb[(long)m * sk.len + lane];
+        }
+        __syncthreads();
+        T *out = dst + (long)f * g.N + f0;
+        for (int jr = w; jr < rows; jr += 4) {
+            const int i = c0 + lane - jr;
+            if (i >= 1 && i < g.nX - 1) out[(long)jr * g.nX + i] = sh[jr][lane];
+        }
+    }
+}
+template <class T, bool IN>
+static void launch_skew(const Geo &g, const Skew &sk, const T *u, const T *q, T *S, T *dst, const int *act, int ghosts,
+                        int nf, hipStream_t s)
+{
+    const dim3 grid((g.nX + 63 + 63) / 64, sk.nyp / 64 * (g.nkmax + 2 * ghosts), nf * g.nslab);
+    hipLaunchKernelGGL((k_skew<T, IN>), grid, dim3(256), 0, s, g, sk, u, q, S, dst, act, ghosts);
+}
+
+// value of the previous (next) lane; edge: lane 0's (lane 63's)
+__device__ __forceinline__ float lane_up(float x, float edge)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge), __builtin_bit_cast(int, x),
+                                                                 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_dn(float x, float edge)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge), __builtin_bit_cast(int, x),
+                                                                 0x130, 0xf, 0xf, false));
+}
+struct F2 { float a, b; };
+__device__ __forceinline__ double lane_up(double x, double edge)
+{
+    const F2 v = __builtin_bit_cast(F2, x), e = __builtin_bit_cast(F2, edge);
+    return __builtin_bit_cast(double, F2{lane_up(v.a, e.a), lane_up(v.b, e.b)});
+}
+__device__ __forceinline__ double lane_dn(double x, double edge)
+{
+    const F2 v = __builtin_bit_cast(F2, x), e = __builtin_bit_cast(F2, edge);
+    return __builtin_bit_cast(double, F2{lane_dn(v.a, e.a), lane_dn(v.b, e.b)});
+}
+
+// a plane's coefficient, in a scalar register: S might alias it for all the
+// compiler knows, and read again in the step loop it would wait for all the
+// loads in flight
+__device__ __forceinline__ float plane_coef(float x)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ double plane_coef(double x)
+{
+    const F2 v = __builtin_bit_cast(F2, x);
+    return __builtin_bit_cast(double, F2{plane_coef(v.a), plane_coef(v.b)});
+}
+
+// a value of S: uniform address, byte offset of the thread
+template <class T> __device__ __forceinline__ T &sk_at(T *base, unsigned off) { return *(T *)((char *)base + off); }
+template <class T> __device__ __forceinline__ T sk_at(const T *base, unsigned off)
+{
+    return *(const T *)((const char *)base + off);
+}
+
+// (no code: keeps the compiler from folding the offset into a 64-bit address per
+// line and from turning a select of a loaded value into a branch)
+template <class T> __device__ __forceinline__ void as_is(T &x) { asm("" : "+v"(x)); }
+
+// Gauss-Seidel sweep of one component over S: fields p (u, in place) and
+// 3 + p (the right-hand side).  A step's operands are loaded SD steps ahead:
+// per line q and the old value of column i+1, which is also what the lane
+// before and the line below read in this step as their j+1 and k+1
+// neighbours; across row blocks and chunks, and at the span wrap's old row
+// nY-2 and the lower ghost plane, one load each.  Nothing loaded ahead is
+// written before its step.  The wrap's new row 1 waits ny - 1 steps in LDS (sR).
+// 32 lines go in groups of 8, the next group's operands loaded ahead.
+// MT: most threads of the workgroup (registers per thread).
+template <class T, int KL, int MT, int SD>
+__global__ __launch_bounds__(MT) void k_helm_lex(Geo g, Skew sk, T *S, const GsCtrl *__restrict__ ctrl, int nkc)
 {
     const int r = blockIdx.x, p = blockIdx.y;
     if (!ctrl->active[p]) return;
-    const int tid = threadIdx.x;
-    const int jj = tid % nyp, kc = tid / nyp;
-    const int nX = g.nX, nY = g.nY, nx = nX - 2, ny = nY - 2;
+    __shared__ T sW[2][MT / 64][KL];
+    __shared__ T sK[2][MT];
+    extern __shared__ double lex_ring[];
+    T *sR = (T *)lex_ring;
+    const int tid = threadIdx.x, lane = tid & 63, nyp = sk.nyp, W = nyp / 64;
+    // the chunk and its planes' coefficients are uniform over a wavefront
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), kc = w / W, wv = w - kc * W;
+    const int nx = g.nX - 2, ny = g.nY - 2;
     const int kb = g.slab[2 * r], nk = g.slab[2 * r + 1] - kb + 1;
-    const long sZ = g.sZ;
-    const bool live = jj < ny;
-    T *u = Uall + (long)p * g.N;
-    const T *q = Qall + (long)p * g.N;
-    const T *hb = halo + (long)(p * 2 * g.nslab + 2 * r) * sZ, *ht = hb + sZ;
-    const int j = jj + 1;
-    // span neighbours: row j+1 (old; for the last row the wrap's row 1, new)
-    // and row j-1 (new, from the previous step; for the first row the
-    // wrap's row nY-2, old)
-    const long dn = (long)(jp1_of(live ? j : 1, nY) - j) * nX, ds = (long)(jm1_of(live ? j : 1, nY) - j) * nX;
-    const T dt = T(g.dt), Re = T(g.Re), Ae = T(g.Ae), Aw = T(g.Aw), An = T(g.An), As = T(g.As);
-    constexpr int LB = sizeof(T) == 8 ? SL_B / 2 : SL_B;     // points per block (FP64: registers)
-    const int nbk = (nx + LB - 1) / LB;
-    const int steps = nbk + ny + nk - 2;
-    for (int t = 0; t < steps; t++) {
-#pragma unroll 1
-        for (int l = 0; l < KL; l++) {
-            const int kk = kc * KL + l, bi = t - jj - kk;
-            if (live && kk < nk && bi >= 0 && bi < nbk) {
-                const int k = kb + kk, i0 = bi * LB;
-                const long c0 = (long)(i0 + 1) + (long)nX * ((long)j + (long)nY * k), pl0 = c0 - (long)k * sZ;
-                const T Abk = T(g.Ab[k]), Atk = T(g.At[k]), Apk = T(g.Ap[k]);
-                // i-1 of the block's first point: the face (first block) or the
-                // line's previous block, written by this thread one step earlier
-                T uw = u[c0 - 1];
-                // every operand of the block is read before its first store:
-                // none is written inside the block except i+1, which must be
-                // read old anyway (points past the line end read in-field
-                // values that are not used)
-                T qv[LB], ue[LB], un[LB], us[LB], ub[LB], ut[LB];
+    const int steps = nx + ny + nk - 2, l0 = kc * KL, jj = wv * 64 + lane;
+    const T h = T(g.dt) / T(g.Re), Ae = T(g.Ae), Aw = T(g.Aw), An = T(g.An), As = T(g.As);
+    const bool first = wv == 0, last = wv == W - 1, hi = lane >= 32;
+    const int Lw = last ? (ny - 1) & 63 : 64;                       // lane of row nY-2
+    // step t updates row t + 2 of S
+    T *U = S + p * sk.fs + r * sk.ss + 2L * sk.len;
+    const T *Q = U + 3 * sk.fs;
+    constexpr int G = KL > 8 ? 8 : KL, NG = KL / G, NS = NG == 1 ? SD + 1 : 2;
+    static_assert(NG == 1 || (SD == 1 && NG % 2 == 0), "a group's slot is its parity");
+    unsigned off[G];                                                // of the first lines, in a row (bytes)
 #pragma unroll
-                for (int b = 0; b < LB; b++) {
-                    const long c = c0 + b, pl = pl0 + b;
-                    qv[b] = q[c];
-                    ue[b] = u[c + 1];
-                    un[b] = u[c + dn];
-                    us[b] = u[c + ds];
-                    ub[b] = kk == 0 ? hb[pl] : u[c - sZ];
-                    ut[b] = kk == nk - 1 ? ht[pl] : u[c + sZ];
-                }
-#pragma unroll
-                for (int b = 0; b < LB; b++) {
-                    if (i0 + b < nx) {
-                        const T rt1 = Ae * ue[b] + Aw * uw + An * un[b] + As * us[b];
-                        const T rt2 = Atk * ut[b] + Abk * ub[b];
-                        const T v = (qv[b] + dt / Re * (rt1 + rt2)) / (T(1.0) - dt / Re * Apk);
-                        u[c0 + b] = v;
-                        uw = v;
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// block SSOR, one workgroup per slab: forward sweep (the stored values are
-// already scaled by ((2 - w)/w) Ap), then the backward sweep in the mirrored
-// order; the forward values a neighbour reads are the unscaled ones
-template <class T, int KL>
-__global__ __launch_bounds__(SL_BOUND(KL)) void k_ssor_block(Geo g, const T *__restrict__ rin, T *out,
-                                                        const int *__restrict__ active, int nkc, int nyp)
-{
-    if (active && !*active) return;
-    const int r = blockIdx.x;
-    __shared__ T sW[2][SL_MAXW][KL];
-    __shared__ T sK[2][SL_MAXT];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int jj = tid % nyp, kc = tid / nyp;
-    const int nX = g.nX, nY = g.nY, nx = nX - 2, ny = nY - 2;
-    const int kb = g.slab[2 * r], nk = g.slab[2 * r + 1] - kb + 1;
-    const bool live = jj < ny;
-    const int j = jj + 1, jc = live ? j : 1;
-    const T om = T(g.omega);
-    const int steps = nx + ny + nk - 2;
-    // per line: its plane's coefficients, and the address of its first point
-    // (the point of a step follows from the step index)
-    T Abk[KL], Atk[KL], Apk[KL], rApk[KL];
-    long c0l[KL];
+    for (int l = 0; l < G; l++) off[l] = ((l0 + l + 1) * nyp + jj) * sizeof(T);
+    // old values across the row block's edges: lane 63's j+1, and in the first
+    // block lane 0's j-1 (row nY-2; a row of S that exists where it is not read)
+    const unsigned ehi = last ? off[0] : (sk.len + (l0 + 1) * nyp + 64 * (wv + 1)) * sizeof(T);
+    const unsigned elo = ((l0 + 1) * nyp + ny - 1) * sizeof(T), line = nyp * sizeof(T), row = sk.len * sizeof(T);
+    T qv[NS][G], ev[NS][G], xv[NS][G], tv[NS], bv[NS];
+    T xprev[KL], Atk[KL], Abk[KL], den[KL];
 #pragma unroll
     for (int l = 0; l < KL; l++) {
-        const int k = kb + min(kc * KL + l, nk - 1);
-        Abk[l] = T(g.Ab[k]); Atk[l] = T(g.At[k]); Apk[l] = T(g.Ap[k]); rApk[l] = T(g.rAp[k]);
-        c0l[l] = 1 + (long)nX * ((long)jc + (long)nY * k);
+        const int k = kb + min(l0 + l, nk - 1);
+        Atk[l] = plane_coef(T(g.At[k]));
+        Abk[l] = plane_coef(T(g.Ab[k]));
+        den[l] = plane_coef(T(1.0) - h * T(g.Ap[k]));
     }
-    // A line's operand of step t (rin forward, the forward result backward)
-    // is loaded SD steps ahead into an SD + 1 slot register ring; the step
-    // loop is unrolled by the slot count, so a slot keeps its registers.
-    // Loads are unconditional at clamped points (the values of steps a line
-    // does not update are never used).  Backward, a line's future points are
-    // written only by the line itself, so the values loaded ahead are the
-    // forward results.
-    constexpr int SD = 2, NS = SD + 1;
-    T rv[NS][KL];
-    T xprev[KL];
-    auto ld_f = [&](int sl, int t) {
+    auto ld = [&](int sl, int t, int gr) {
+        t = min(t, steps - 1);
+        const T *u = U + (long)t * sk.len + gr * G * nyp, *u1 = u + sk.len, *q = Q + (long)t * sk.len + gr * G * nyp;
+        const unsigned ex = hi ? ehi : elo + (unsigned)(min(t + ny + 1, sk.rows - 1) - (t + 2)) * row;
 #pragma unroll
-        for (int l = 0; l < KL; l++) {
-            const int ii = min(max(t - jj - (kc * KL + l), 0), nx - 1);
-            rv[sl][l] = rin[c0l[l] + ii];
+        for (int l = 0; l < G; l++) {
+            as_is(off[l]);
+            qv[sl][l] = sk_at(q, off[l]);
+            ev[sl][l] = sk_at(u1, off[l]);
+            xv[sl][l] = sk_at(u, ex + l * line);
         }
+        if (gr == NG - 1) tv[sl] = sk_at(u1, off[G - 1] + line);
+        if (gr == 0) bv[sl] = sk_at(u - sk.len, off[0] - line);
     };
+    // the inflow face: column 0, row jj + kk + 1
 #pragma unroll
-    for (int l = 0; l < KL; l++) xprev[l] = T(0);
+    for (int l = 0; l < KL; l++)
+        xprev[l] = jj < ny && l0 + l < nk ? sk_at((const T *)U + (long)(jj + l0 + l - 1) * sk.len, off[0] + l * line) : T(0);
 #pragma unroll
-    for (int q = 0; q < SD; q++) ld_f(q, q);
-    auto fwd = [&](auto S, int t) {
-        constexpr int sl = decltype(S)::value;
-        ld_f((sl + SD) % NS, t + SD);
-        const int b = t & 1;
-        const T kin = kc > 0 ? sK[b ^ 1][tid - nyp] : T(0);
+    for (int m = 0; m < SD; m++) {
+        ld(m, m, NG - 1);
+        __builtin_amdgcn_sched_barrier(0);       // in the order that the steps wait for
+    }
+    int mw = 0, mr = 1;                          // ring slots of this step and of ny - 1 steps ago
+    auto step = [&](auto C, int t) {
+        const int b = t & 1, c0 = t - l0 - jj;   // column of line l less one: c0 - l
+        T kl = sK[b ^ 1][tid >= nyp ? tid - nyp : tid], above = T(0);
+        // highest line first: line l reads line l-1's value of step t-1
 #pragma unroll
-        for (int l = KL - 1; l >= 0; l--) {
-            T sj = __shfl_up(xprev[l], 1, 64);
-            if (lane == 0 && jj > 0) sj = sW[b ^ 1][w - 1][l];
-            const int kk = kc * KL + l, ii = t - jj - kk;
-            if (live && kk < nk && ii >= 0 && ii < nx) {
-                const long c = c0l[l] + ii;
-                const T rw = ii == 0 ? T(0) : xprev[l];
-                const T rs = jj == 0 ? T(0) : sj;
-                const T rb = kk == 0 ? T(0) : (l == 0 ? kin : xprev[l - 1]);
-                const T v = -om * (rv[sl][l] + T(g.Aw) * rw + T(g.As) * rs + Abk[l] * rb) * rApk[l];
-                out[c] = (T(2) - om) / om * Apk[l] * v;
-                xprev[l] = v;
+        for (int gi = 0; gi < NG; gi++) {
+            const int gr = NG - 1 - gi, sl = NG == 1 ? decltype(C)::value : gi & 1, lb = gr * G;
+            if (NG == 1) ld((sl + SD) % NS, t + SD, 0);
+            else if (gi + 1 < NG) ld(sl ^ 1, t, gr - 1);
+            else ld(sl ^ 1, t + 1, NG - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            T *u = U + (long)t * sk.len + lb * nyp;
+            T sw[G], wrap[G];
+#pragma unroll
+            for (int l = 0; l < G; l++) {
+                sw[l] = sW[b ^ 1][first ? 0 : w - 1][lb + l];
+                wrap[l] = sR[(l0 + lb + l) * ny + mr];
             }
+            if (gr == NG - 1) above = tv[sl];
+            if (gr == 0) as_is(kl);
+            const T kin = tid >= nyp ? kl : bv[sl];
+            // the lines side by side, so that their dependent chains overlap
+            T us[G], un[G], a[G], v[G];
+#pragma unroll
+            for (int l = 0; l < G; l++) {
+                as_is(sw[l]);
+                as_is(wrap[l]);
+                us[l] = lane_up(xprev[lb + l], jj == 0 ? xv[sl][l] : sw[l]);
+                un[l] = lane_dn(ev[sl][l], xv[sl][l]);
+                un[l] = lane == Lw ? wrap[l] : un[l];
+            }
+#pragma unroll
+            for (int l = 0; l < G; l++) a[l] = Ae * ev[sl][l] + Aw * xprev[lb + l];
+#pragma unroll
+            for (int l = 0; l < G; l++) a[l] = a[l] + An * un[l];
+#pragma unroll
+            for (int l = 0; l < G; l++) a[l] = a[l] + As * us[l];
+#pragma unroll
+            for (int l = 0; l < G; l++) {
+                const T ub = lb + l == 0 ? kin : xprev[max(lb + l - 1, 0)];
+                const T ut = l == G - 1 ? above : ev[sl][l + 1 < G ? l + 1 : l];
+                v[l] = qv[sl][l] + h * (a[l] + (Atk[lb + l] * ut + Abk[lb + l] * ub));
+            }
+#pragma unroll
+            for (int l = 0; l < G; l++) v[l] = v[l] / den[lb + l];
+#pragma unroll
+            for (int l = 0; l < G; l++) {
+                sk_at(u, off[l]) = v[l];
+                xprev[lb + l] = c0 >= lb + l ? v[l] : xprev[lb + l];
+            }
+            above = ev[sl][0];
         }
         if (lane == 63) {
 #pragma unroll
             for (int l = 0; l < KL; l++) sW[b][w][l] = xprev[l];
         }
+        if (jj == 0) {
+#pragma unroll
+            for (int l = 0; l < KL; l++) sR[(l0 + l) * ny + mw] = xprev[l];
+        }
         sK[b][tid] = xprev[KL - 1];
-        __syncthreads();
+        mw = mr;
+        mr = mr + 1 == ny ? 0 : mr + 1;
+        lds_barrier();
+    };
+    constexpr int RS = NG == 1 ? NS : 1;
+    int t = 0;
+    for (; t + RS <= steps; t += RS) ring_steps<0, RS>(step, t);
+    ring_tail<0, RS>(step, t, steps);
+}
+
+// block SSOR over S (in place): forward sweep (the stored values are already
+// scaled by ((2 - w)/w) Ap), then the backward sweep in the mirrored order;
+// the forward values a neighbour reads are the unscaled ones.  A line's
+// operand of step t is loaded SD steps ahead.
+template <class T, int KL, int MT, int SD>
+__global__ __launch_bounds__(MT) void k_ssor_block(Geo g, Skew sk, T *S, const int *__restrict__ active, int nkc)
+{
+    if (active && !*active) return;
+    const int r = blockIdx.x;
+    __shared__ T sW[2][MT / 64 + 1][KL];                            // the last: zero
+    __shared__ T sK[2][MT];
+    const int tid = threadIdx.x, lane = tid & 63, nyp = sk.nyp, W = nyp / 64;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), kc = w / W, wv = w - kc * W;
+    const int nx = g.nX - 2, ny = g.nY - 2;
+    const int kb = g.slab[2 * r], nk = g.slab[2 * r + 1] - kb + 1;
+    const int steps = nx + ny + nk - 2, l0 = kc * KL, jj = wv * 64 + lane;
+    const T om = T(g.omega), back = (T(2) - om) / om;
+    const T Aw = T(g.Aw), As = T(g.As), Ae = T(g.Ae), An = T(g.An);
+    const bool first = wv == 0, last = wv == W - 1;
+    // step t updates row t + 2 of S, backward row steps + 1 - t
+    T *U = S + r * sk.ss + 2L * sk.len;
+    if (tid < 2 * KL) sW[tid / KL][MT / 64][tid % KL] = T(0);
+    __syncthreads();
+    unsigned off[KL];                                               // of the lines, in a row (bytes)
+#pragma unroll
+    for (int l = 0; l < KL; l++) off[l] = ((l0 + l + 1) * nyp + jj) * sizeof(T);
+    constexpr int NS = SD + 1;
+    T rv[NS][KL];
+    T xprev[KL], rAp[KL], Abk[KL], Atk[KL], bAp[KL];
+#pragma unroll
+    for (int l = 0; l < KL; l++) {
+        const int k = kb + min(l0 + l, nk - 1);
+        rAp[l] = plane_coef(T(g.rAp[k]));
+        Abk[l] = plane_coef(T(g.Ab[k]));
+        Atk[l] = plane_coef(T(g.At[k]));
+        bAp[l] = plane_coef(back * T(g.Ap[k]));
+    }
+    auto ld = [&](int sl, int row) {
+        const T *u = U + (long)row * sk.len;
+#pragma unroll
+        for (int l = 0; l < KL; l++) {
+            as_is(off[l]);
+            rv[sl][l] = sk_at(u, off[l]);
+        }
+    };
+#pragma unroll
+    for (int l = 0; l < KL; l++) xprev[l] = T(0);
+#pragma unroll
+    for (int m = 0; m < SD; m++) {
+        ld(m, min(m, steps - 1));
+        __builtin_amdgcn_sched_barrier(0);       // in the order that the steps wait for
+    }
+    auto fwd = [&](auto C, int t) {
+        constexpr int sl = decltype(C)::value;
+        ld((sl + SD) % NS, min(t + SD, steps - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        const int b = t & 1, c0 = t - l0 - jj;   // column of line l less one: c0 - l
+        T *u = U + (long)t * sk.len;
+        const T kl = sK[b ^ 1][tid >= nyp ? tid - nyp : tid], kin = tid >= nyp ? kl : T(0);
+        // the lines side by side, so that their dependent chains overlap
+        T a[KL], y[KL], z[KL];
+#pragma unroll
+        for (int l = 0; l < KL; l++) {
+            const T rw = c0 == l ? T(0) : xprev[l];                           // column 1
+            const T rs = lane_up(xprev[l], sW[b ^ 1][first ? MT / 64 : w - 1][l]);
+            const T rb = l == 0 ? kin : xprev[l - 1];
+            a[l] = rv[sl][l] + Aw * rw;
+            y[l] = As * rs;
+            z[l] = Abk[l] * rb;
+        }
+#pragma unroll
+        for (int l = 0; l < KL; l++) a[l] = a[l] + y[l];
+#pragma unroll
+        for (int l = 0; l < KL; l++) a[l] = -om * (a[l] + z[l]);
+#pragma unroll
+        for (int l = 0; l < KL; l++) xprev[l] = a[l] * rAp[l];
+#pragma unroll
+        for (int l = 0; l < KL; l++) sk_at(u, off[l]) = bAp[l] * xprev[l];
+        if (lane == 63) {
+#pragma unroll
+            for (int l = 0; l < KL; l++) sW[b][w][l] = xprev[l];
+        }
+        sK[b][tid] = xprev[KL - 1];
+        lds_barrier();
     };
     int t = 0;
     for (; t + NS <= steps; t += NS) ring_steps<0, NS>(fwd, t);
     ring_tail<0, NS>(fwd, t, steps);
+    __syncthreads();
     // backward: mirrored coordinates (nx-1-ii, ny-1-jj, nk-1-kk); the new
     // neighbours are i+1 (itself), j+1 (next lane) and k+1 (next line)
 #pragma unroll
     for (int l = 0; l < KL; l++) xprev[l] = T(0);
-    const int jr = ny - 1 - jj;
-    auto ld_b = [&](int sl, int t) {
+#pragma unroll
+    for (int m = 0; m < SD; m++) {
+        ld(m, max(steps - 1 - m, 0));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int Ln = last ? (ny - 1) & 63 : 64;                                // lane of row nY-2
+    auto bwd = [&](auto C, int t) {
+        constexpr int sl = decltype(C)::value;
+        const int tb = steps - 1 - t;
+        ld((sl + SD) % NS, max(tb - SD, 0));
+        __builtin_amdgcn_sched_barrier(0);
+        const int b = t & 1, c0 = tb - l0 - jj - (nx - 1);
+        T *u = U + (long)tb * sk.len;
+        const T kl = sK[b ^ 1][kc < nkc - 1 ? tid + nyp : tid], kin = kc < nkc - 1 ? kl : T(0);
+        T a[KL], y[KL], z[KL];
 #pragma unroll
         for (int l = 0; l < KL; l++) {
-            const int ir = min(max(t - jr - (nk - 1 - (kc * KL + l)), 0), nx - 1);
-            rv[sl][l] = out[c0l[l] + (nx - 1 - ir)];
+            const T re = c0 == l ? T(0) : xprev[l];                           // column nX-2
+            const T sw = sW[b ^ 1][last ? w : w + 1][l];
+            T rn = lane_dn(xprev[l], sw);
+            rn = lane == Ln ? T(0) : rn;
+            T rt = l == KL - 1 ? kin : xprev[l + 1];
+            rt = l0 + l == nk - 1 ? T(0) : rt;
+            a[l] = rv[sl][l] + Ae * re;
+            y[l] = An * rn;
+            z[l] = Atk[l] * rt;
         }
-    };
 #pragma unroll
-    for (int q = 0; q < SD; q++) ld_b(q, q);
-    auto bwd = [&](auto S, int t) {
-        constexpr int sl = decltype(S)::value;
-        ld_b((sl + SD) % NS, t + SD);
-        const int b = t & 1;
-        const T kin = kc < nkc - 1 ? sK[b ^ 1][tid + nyp] : T(0);
-        // lowest line first: line l reads line l+1's value of step t-1
+        for (int l = 0; l < KL; l++) a[l] = a[l] + y[l];
 #pragma unroll
-        for (int l = 0; l < KL; l++) {
-            T sj = __shfl_down(xprev[l], 1, 64);              // row jj+1, step t-1
-            if (lane == 63 && jj < ny - 1) sj = sW[b ^ 1][w + 1][l];
-            const int kk = kc * KL + l, ir = t - jr - (nk - 1 - kk), ii = nx - 1 - ir;
-            if (live && kk < nk && ir >= 0 && ir < nx) {
-                const long c = c0l[l] + ii;
-                const T re = ii == nx - 1 ? T(0) : xprev[l];
-                const T rn = jj == ny - 1 ? T(0) : sj;
-                const T rt = kk == nk - 1 ? T(0) : (l == KL - 1 ? kin : xprev[l + 1]);
-                const T v = -om * (rv[sl][l] + T(g.Ae) * re + T(g.An) * rn + Atk[l] * rt) * rApk[l];
-                out[c] = v;
-                xprev[l] = v;
-            }
-        }
+        for (int l = 0; l < KL; l++) a[l] = -om * (a[l] + z[l]);
+#pragma unroll
+        for (int l = 0; l < KL; l++) xprev[l] = a[l] * rAp[l];
+#pragma unroll
+        for (int l = 0; l < KL; l++) sk_at(u, off[l]) = xprev[l];
         if (lane == 0) {
 #pragma unroll
             for (int l = 0; l < KL; l++) sW[b][w][l] = xprev[l];
         }
         sK[b][tid] = xprev[0];
-        __syncthreads();
+        lds_barrier();
     };
     t = 0;
     for (; t + NS <= steps; t += NS) ring_steps<0, NS>(bwd, t);
     ring_tail<0, NS>(bwd, t, steps);
 }
 
-int slab_threads(const Geo &g, int nkmax)
-{
-    int KL, nkc, nyp;
-    return slab_shape(g, nkmax, KL, nkc, nyp);
-}
-template <class T>
-void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *halo, const void *ctrl, int nkmax, hipStream_t s)
-{
-    int KL, nkc, nyp;
-    const int nt = slab_shape(g, nkmax, KL, nkc, nyp);
-    const GsCtrl *gc = (const GsCtrl *)ctrl;
-    hipLaunchKernelGGL(k_slab_halo<T>, dim3((unsigned)((g.sZ + 255) / 256), 2 * g.nslab, 3), dim3(256), 0, s, g,
-                       (const T *)Ut, halo, gc);
-    const dim3 grid(g.nslab, 3), blk(nt);
-    switch (KL) {
-    case 4: hipLaunchKernelGGL((k_helm_lex<T, 4>), grid, blk, 0, s, g, Q, Ut, (const T *)halo, gc, nkc, nyp); break;
-    case 8: hipLaunchKernelGGL((k_helm_lex<T, 8>), grid, blk, 0, s, g, Q, Ut, (const T *)halo, gc, nkc, nyp); break;
-    case 16: hipLaunchKernelGGL((k_helm_lex<T, 16>), grid, blk, 0, s, g, Q, Ut, (const T *)halo, gc, nkc, nyp); break;
-    default: hipLaunchKernelGGL((k_helm_lex<T, 32>), grid, blk, 0, s, g, Q, Ut, (const T *)halo, gc, nkc, nyp); break;
+// CASE(KL, threads, steps that Gauss-Seidel and SSOR load ahead): what the
+// registers of the workgroup's threads hold, of KL + 2 loads a line and one a line
+#define SLAB_CASES(CASE)                                                                                             \
+    switch (KL) {                                                                                                    \
+    case 1: CASE(1, 1024, 4, 8); break;                                                                              \
+    case 2: CASE(2, 1024, 3, 6); break;                                                                              \
+    case 5: CASE(5, 512, 2, 5); break;                                                                               \
+    case 6: CASE(6, 512, 2, 4); break;                                                                               \
+    case 8: CASE(8, 1024, 0, 2); break;                                                                              \
+    default: CASE(32, 512, 1, 1); break;                                                                             \
     }
-}
 template <class T>
-static void launch_ssor_block(const Geo &g, const T *r, T *out, const int *active, hipStream_t s)
+void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *scr, const void *ctrl, hipStream_t s)
 {
     int KL, nkc, nyp;
     const int nt = slab_shape(g, g.nkmax, KL, nkc, nyp);
-    const dim3 grid(g.nslab), blk(nt);
-    switch (KL) {
-    case 4: hipLaunchKernelGGL((k_ssor_block<T, 4>), grid, blk, 0, s, g, r, out, active, nkc, nyp); break;
-    case 8: hipLaunchKernelGGL((k_ssor_block<T, 8>), grid, blk, 0, s, g, r, out, active, nkc, nyp); break;
-    case 16: hipLaunchKernelGGL((k_ssor_block<T, 16>), grid, blk, 0, s, g, r, out, active, nkc, nyp); break;
-    default: hipLaunchKernelGGL((k_ssor_block<T, 32>), grid, blk, 0, s, g, r, out, active, nkc, nyp); break;
-    }
+    const Skew sk = skew_of(g);
+    const GsCtrl *gc = (const GsCtrl *)ctrl;
+    const size_t ring = sizeof(T) * (size_t)(nkc * KL) * (g.nY - 2);
+    launch_skew<T, true>(g, sk, Ut, Q, scr, nullptr, gc->active, 1, 6, s);
+#define LEX_CASE(kl, mt, sd, sds) \
+    hipLaunchKernelGGL((k_helm_lex<T, kl, mt, sd>), dim3(g.nslab, 3), dim3(nt), ring, s, g, sk, scr, gc, nkc)
+    SLAB_CASES(LEX_CASE)
+#undef LEX_CASE
+    launch_skew<T, false>(g, sk, nullptr, nullptr, scr, Ut, gc->active, 0, 3, s);
 }
+template <class T>
+static void launch_ssor_block(const Geo &g, const T *r, T *scr, T *out, const int *active, hipStream_t s)
+{
+    int KL, nkc, nyp;
+    const int nt = slab_shape(g, g.nkmax, KL, nkc, nyp);
+    const Skew sk = skew_of(g);
+    launch_skew<T, true>(g, sk, r, nullptr, scr, nullptr, active, 0, 1, s);
+#define SSOR_CASE(kl, mt, sd, sds) \
+    hipLaunchKernelGGL((k_ssor_block<T, kl, mt, sds>), dim3(g.nslab), dim3(nt), 0, s, g, sk, scr, active, nkc)
+    SLAB_CASES(SSOR_CASE)
+#undef SSOR_CASE
+    launch_skew<T, false>(g, sk, nullptr, nullptr, scr, out, active, 0, 1, s);
+}
+#undef SLAB_CASES
 
 template <class T>
 void launch_precond(const Geo &g, int pc, const FastPC *fast, const T *r, T *scratch, T *out, const int *active,
@@ -2085,7 +2302,7 @@ void launch_precond(const Geo &g, int pc, const FastPC *fast, const T *r, T *scr
     if (pc == PC_FAST) {
         run_fastpc<T>(fast, g, r, out, active, s, part);
     } else if (pc == PC_SSOR_BLOCK) {
-        launch_ssor_block<T>(g, r, out, active, s);
+        launch_ssor_block<T>(g, r, scratch, out, active, s);
     } else if (pc == PC_SSOR_RB) {
         hipLaunchKernelGGL(k_ssor_fwd<T>, pairs3(g), dim3(256), 0, s, g, r, scratch, active);
         unsigned nbx = (g.nX - 1 + 63) / 64, nby = (g.nY - 2 + 3) / 4, nbz = g.nZ - 2;
@@ -2138,7 +2355,7 @@ void launch_recycle(const Geo &g, T *Ut, int i_rec0, double eps, const double *l
     template void launch_helm_zebra<T>(const Geo &, const T *, const T *, const T *, T *, const T *, const void *, int, \
                                        hipStream_t);                                                                    \
     template void launch_copy_faces3<T>(const Geo &, const T *, T *, void *, hipStream_t);                                     \
-    template void launch_helm_lex<T>(const Geo &, const T *, T *, T *, const void *, int, hipStream_t);                \
+    template void launch_helm_lex<T>(const Geo &, const T *, T *, T *, const void *, hipStream_t);                     \
     template void launch_ppe_rhs<T>(const Geo &, const T *, double *, hipStream_t, const void *);          \
     template unsigned launch_poisson<T>(const Geo &, const T *, T *, const int *, const double *, hipStream_t, \
                                         const T *, double *);                                              \
