@@ -145,3 +145,22 @@ def test_slab_sweeps(tbl, grid, P, precision):
     else:
         assert np.abs(Ut - Uo).max() <= 1e-4 * np.abs(Uo).max()
         assert np.abs(y[I] - yo[I]).max() <= 1e-4 * np.abs(yo[I]).max()
+
+
+# chunks of the FP64 reductions: one plane, a few with a shorter last chunk, the
+# 12-plane limit, and few planes on many tiles.  A sum of n terms in another order
+# moves by at most n eps sum |terms|
+@pytest.mark.parametrize("grid", [(8, 8, 8), (66, 130, 131), (520, 130, 97), (700, 200, 150), (1500, 400, 8)])
+def test_reduction_chunks(tbl, grid):
+    g, s = make_case(grid, seed=5)
+    _, Q = g.momentum_rhs(s.Ut, s.Press)
+    n = (grid[0] - 2) * (grid[1] - 2) * (grid[2] - 2)
+    with gpu_from_case(g, s) as sv:
+        _, sdiv = sv.div_check()
+        sv.set_field(tbl.F_Q, Q)
+        _, res = sv.diffusion_solve(1e-30, 1)
+    _, sdivo = g.div_check(s.Ut)
+    mag = np.abs(g.ppe_rhs(s.Ut)).sum() * g.dt * 10 + 1.0
+    assert abs(sdiv - sdivo) <= n * 2.2e-16 * mag
+    _, reso = g.diffusion_solve(Q, s.Ut.copy(order="F"), order=orc.GS_LEX_BLOCK, errorstop=1e-30, mmax=1)
+    assert np.all(np.abs(res - reso) <= n * 2.2e-16 * reso)

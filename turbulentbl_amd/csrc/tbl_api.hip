@@ -314,6 +314,8 @@ static int create_impl(tbl_ctx *c)
     if (p.tol_mode == TBL_TOL_TRUE) CHK(dalloc(c, &c->Z, (size_t)p.kmax * c->ldv * c->es));
     if (p.helm_mode == TBL_HELM_ZEBRA) CHK(dalloc(c, &c->Ualt, 3 * N * c->es));
     c->g.nslab = 0; c->g.nkmax = 0; c->g.slab = nullptr;
+    c->g.rblk = c->mixed ? 8192 : 2048;
+    c->g.rpl = c->mixed ? p.nZ : 12;
     size_t nscr = N;
     if (p.helm_mode == TBL_HELM_LEX_SLAB || p.precond == TBL_PC_SSOR_BLOCK) {
         // the reference's slab bounds (dnssetbl.f90:76-92): nZ/P planes per

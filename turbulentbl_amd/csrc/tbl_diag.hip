@@ -437,7 +437,7 @@ __global__ void k_tau_window(int nX, int nY, double Ue, int window, double *acc,
 // ---------------------------------------------------------------- launchers
 static inline dim3 rgrid(const Geo &g, int *kchunk)
 {
-    RTiles r = rtiles_of(g.nX, g.nY, g.nZ);
+    RTiles r = rtiles_of(g);
     *kchunk = r.kchunk;
     return dim3(r.gx, r.gy, r.kb);
 }

@@ -1575,11 +1575,11 @@ static inline dim3 tiles3(const Geo &g) { return dim3((g.nX - 1 + 63) / 64, (g.n
 static inline dim3 pairs3(const Geo &g) { return dim3(((g.nX - 1) / 2 + 63) / 64, (g.nY - 2 + 3) / 4, g.nZ - 2); }
 static inline dim3 rgrid(const Geo &g, int *kchunk)
 {
-    RTiles r = rtiles_of(g.nX, g.nY, g.nZ);
+    RTiles r = rtiles_of(g);
     *kchunk = r.kchunk;
     return dim3(r.gx, r.gy, r.kb);
 }
-unsigned resid_blocks(const Geo &g) { RTiles r = rtiles_of(g.nX, g.nY, g.nZ); return (unsigned)(r.gx * r.gy * r.kb); }
+unsigned resid_blocks(const Geo &g) { RTiles r = rtiles_of(g); return (unsigned)(r.gx * r.gy * r.kb); }
 
 // planes per block of the momentum kernels: the column is cut into the
 // number of chunks that minimises (waves of blocks over the resident slots) x
