@@ -606,24 +606,27 @@ static void *field_ptr(tbl_ctx *c, int f, bool *is_double)
 // threads convert and copy between the chunks and the host array.  The ring
 // belongs to the context (XF_SLOTS chunks, allocated by the first transfer).
 // Up / down, before -> after: 1024x256x192 mixed velocity 167 / 213 -> 19 / 23
-// ms, 512x128x128 FP64 6.9 / 19.4 -> 5.1 / 5.6 ms; 4 to 16 threads differ by
-// 10 %, chunks of 64 k values take twice as long.  FP64 fields that a pageable
-// copy moves sooner take it (move_field): up to 2 M values to the device
-// (90x80x50: 0.25 against 0.30 ms) and half a million from it.
+// ms, 512x128x128 FP64 6.9 / 19.4 -> 5.1 / 5.9 ms; 4 to 16 threads differ by
+// 10 %, 2 take half as long again from the device, chunks of 64 k values twice
+// as long.  Four threads that sleep while they wait: eight that yielded ran a
+// process whose other threads were busy into its CPU quota (16 cores), and an
+// upload of 18 M values that takes 4 ms took 38.  FP64 fields that a pageable
+// copy moves sooner take it (move_field): up to 3 M values to the device
+// (128x80x80 velocity: 0.56 against 0.66 ms) and half a million from it.
 #define XF_SLOTS 8
 #define XF_CHUNK ((size_t)1 << 18)       // elements per chunk: 2 MB of doubles
-#define XF_THREADS 8
+#define XF_THREADS 4
+#define XF_NAP std::this_thread::sleep_for(std::chrono::microseconds(10))
 struct XferRing {
-    char *buf[XF_SLOTS] = {nullptr};
+    char *mem = nullptr, *buf[XF_SLOTS] = {nullptr};     // buf: into mem
     hipEvent_t ev[XF_SLOTS] = {nullptr};
 };
 static void ring_free(tbl_ctx *c)
 {
     if (!c->ring) return;
-    for (int q = 0; q < XF_SLOTS; q++) {
-        if (c->ring->buf[q]) hipHostFree(c->ring->buf[q]);
+    if (c->ring->mem) hipHostFree(c->ring->mem);
+    for (int q = 0; q < XF_SLOTS; q++)
         if (c->ring->ev[q]) hipEventDestroy(c->ring->ev[q]);
-    }
     delete c->ring;
     c->ring = nullptr;
 }
@@ -631,13 +634,15 @@ static int ring_get(tbl_ctx *c)
 {
     if (c->ring) return 0;
     c->ring = new XferRing();
-    for (int q = 0; q < XF_SLOTS; q++) {
-        hipError_t e = hipHostMalloc((void **)&c->ring->buf[q], XF_CHUNK * sizeof(double), hipHostMallocDefault);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ring->ev[q], hipEventDisableTiming);
-        if (e != hipSuccess) {
-            ring_free(c);
-            HIPCHK(c, e);
-        }
+    const size_t slot = XF_CHUNK * sizeof(double);
+    hipError_t e = hipHostMalloc((void **)&c->ring->mem, XF_SLOTS * slot, hipHostMallocDefault);
+    for (int q = 0; q < XF_SLOTS && e == hipSuccess; q++) {
+        c->ring->buf[q] = c->ring->mem + q * slot;
+        e = hipEventCreateWithFlags(&c->ring->ev[q], hipEventDisableTiming);
+    }
+    if (e != hipSuccess) {
+        ring_free(c);
+        HIPCHK(c, e);
     }
     return 0;
 }
@@ -654,7 +659,7 @@ static void chunk_convert(char *slot, bool dbl, double *host, size_t m, bool to_
 // when they have arrived
 static int move_field(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, bool to_dev)
 {
-    if (dbl && n < (to_dev ? 8 : 2) * XF_CHUNK) {
+    if (dbl && n < (to_dev ? 12 : 2) * XF_CHUNK) {
         HIPCHK(c, to_dev ? hipMemcpyAsync(dev, host, n * sizeof(double), hipMemcpyHostToDevice, c->s)
                          : hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c->s));
         HIPCHK(c, hipStreamSynchronize(c->s));
@@ -692,7 +697,7 @@ static int move_field(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, b
         for (long q; (q = next.fetch_add(1)) < nch;) {
             while (ready.load(std::memory_order_acquire) <= q) {
                 if (err.load()) return;
-                sched_yield();
+                XF_NAP;
             }
             if (err.load()) return;
             convert(q);
@@ -707,7 +712,7 @@ static int move_field(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, b
     // without workers the calling thread converts each chunk itself
     auto wait_done = [&](long q) {
         if (pool.empty()) { if (!done[q].load()) convert(q); return; }
-        while (!done[q].load(std::memory_order_acquire) && !err.load()) sched_yield();
+        while (!done[q].load(std::memory_order_acquire) && !err.load()) XF_NAP;
     };
     long freed = 0;
     for (long q = 0; q < nch && !err.load(); q++) {
