@@ -164,3 +164,17 @@ def test_reduction_chunks(tbl, grid):
     assert abs(sdiv - sdivo) <= n * 2.2e-16 * mag
     _, reso = g.diffusion_solve(Q, s.Ut.copy(order="F"), order=orc.GS_LEX_BLOCK, errorstop=1e-30, mmax=1)
     assert np.all(np.abs(res - reso) <= n * 2.2e-16 * reso)
+
+
+# k groups of the FP64 transforms: one (8 rows are less than a group), two, three,
+# four, five and eight, odd counts and partly filled last groups.  The inverse of A
+# applied to A x gives x up to rounding times the operator's condition (1e3 to 1e6
+# on these grids)
+@pytest.mark.parametrize("grid", [(16, 8, 10), (20, 34, 18), (24, 50, 45), (20, 66, 66), (16, 82, 50), (12, 130, 130)])
+def test_transform_groups(tbl, grid):
+    g, s = make_case(grid, seed=7)
+    x = g.zeros()
+    x[I] = np.random.default_rng(4).standard_normal([n - 2 for n in grid])
+    with gpu_from_case(g, s, precond=tbl.TBL_PC_FAST) as sv:
+        y = sv.apply_operator(1, g.poisson_apply(x))
+    assert np.abs(y[I] - x[I]).max() <= 1e-9 * np.abs(x).max()

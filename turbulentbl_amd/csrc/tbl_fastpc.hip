@@ -438,8 +438,7 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
     // has its own staging registers (as in the FP32 kernel): the step of group
     // g masks A(g), issues the loads of group g + 2 into the registers it has
     // just freed, forms the 4 MT NT products from LDS buffer g % 2, then
-    // stores the B slice of group g + 1 into the other buffer.  The group
-    // count is padded to even; a padding group's A values are masked to zero.
+    // stores the B slice of group g + 1 into the other buffer.
     double an[2][4 * MT];
     double st[2][NT];
     ldA(0, an[0]);
@@ -449,7 +448,7 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
 #pragma unroll
     for (int q = 0; q < NT; q++) sB[0][q * 256 + t] = st[0][q];
     __syncthreads();
-    auto step = [&](int kg, auto bc) {
+    auto step = [&](int kg, auto bc, auto ld) {
         constexpr int b = decltype(bc)::value;
         double a[4 * MT];
 #pragma unroll
@@ -459,8 +458,10 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
             for (int mt = 0; mt < MT; mt++) a[mt * 4 + ks] = kin && aok[mt] ? an[b][mt * 4 + ks] : 0.0;
         }
         __builtin_amdgcn_sched_barrier(0);
-        ldA(kg + 2, an[b]);
-        ldB(kg + 2, st[b]);
+        if constexpr (decltype(ld)::value) {
+            ldA(kg + 2, an[b]);
+            ldB(kg + 2, st[b]);
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int ks = 0; ks < 4; ks++)
@@ -471,13 +472,42 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
                 for (int mt = 0; mt < MT; mt++)
                     acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf, a[mt * 4 + ks], acc[mt][nt], 0, 0, 0);
             }
+        if (MT == 2 || kg + 1 < KG) {
 #pragma unroll
-        for (int q = 0; q < NT; q++) sB[b ^ 1][q * 256 + t] = st[b ^ 1][q];
-        __syncthreads();
+            for (int q = 0; q < NT; q++) sB[b ^ 1][q * 256 + t] = st[b ^ 1][q];
+            __syncthreads();
+        }
     };
-    for (int kg = 0; kg < KG; kg += 2) {
-        step(kg, std::integral_constant<int, 0>{});
-        step(kg + 1, std::integral_constant<int, 1>{});
+    constexpr std::integral_constant<int, 0> p0{};
+    constexpr std::integral_constant<int, 1> p1{};
+    int kg = 0;
+    if constexpr (MT == 1) {
+        // The last two steps have no group left to load, and an odd count ends
+        // on the first parity.  With clamped loads there and the count padded to
+        // even, 62 span rows loaded six groups for four, and 43 planes formed four
+        // for three: the transforms of 256x64x96, three components, 30.5 -> 28.5
+        // and 24 -> 22.4 us, one 13.6 -> 11.7 and 10.7 -> 8.8; a step of 90x80x50
+        // 341 -> 327 us.
+        for (; kg + 3 < KG; kg += 2) {
+            step(kg, p0, std::true_type{});
+            step(kg + 1, p1, std::true_type{});
+        }
+        if (KG - kg == 3) {
+            step(kg, p0, std::true_type{});
+            step(kg + 1, p1, std::false_type{});
+            step(kg + 2, p0, std::false_type{});
+        } else {
+            step(kg, p0, std::false_type{});
+            if (KG - kg == 2) step(kg + 1, p1, std::false_type{});
+        }
+    } else {
+        // Two row tiles, on many rows: the count is padded to even (a padding
+        // group's A values are masked to zero).  With the ending above a step of
+        // 1024x256x192 took 11.5 instead of 11.2 ms; the FP32 kernel the same.
+        for (; kg < KG; kg += 2) {
+            step(kg, p0, std::true_type{});
+            step(kg + 1, p1, std::true_type{});
+        }
     }
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
