@@ -223,7 +223,8 @@ class Solver:
         self._chk(self.lib.tbl_checkpoint_load(self.h, os.fsencode(path)))
 
     def set_field(self, f, a):
-        self._chk(self.lib.tbl_field_set(self.h, f, _ptr(_f64(a))))
+        a = _f64(a)                                          # held until the call returns
+        self._chk(self.lib.tbl_field_set(self.h, f, _ptr(a)))
 
     def get_field(self, f):
         out = self.zeros(3) if f in (F_UT, F_UTOLD, F_Q) else self.zeros()
@@ -339,8 +340,8 @@ class Solver:
         return [d[q].as_dict() for q in range(n)]
 
     def apply_operator(self, op, x):
-        out = self.zeros()
-        self._chk(self.lib.tbl_apply_operator(self.h, op, _ptr(_f64(x)), _ptr(out)))
+        x, out = _f64(x), self.zeros()
+        self._chk(self.lib.tbl_apply_operator(self.h, op, _ptr(x), _ptr(out)))
         return out
 
     # -- timers
