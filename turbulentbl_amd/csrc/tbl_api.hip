@@ -1321,7 +1321,8 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         // operator apply, the dot product and the orthogonalisation pass of
         // the Arnoldi step are not run, nor the read-back at the solve's start.
         // The step's residual goes to the other of two vectors (v0, v1), so
-        // that a refused step leaves v_0 for the Arnoldi steps.
+        // that a refused step leaves v_0 for the Arnoldi steps; the other is W,
+        // which these solves do not use otherwise (r is the caller's TBL_F_WORK).
         // Mixed contexts run the Arnoldi step: its coefficient differs from 1
         // in the seventh digit there, and a PCorr that differs at all moves
         // some value of the FP32 fields by a rounding, which grows to what
@@ -1330,7 +1331,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         bool unit = unit_steps;
         bool opened = false;                   // the last unit step opened this cycle
         bool head = false;                     // its first transform ran behind the last read-back
-        T *v0 = V, *v1 = r;
+        T *v0 = V, *v1 = W;
         for (int m = 0; m < mmax; m++) {
             const bool try_unit = unit && m + 1 < mmax;   // the last cycle allowed is not followed by a start
             if (opened) {
