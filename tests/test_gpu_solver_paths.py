@@ -1,5 +1,7 @@
 """Pressure and direct solves: the routes a solve takes when its first step is
 not enough, and the buffers it shares with the caller."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -39,3 +41,29 @@ def test_true_residual_solve_leaves_the_work_field(tbl):
         sv.set_field(tbl.F_WORK, w)
         _solve(tbl, sv, g, b, errtol=1e-10)
         assert np.array_equal(sv.get_field(tbl.F_WORK)[I], w[I])
+
+
+def _solver(tbl, grid, **kw):
+    nX = grid[0]
+    return tbl.Solver(*grid, i_rec=int(0.8 * (nX - 1)), planes=(2, 3, 4, 5, 6), **kw)
+
+
+def test_device_bytes_are_those_held(tbl):
+    """what a context takes from the device, first solves included"""
+    hip = C.CDLL("libamdhip64.so.7")             # the runtime that the library is linked to
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    for grid, kw in (((900, 96, 64), dict(helm_mode=tbl.TBL_HELM_DIRECT)), ((256, 96, 64), dict(helm_mode=tbl.TBL_HELM_DIRECT)),
+                     ((1024, 8, 130), dict(helm_mode=tbl.TBL_HELM_LEX_SLAB, precond=tbl.TBL_PC_SSOR_BLOCK, slabs=64))):
+        before = free()
+        with _solver(tbl, grid, kmax=4, **kw) as sv:
+            sv.upload(sv.zeros(3))
+            sv.diffusion_solve(1e-6, 1)
+            sv.ppe_solve(1e-5, 4, 1)
+            taken = before - free()
+            # each of some 45 allocations takes whole 2 MB pages
+            assert 0.98 * sv.device_bytes <= taken <= sv.device_bytes + 100e6

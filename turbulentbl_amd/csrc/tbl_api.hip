@@ -57,6 +57,7 @@ struct tbl_ctx {
     long ldv = 0;
     double *part = nullptr;
     size_t npart = 0;
+    size_t bytes = 0;                    // device memory held, without the fast solver's own
     GmCtrl *gm = nullptr;
     // pinned host block that kernels publish their results to (see Pub), and
     // its parts: GMRES status, Gauss-Seidel control, diagnostics record
@@ -252,10 +253,18 @@ extern "C" void tbl_default_params(tbl_params *p)
 
 static int h2d(tbl_ctx *c, void *d, const void *h, size_t b);
 
+// device memory of the context, cleared; its sum is what tbl_device_bytes reports
+template <class X> static hipError_t alloc_clear(tbl_ctx *c, X **ptr, size_t bytes)
+{
+    if (bytes == 0) bytes = 8;
+    hipError_t e = hipMalloc((void **)ptr, bytes);
+    if (e != hipSuccess) { *ptr = nullptr; return e; }
+    c->bytes += bytes;
+    return hipMemsetAsync(*ptr, 0, bytes, c->s);
+}
 template <class X> static int dalloc(tbl_ctx *c, X **ptr, size_t bytes)
 {
-    HIPCHK(c, hipMalloc((void **)ptr, bytes ? bytes : 8));
-    HIPCHK(c, hipMemsetAsync(*ptr, 0, bytes ? bytes : 8, c->s));
+    HIPCHK(c, alloc_clear(c, ptr, bytes));
     return 0;
 }
 
@@ -568,12 +577,7 @@ extern "C" int tbl_sync(tbl_ctx *c)
 extern "C" double tbl_device_bytes(const tbl_ctx *c)
 {
     if (!c) return 0.0;
-    const tbl_params &p = c->p;
-    const double N = (double)p.nX * p.nY * p.nZ, M = (double)p.nX * p.nZ;
-    double b = (3 * 3 + 1) * N * c->es + 2 * N * 8 + ((double)(p.kmax + 1) * c->ldv + 3 * N) * c->es;
-    if (c->Ualt) b += 3 * N * c->es;
-    b += (18 * M + M) * 8 + c->npart * 8 + sizeof(GmCtrl);
-    return b;
+    return (double)(c->bytes + (c->fast ? fastpc_bytes(c->fast) : 0));
 }
 
 // ------------------------------------------------------------------ fields
@@ -1096,18 +1100,19 @@ template <class T> static int helm_direct(tbl_ctx *c, int *sweeps, double *res)
     const long N = g.N;
     CHK(direct_work(c));
     const int nc = solve_batched(g, c->mixed) ? 3 : 1;         // components per solve
+    T *r = F<T>(c->r3);
     const double h = c->p.dt / c->p.Re;
     const int passes = sizeof(T) == sizeof(double) ? 2 : 1;
     for (int p = 0; p < 3; p += nc) {
         FastIO io;
-        io.in = c->r3;
+        io.in = r;
         io.out = F<T>(c->Ut) + p * N;
         io.in64 = io.out64 = sizeof(T) == sizeof(double);
         io.add = 1;
         io.ncomp = nc;
         for (int it = 0; it < passes; it++) {
             Tscope ts(c, TBL_K_HELM, 4.0 * nc * (double)N * sizeof(T));
-            launch_helm_rfield<T>(g, F<T>(c->Q) + p * N, F<T>(c->Ut) + p * N, F<T>(c->r3), nc, c->s);
+            launch_helm_rfield<T>(g, F<T>(c->Q) + p * N, F<T>(c->Ut) + p * N, r, nc, c->s);
             if (run_fast_solve(c->fast, g, io, nullptr, 1.0, -h, false, c->s))
                 return fail(c, TBL_EARG, "fast solver failure in the direct Helmholtz solve");
         }
@@ -1958,6 +1963,7 @@ static int solve_T(tbl_ctx *c, const double *b, double *x, double alpha, double 
     const Geo &g = c->g;
     const int nc = solve_batched(g, c->mixed) ? ncomp : 1;
     CHK(direct_work(c));
+    void *r = c->r3;
     for (int p = 0; p < ncomp; p += nc) {
         const double *bp = b + (long)p * g.N;
         double *xp = x + (long)p * g.N;
@@ -1967,9 +1973,9 @@ static int solve_T(tbl_ctx *c, const double *b, double *x, double alpha, double 
         io.in64 = io.out64 = io.mask = 1;
         io.ncomp = nc;
         if (run_fast_solve(c->fast, g, io, nullptr, alpha, beta, true, c->s)) return fail(c, TBL_EARG, "fast solver failure");
-        if (c->mixed) launch_opT_res<float>(g, bp, xp, alpha, beta, F<float>(c->r3), nc, c->s);
-        else launch_opT_res<double>(g, bp, xp, alpha, beta, F<double>(c->r3), nc, c->s);
-        io.in = c->r3;
+        if (c->mixed) launch_opT_res<float>(g, bp, xp, alpha, beta, F<float>(r), nc, c->s);
+        else launch_opT_res<double>(g, bp, xp, alpha, beta, F<double>(r), nc, c->s);
+        io.in = r;
         io.in64 = !c->mixed;
         io.mask = 0;
         io.add = 1;
@@ -2105,6 +2111,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         if (c->br_steps < o->nsteps) {
             if (c->br) hipFree(c->br);
             c->br = nullptr;
+            c->bytes -= (size_t)c->br_steps * N;
             c->br_steps = 0;
             CHK(dalloc(c, &c->br, (size_t)o->nsteps * N));
             c->br_steps = o->nsteps;

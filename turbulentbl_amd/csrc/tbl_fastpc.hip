@@ -43,6 +43,7 @@ struct FastPC {
     double *ly = nullptr, *lz = nullptr;                 // eigenvalues (full-index arrays)
     void *t1 = nullptr, *t2 = nullptr;                   // work fields (storage type), ncap components each
     int ncap = 1;
+    size_t bytes = 0;                                    // device memory held
     bool single = false;
     // FP32 storage: the transform matrices split into three bf16 parts in
     // matrix-core fragment order (see k_xform): z forward, y forward, y
@@ -623,7 +624,10 @@ int fastpc_create(const Geo &g, const double *Ab, const double *At, const double
     }
     const size_t es = single ? sizeof(float) : sizeof(double);
     hipError_t e = hipSuccess;
-    auto al = [&](void **p, size_t b) { if (hipMalloc(p, b) != hipSuccess) e = hipErrorOutOfMemory; };
+    auto al = [&](void **p, size_t b) {
+        if (hipMalloc(p, b) != hipSuccess) e = hipErrorOutOfMemory;
+        else f->bytes += b;
+    };
     al((void **)&f->ly, sizeof(double) * g.nY);
     al((void **)&f->lz, sizeof(double) * g.nZ);
     al(&f->t1, es * g.N);
@@ -844,25 +848,32 @@ static void launch_line_solve(const Geo &g, T *d, const double *ly, const double
 // Three components go through one solve while its two work fields stay in
 // the 256 MB last-level cache (6 N values; FP32 operands of a batch then also
 // stay within the transforms' 32-bit byte offsets).  Beyond it a solve of one
-// component still keeps them there and the batch does not: 1024x192x160 FP32,
-// a
+// component still keeps them there and the batch does not: 1024x192x160 FP32, a
 // component's launches take 509 us batched, 379 us one by one.
 bool solve_batched(const Geo &g, bool single) { return 6.0 * (double)g.N * (single ? 4 : 8) <= 256e6; }
+
+size_t fastpc_bytes(const FastPC *f) { return f->bytes; }
 
 int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s)
 {
     if (!f || ncomp <= f->ncap) return f ? 0 : 1;
-    const size_t b = (f->single ? sizeof(float) : sizeof(double)) * (size_t)g.N * ncomp;
+    const size_t b1 = (f->single ? sizeof(float) : sizeof(double)) * (size_t)g.N, b = b1 * ncomp;
     void *n1 = nullptr, *n2 = nullptr;
     if (hipStreamSynchronize(s) != hipSuccess) return 1;
-    if (hipMalloc(&n1, b) != hipSuccess) return 1;
-    if (hipMalloc(&n2, b) != hipSuccess) { hipFree(n1); return 1; }
+    if (hipMalloc(&n1, b) != hipSuccess || hipMalloc(&n2, b) != hipSuccess || hipMemsetAsync(n1, 0, b, s) != hipSuccess ||
+        hipMemsetAsync(n2, 0, b, s) != hipSuccess) {
+        if (n1) hipFree(n1);
+        if (n2) hipFree(n2);
+        (void)hipGetLastError();               // the caller does with fewer components
+        return 1;
+    }
     hipFree(f->t1);
     hipFree(f->t2);
     f->t1 = n1;
     f->t2 = n2;
+    f->bytes += 2 * b1 * (ncomp - f->ncap);
     f->ncap = ncomp;
-    return hipMemsetAsync(n1, 0, b, s) == hipSuccess && hipMemsetAsync(n2, 0, b, s) == hipSuccess ? 0 : 1;
+    return 0;
 }
 
 // out = (alpha I + beta A)^{-1} in, or its transpose, on the interior planes

@@ -87,8 +87,10 @@ struct FastIO {
 // out = (alpha I + beta A)^{-1} in, or its transpose
 int run_fast_solve(const FastPC *f, const Geo &g, const FastIO &io, const int *active, double alpha, double beta,
                    bool transpose, hipStream_t s, int part = FPC_ALL);
-// work fields for solves of ncomp components (synchronises when they grow);
-// solve_batched: whether three components may go through one solve
+// work fields for solves of ncomp components (synchronises when they grow; 1,
+// and what there was, if there is no memory); solve_batched: whether three
+// components may go through one solve
+size_t fastpc_bytes(const FastPC *f);    // device memory held
 int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s);
 bool solve_batched(const Geo &g, bool single);
 
