@@ -48,6 +48,41 @@ def _solver(tbl, grid, **kw):
     return tbl.Solver(*grid, i_rec=int(0.8 * (nX - 1)), planes=(2, 3, 4, 5, 6), **kw)
 
 
+# fields beyond the size up to which three components go through one solve
+# (6 N values above 256 MB), and below it
+@pytest.mark.parametrize("precision,grid", [("fp64", (900, 96, 64)), ("mixed", (1100, 100, 98)), ("fp64", GRID), ("mixed", GRID)])
+def test_direct_diffusion_solve(tbl, precision, grid):
+    """(I - hA) u = Q + boundary terms, three different components; memory beyond
+    the solver's own is taken for three components at once only"""
+    rng = np.random.default_rng(2)
+    h = 1e-4 / 150.92
+    N, es = int(np.prod(grid)), 4 if precision == "mixed" else 8
+    one = 6 * N * es > 256e6
+    with _solver(tbl, grid, precision=precision, helm_mode=tbl.TBL_HELM_DIRECT, precond=tbl.TBL_PC_FAST, kmax=1) as sv:
+        U, Q = sv.zeros(3), sv.zeros(3)
+        for a in (U, Q):
+            a[...] = rng.standard_normal(a.shape, dtype=np.float32)
+        sv.upload(U)
+        sv.set_field(tbl.F_Q, Q)
+        held = sv.device_bytes
+        sv.diffusion_solve()
+        assert sv.device_bytes - held == (0 if one else (3 + 4) * N * es)
+        u, m = sv.get_field(tbl.F_UT), sv.mesh()
+    dx, dy = m["x1"][1] - m["x1"][0], m["x2"][1] - m["x2"][0]
+    At, Ab, Ap = (m[q][1:-1] for q in ("At", "Ab", "Ap"))
+    c = u[I]
+    rows = np.arange(1, grid[1] - 1)
+    up, dn = np.where(rows == rows[-1], 1, rows + 1), np.where(rows == 1, rows[-1], rows - 1)
+    x = u[1:-1, :, 1:-1]
+    A = ((u[2:, 1:-1, 1:-1] + u[:-2, 1:-1, 1:-1]) / dx ** 2 + (x[:, up] + x[:, dn]) / dy ** 2
+         + At[:, None] * u[1:-1, 1:-1, 2:] + Ab[:, None] * u[1:-1, 1:-1, :-2] + Ap[:, None] * c)
+    r = Q[I] - (c - h * A)
+    # a solution rounded to the storage type: its rounding times the row sum of
+    # I - hA, at most 1 + 2 h max |Ap|; the FP64 solve refines once
+    eps = 1.2e-7 if precision == "mixed" else 2.3e-16
+    assert np.abs(r).max() <= 64 * eps * np.abs(u).max() * (1 + 2 * h * np.abs(Ap).max())
+
+
 def test_device_bytes_are_those_held(tbl):
     """what a context takes from the device, first solves included"""
     hip = C.CDLL("libamdhip64.so.7")             # the runtime that the library is linked to

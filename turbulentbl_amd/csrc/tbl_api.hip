@@ -267,6 +267,13 @@ template <class X> static int dalloc(tbl_ctx *c, X **ptr, size_t bytes)
     HIPCHK(c, alloc_clear(c, ptr, bytes));
     return 0;
 }
+// for memory that a slower route does without: 1 (and *ptr null) if there is none
+template <class X> static int try_alloc(tbl_ctx *c, X **ptr, size_t bytes)
+{
+    if (alloc_clear(c, ptr, bytes) == hipSuccess) return 0;
+    (void)hipGetLastError();                   // the next launch is not what failed
+    return 1;
+}
 
 // ------------------------------------------------------------------ static scratch
 // Scratch of tbl_div_check_noalloc: the block partials of the divergence sum,
@@ -1080,13 +1087,16 @@ extern "C" int tbl_momentum_rhs(tbl_ctx *c)
     return c->mixed ? rhs_impl<float>(c) : rhs_impl<double>(c);
 }
 
-// work of the direct and transposed solves, allocated by the first of them
-static int direct_work(tbl_ctx *c)
+// Components per launch of the direct and transposed solves.  Three (see
+// solve_batched) need a residual field and work fields of three components,
+// allocated by the first such solve; without the memory, and on larger grids,
+// the solves go one by one, with the work vector r (its faces are zero) for the
+// residual.
+static int direct_batch(tbl_ctx *c)
 {
-    if (!c->r3) CHK(dalloc(c, &c->r3, 3 * (size_t)c->g.N * c->es));
-    if (fastpc_reserve(c->fast, c->g, solve_batched(c->g, c->mixed) ? 3 : 1, c->s))
-        return fail(c, TBL_EARG, "fast solver: no memory for the solves of three components");
-    return 0;
+    if (!solve_batched(c->g, c->mixed)) return 1;
+    if (!c->r3 && try_alloc(c, &c->r3, 3 * (size_t)c->g.N * c->es)) return 1;
+    return fastpc_reserve(c->fast, c->g, 3, c->s) ? 1 : 3;
 }
 // exact Helmholtz solve of the three components: u += (I - hA)^{-1} (Q - H u), by fast
 // diagonalisation; in FP64 twice (one refinement step on the residual).  In
@@ -1098,9 +1108,8 @@ template <class T> static int helm_direct(tbl_ctx *c, int *sweeps, double *res)
     if (!c->fast) return fail(c, TBL_ESTATE, "direct Helmholtz solve without the fast solver");
     const Geo &g = c->g;
     const long N = g.N;
-    CHK(direct_work(c));
-    const int nc = solve_batched(g, c->mixed) ? 3 : 1;         // components per solve
-    T *r = F<T>(c->r3);
+    const int nc = direct_batch(c);            // components per solve
+    T *r = F<T>(nc == 3 ? c->r3 : c->r);
     const double h = c->p.dt / c->p.Re;
     const int passes = sizeof(T) == sizeof(double) ? 2 : 1;
     for (int p = 0; p < 3; p += nc) {
@@ -1961,9 +1970,8 @@ static int win_step(tbl_ctx *c, AdjWin &A, bool accJ)
 static int solve_T(tbl_ctx *c, const double *b, double *x, double alpha, double beta, int ncomp)
 {
     const Geo &g = c->g;
-    const int nc = solve_batched(g, c->mixed) ? ncomp : 1;
-    CHK(direct_work(c));
-    void *r = c->r3;
+    const int nc = ncomp == 3 ? direct_batch(c) : 1;
+    void *r = nc == 3 ? c->r3 : c->r;
     for (int p = 0; p < ncomp; p += nc) {
         const double *bp = b + (long)p * g.N;
         double *xp = x + (long)p * g.N;
