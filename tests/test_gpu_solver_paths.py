@@ -102,3 +102,22 @@ def test_device_bytes_are_those_held(tbl):
             taken = before - free()
             # each of some 45 allocations takes whole 2 MB pages
             assert 0.98 * sv.device_bytes <= taken <= sv.device_bytes + 100e6
+
+
+# long lines whose diagonal is close to twice the streamwise coupling.  The
+# residual that the FP64 solve leaves with every quotient of the cyclic reduction
+# rounded once (divided), measured, and three times that: products with a rounded
+# reciprocal leave 5 to 22 times as much on these three
+@pytest.mark.parametrize("nX,Lx,divided", [(100, 6.0, 7.2e-13), (2000, 3.0, 2.6e-9), (2050, 1.0, 1.4e-8)])
+def test_line_solve_rounding(tbl, nX, Lx, divided):
+    grid = (nX, 10, 20)
+    x = [np.sin(np.pi * np.arange(n) / (n - 1)) for n in grid]
+    with _solver(tbl, grid, precond=tbl.TBL_PC_FAST, kmax=1, Lx=Lx, Ly=4.0, Lz=3.4) as sv:
+        b = sv.zeros()
+        b[...] = x[0][:, None, None] * (1 + 0.3 * np.cos(2 * np.pi * np.arange(10) / 8))[None, :, None] * x[2][None, None, :]
+        b[I] *= 1 + 0.1 * np.random.default_rng(nX).standard_normal((nX - 2, 8, 18))
+        for q in range(3):
+            f = np.moveaxis(b, q, 0)
+            f[0] = f[-1] = 0.0
+        r = b - sv.apply_operator(0, sv.apply_operator(1, b))
+    assert np.linalg.norm(r[I]) <= 3 * divided * np.linalg.norm(b)
