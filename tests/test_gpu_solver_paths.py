@@ -1,5 +1,6 @@
 """Pressure and direct solves: the routes a solve takes when its first step is
 not enough, and the buffers it shares with the caller."""
+import contextlib
 import ctypes as C
 
 import numpy as np
@@ -41,6 +42,33 @@ def test_true_residual_solve_leaves_the_work_field(tbl):
         sv.set_field(tbl.F_WORK, w)
         _solve(tbl, sv, g, b, errtol=1e-10)
         assert np.array_equal(sv.get_field(tbl.F_WORK)[I], w[I])
+
+
+class _hip:
+    """the runtime that the library is linked to"""
+
+    def __init__(self):
+        self.lib = C.CDLL("libamdhip64.so.7")
+        self.lib.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+        self.lib.hipFree.argtypes = [C.c_void_p]
+
+    def free(self):
+        a, b = C.c_size_t(), C.c_size_t()
+        assert self.lib.hipDeviceSynchronize() == 0 and self.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    @contextlib.contextmanager
+    def left(self, nbytes):
+        """all but nbytes of the device's memory is taken"""
+        held = []
+        while self.free() - nbytes > 32e6 and len(held) < 8:      # a large allocation may come out smaller
+            held.append(C.c_void_p())
+            assert self.lib.hipMalloc(C.byref(held[-1]), int(self.free() - nbytes)) == 0
+        try:
+            yield
+        finally:
+            for p in held:
+                self.lib.hipFree(p)
 
 
 def _solver(tbl, grid, **kw):
@@ -85,13 +113,7 @@ def test_direct_diffusion_solve(tbl, precision, grid):
 
 def test_device_bytes_are_those_held(tbl):
     """what a context takes from the device, first solves included"""
-    hip = C.CDLL("libamdhip64.so.7")             # the runtime that the library is linked to
-
-    def free():
-        a, b = C.c_size_t(), C.c_size_t()
-        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
-        return a.value
-
+    free = _hip().free
     for grid, kw in (((900, 96, 64), dict(helm_mode=tbl.TBL_HELM_DIRECT)), ((256, 96, 64), dict(helm_mode=tbl.TBL_HELM_DIRECT)),
                      ((1024, 8, 130), dict(helm_mode=tbl.TBL_HELM_LEX_SLAB, precond=tbl.TBL_PC_SSOR_BLOCK, slabs=64))):
         before = free()
@@ -121,3 +143,28 @@ def test_line_solve_rounding(tbl, nX, Lx, divided):
             f[0] = f[-1] = 0.0
         r = b - sv.apply_operator(0, sv.apply_operator(1, b))
     assert np.linalg.norm(r[I]) <= 3 * divided * np.linalg.norm(b)
+
+
+def test_solve_without_memory_for_unit_steps(tbl):
+    """a solve by the reference's rule did without the second pressure
+    correction's 8 N bytes before unit steps, and does when they are not there"""
+    grid = (600, 250, 200)
+    N = int(np.prod(grid))
+    with _solver(tbl, grid, precond=tbl.TBL_PC_FAST, kmax=1, errtol=1e-6) as sv:
+        b = sv.zeros()
+        b[I] = np.random.default_rng(3).standard_normal([n - 2 for n in grid], dtype=np.float32)
+        sv.set_field(tbl.F_PRHS, b)
+        held = sv.device_bytes
+        with _hip().left(5 * N):
+            out = sv.ppe_solve(1e-6, 1, 20)
+        assert sv.device_bytes == held
+        x = sv.get_field(tbl.F_PCORR)
+        r = b - sv.apply_operator(0, x)
+        for q in range(3):
+            f = np.moveaxis(r, q, 0)
+            f[0] = f[-1] = 0.0
+        assert np.linalg.norm(sv.apply_operator(1, r)) <= 1e-6 * np.linalg.norm(sv.apply_operator(1, b))
+        assert abs(out["true_res"] - np.linalg.norm(r)) <= 1e-6 * np.linalg.norm(r) + 1e-13 * np.linalg.norm(b)
+        sv.set_field(tbl.F_PCORR, np.zeros_like(x, order="F"))
+        sv.ppe_solve(1e-6, 1, 20)
+        assert sv.device_bytes == held + 8 * N

@@ -1287,10 +1287,13 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
     if (kmax > c->p.kmax) return fail(c, TBL_EARG, "kmax above the allocated restart length");
     const int mode = (c->p.tol_mode == TBL_TOL_TRUE) ? GM_MODE_TRUE : GM_MODE_REF;
     const int poll = (N > 2000000 || c->p.precond == TBL_PC_FAST) ? 1 : 4;
-    // the second PCorr buffer of fused updates (TRUE) and unit steps
-    const bool unit_steps = c->p.precond == TBL_PC_FAST && sizeof(T) == sizeof(double);
-    const bool two = unit_steps || (mode == GM_MODE_TRUE && poll == 1);
-    if (two && !c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
+    // the second PCorr buffer of fused updates (TRUE) and of unit steps, which a
+    // solve by the reference's rule does without where there is no memory for it
+    const bool fused = mode == GM_MODE_TRUE && poll == 1;
+    bool unit_steps = c->p.precond == TBL_PC_FAST && sizeof(T) == sizeof(double);
+    if (fused && !c->PCalt) CHK(dalloc(c, &c->PCalt, (size_t)N * sizeof(double)));
+    if (unit_steps && !c->PCalt && try_alloc(c, &c->PCalt, (size_t)N * sizeof(double))) unit_steps = false;
+    const bool two = fused || unit_steps;
     launch_gm_init(g, c->gm, errtol, c->p.inner_tol, kmax, mmax, mode, c->PCorr, two ? c->PCalt : nullptr, c->s);
     double *part_r = c->part;                  // residual partials
     double *part_z = c->part + nbr + 8;        // norm partials (and dot partials)
