@@ -168,3 +168,16 @@ def test_solve_without_memory_for_unit_steps(tbl):
         sv.set_field(tbl.F_PCORR, np.zeros_like(x, order="F"))
         sv.ppe_solve(1e-6, 1, 20)
         assert sv.device_bytes == held + 8 * N
+
+
+@pytest.mark.parametrize("rule", ["ref", "true"])
+def test_timers_see_an_accepted_unit_step(tbl, rule):
+    """two residual passes and two applications by the reference's rule (of M^-1 b
+    and of what the step left), one application where the true residual is asked for"""
+    g, s = make_case(GRID, seed=4)
+    with gpu_from_case(g, s, precond=tbl.TBL_PC_FAST, tol_mode=int(rule == "true"), inner_tol=1e-6) as sv:
+        sv.timer_enable(["resid", "precond"])
+        out, _ = _solve(tbl, sv, g, _rhs(g), errtol=1e-5)
+        n = {q: v["count"] for q, v in sv.timer_read().items()}
+    assert out["iters"] == 1
+    assert n == dict(resid=2, precond=2 if rule == "ref" else 1)

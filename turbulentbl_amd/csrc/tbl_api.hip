@@ -1507,8 +1507,14 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         if (m == 0 && unit_steps) {
             // unit step (k_fin_unit): the preconditioned residual of PCorr + V_0
             // (into W; r holds the residual) ends the solve, or is dropped
-            launch_resid_upd<T>(g, c->pRhs, c->PCorr, V, c->gm, c->PCalt, r, part_r, c->s, RU_UNIT);
-            launch_precond<T>(g, c->p.precond, c->fast, r, scr, W, act, c->s);
+            {
+                Tscope ts(c, TBL_K_RESID, (double)N * (24.0 + 2.0 * sizeof(T)));
+                launch_resid_upd<T>(g, c->pRhs, c->PCorr, V, c->gm, c->PCalt, r, part_r, c->s, RU_UNIT);
+            }
+            {
+                Tscope ts(c, TBL_K_PRECOND, precond_bytes(c, sizeof(T)));
+                launch_precond<T>(g, c->p.precond, c->fast, r, scr, W, act, c->s);
+            }
             launch_norm2<T>(W, N, part_z, act, c->s);
             launch_fin_unit(c->gm, part_r, (int)nbr, part_z, (int)nbv, pub_of(c, c->gm_h), c->s);
             HIPCHK(c, hipGetLastError());
