@@ -181,3 +181,16 @@ def test_timers_see_an_accepted_unit_step(tbl, rule):
         n = {q: v["count"] for q, v in sv.timer_read().items()}
     assert out["iters"] == 1
     assert n == dict(resid=2, precond=2 if rule == "ref" else 1)
+
+
+# the usual tolerance, and one that no solve's accuracy meets
+@pytest.mark.parametrize("errtol", [1e-5, 1e-16])
+def test_no_step_is_tried_that_cannot_be_accepted(tbl, errtol):
+    """reference's rule: one application at each cycle's start and one for each
+    step, an accepted unit step among them"""
+    g, s = make_case((64, 32, 48), seed=4)
+    with gpu_from_case(g, s, precond=tbl.TBL_PC_FAST) as sv:
+        sv.timer_enable(["precond"])
+        out, _ = _solve(tbl, sv, g, _rhs(g), errtol=errtol, kmax=5, mmax=3)
+        n = sv.timer_read()["precond"]["count"]
+    assert n == out["cycles"] + out["iters"]

@@ -44,6 +44,7 @@ struct FastPC {
     void *t1 = nullptr, *t2 = nullptr;                   // work fields (storage type), ncap components each
     int ncap = 1;
     size_t bytes = 0;                                    // device memory held
+    double reach = 0.0;                                  // see fastpc_reach
     bool single = false;
     // FP32 storage: the transform matrices split into three bf16 parts in
     // matrix-core fragment order (see k_xform): z forward, y forward, y
@@ -597,6 +598,13 @@ int fastpc_create(const Geo &g, const double *Ab, const double *At, const double
     }
     for (int q = 0; q < nz; q++) T[(size_t)q * nz + q] = Ap[q + 1] + 2.0 * g.Aw + 2.0 * g.An;
     jacobi_eig(nz, T, Q);
+    // what one solve leaves (fastpc_reach): the eigensolver ends on the norm of the
+    // whole matrix, and what it left beside the diagonal couples the modes of the
+    // smallest eigenvalues
+    for (int p = 0; p < nz; p++)
+        for (int q = 0; q < nz; q++)
+            if (p != q) f->reach = std::max(f->reach, fabs(T[(size_t)p * nz + q] / T[(size_t)p * nz + p]));
+    f->reach = std::max(0.03 * f->reach, 2e-14);
     // forward Wf(k,q) = Q(k,q)/s_k ; inverse Wi(q,k) = s_k Q(k,q)  (column-major nz x nz)
     std::vector<double> Wf((size_t)nz * nz), Wi((size_t)nz * nz), lz(g.nZ, 0.0);
     for (int q = 0; q < nz; q++) {
@@ -859,6 +867,7 @@ static void launch_line_solve(const Geo &g, T *d, const double *ly, const double
 bool solve_batched(const Geo &g, bool single) { return 6.0 * (double)g.N * (single ? 4 : 8) <= 256e6; }
 
 size_t fastpc_bytes(const FastPC *f) { return f->bytes; }
+double fastpc_reach(const FastPC *f) { return f->reach; }
 
 int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s)
 {

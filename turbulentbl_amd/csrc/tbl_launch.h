@@ -91,6 +91,8 @@ int run_fast_solve(const FastPC *f, const Geo &g, const FastIO &io, const int *a
 // and what there was, if there is no memory); solve_batched: whether three
 // components may go through one solve
 size_t fastpc_bytes(const FastPC *f);    // device memory held
+// about what |M^-1 r| / |M^-1 b| is after one FP64 solve of A x = b (the same for any b)
+double fastpc_reach(const FastPC *f);
 int fastpc_reserve(FastPC *f, const Geo &g, int ncomp, hipStream_t s);
 bool solve_batched(const Geo &g, bool single);
 
