@@ -1332,10 +1332,16 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
         // behind that step's status read-back, gated on the cycle having ended
         // (off while the residual class is timed)
         const bool ahead_res = fuse_upd && !(c->tmask & (1u << TBL_K_RESID));
-        // the first Arnoldi step is the last of its cycle with the fast
-        // preconditioner: its vector is only measured, and formed when the
-        // status asks for a second step (1024x256x192 mixed 98 -> 77 us)
-        const bool norm_only = c->p.precond == TBL_PC_FAST && kmax > 1 && poll == 1;
+        // With the fast preconditioner the first Arnoldi step is the last of its
+        // cycle if the cycle asks for no more than one solve gives: its vector is
+        // then only measured, and formed when the status asks for a second step
+        // after all (1024x256x192 mixed 98 -> 77 us).  One FP32 solve gives 1e-4 to
+        // 1e-5 on the larger grids (with an inner_tol of 1e-5 and the vector formed
+        // after its norm, a solve of 1024x256x192 took 5.83 instead of 5.70 ms); in
+        // FP64 a unit step was refused if the Arnoldi steps run before the last cycle.
+        auto norm_only = [&](bool unit) {
+            return c->p.precond == TBL_PC_FAST && kmax > 1 && (unit_steps ? unit : c->p.inner_tol >= 3e-5);
+        };
         bool pend = false;
         bool queued = false;                   // the cycle's residual pass ran behind the last read-back
         // unit steps (k_fin_unit) while they are accepted, in FP64: the fast
@@ -1421,6 +1427,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                 opened = false;
             }
             bool one_step = false;             // the cycle stopped after its first Arnoldi step
+            const bool measure = norm_only(unit);
             for (int j = 0; j < kmax; j++) {
                 T *vj = V + (long)j * ldv, *vj1 = V + (long)(j + 1) * ldv, *zj = Z + (long)j * ldv;
                 if (!(j == 0 && have_z0)) {
@@ -1449,8 +1456,8 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                     launch_fin_dots(c->gm, part_z, (int)nbv, j, c->s);
                 }
                 {
-                    Tscope ts(c, TBL_K_UPDATE, (j + (norm_only && j == 0 ? 2.0 : 3.0)) * (double)N * sizeof(T));
-                    launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s, !(norm_only && j == 0));
+                    Tscope ts(c, TBL_K_UPDATE, (j + (measure && j == 0 ? 2.0 : 3.0)) * (double)N * sizeof(T));
+                    launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s, !(measure && j == 0));
                 }
                 launch_fin_update(c->gm, part_z, (int)nbv, j, c->s);
                 HIPCHK(c, hipGetLastError());
@@ -1471,7 +1478,10 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
                         }
                         break;
                     }
-                    if (norm_only && j == 0) launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s);
+                    if (measure && j == 0) {
+                        Tscope ts(c, TBL_K_UPDATE, 3.0 * (double)N * sizeof(T));
+                        launch_update<T>(V, ldv, j, N, c->gm, part_z, c->s);
+                    }
                 }
             }
             if (!queued) {                     // (queued: fin_cycle and PCorr += y z0 have run)
