@@ -194,3 +194,24 @@ def test_no_step_is_tried_that_cannot_be_accepted(tbl, errtol):
         out, _ = _solve(tbl, sv, g, _rhs(g), errtol=errtol, kmax=5, mmax=3)
         n = sv.timer_read()["precond"]["count"]
     assert n == out["cycles"] + out["iters"]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_transfers_of_page_locked_arrays(tbl, precision):
+    """a size that goes through the ring from pageable memory"""
+    grid = (128, 128, 66)
+    n, hip = 3 * int(np.prod(grid)), _hip()
+    p = C.c_void_p()
+    hip.lib.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    hip.lib.hipHostFree.argtypes = [C.c_void_p]
+    with _solver(tbl, grid, precision=precision, kmax=1) as sv:
+        assert hip.lib.hipHostMalloc(C.byref(p), 8 * n, 0) == 0
+        a = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), (n,))
+        x = np.random.default_rng(8).standard_normal(n)
+        a[:] = x
+        sv._chk(sv.lib.tbl_field_set(sv.h, tbl.F_UT, p))
+        a[:] = 0.0
+        sv._chk(sv.lib.tbl_field_get(sv.h, tbl.F_UT, p))
+        assert np.array_equal(a, x if precision == "fp64" else x.astype(np.float32))
+        hip.lib.hipHostFree(p)
+        assert np.array_equal(sv.get_field(tbl.F_UT).ravel(order="F"), x if precision == "fp64" else x.astype(np.float32))

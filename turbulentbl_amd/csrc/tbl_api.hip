@@ -18,7 +18,9 @@
 #include <atomic>
 #include <chrono>
 #include <exception>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <utility>
@@ -608,24 +610,31 @@ static void *field_ptr(tbl_ctx *c, int f, bool *is_double)
     return nullptr;
 }
 
-// Host transfers of fields.  Host arrays are FP64 and pageable; mixed
+// Host transfers of fields.  Host arrays are FP64 and mostly pageable; mixed
 // contexts hold FP32.  A pageable copy runs at 18 GB/s from the device (31 to
 // it), and converting and filling an array of untouched pages on one thread
 // cost more than that: reading the velocity and pressure of 1024x256x192
 // mixed took 300 ms, 60 steps' worth.  The field goes through a ring of pinned
 // chunks instead: the copy engine fills (drains) them at 57 GB/s while a few
 // threads convert and copy between the chunks and the host array.  The ring
-// belongs to the context (XF_SLOTS chunks, allocated by the first transfer).
-// Up / down, before -> after: 1024x256x192 mixed velocity 167 / 213 -> 19 / 23
-// ms, 512x128x128 FP64 6.9 / 19.4 -> 5.1 / 5.9 ms; 4 to 16 threads differ by
-// 10 %, 2 take half as long again from the device, chunks of 64 k values twice
-// as long.  Four threads that sleep while they wait: eight that yielded ran a
-// process whose other threads were busy into its CPU quota (16 cores), and an
-// upload of 18 M values that takes 4 ms took 38.  FP64 fields that a pageable
-// copy moves sooner take it (move_field): up to 3 M values to the device
-// (128x80x80 velocity: 0.56 against 0.66 ms) and half a million from it.
+// belongs to the context (XF_SLOTS chunks, allocated by the first transfer that
+// takes it).  Up / down, before -> after: 1024x256x192 mixed velocity 167 / 213 ->
+// 19 / 23 ms, 512x128x128 FP64 6.9 / 19.4 -> 5.1 / 5.9 ms; 4 to 16 threads differ
+// by 10 %, 2 take half as long again from the device, chunks of 64 k values twice
+// as long.  Four threads, which sleep while they wait for each other: eight that
+// yielded ran a process whose other threads were busy into its CPU quota (16
+// cores), and an upload of 18 M values that takes 4 ms took 38.
+//
+// A plain copy (move_plain) is the sooner one, and is taken,
+//  * from and to page-locked memory in FP64, which the copy engine reads and
+//    writes itself: 512x128x128 velocity 3.5 ms, through the ring 5.1;
+//  * below the sizes XF_*: FP64 to the device 3 M values (128x80x80 velocity 0.56
+//    against 0.66 ms), from it half a million;
+//  * where there is no pinned memory for the ring.
 #define XF_SLOTS 8
 #define XF_CHUNK ((size_t)1 << 18)       // elements per chunk: 2 MB of doubles
+#define XF_D_UP (12 * XF_CHUNK)          // least elements through the ring
+#define XF_D_DOWN (2 * XF_CHUNK)
 #define XF_THREADS 4
 #define XF_NAP std::this_thread::sleep_for(std::chrono::microseconds(10))
 struct XferRing {
@@ -641,21 +650,22 @@ static void ring_free(tbl_ctx *c)
     delete c->ring;
     c->ring = nullptr;
 }
+// 1 if there is no memory for it
 static int ring_get(tbl_ctx *c)
 {
     if (c->ring) return 0;
-    c->ring = new XferRing();
+    c->ring = new (std::nothrow) XferRing();
+    if (!c->ring) return 1;
     const size_t slot = XF_CHUNK * sizeof(double);
     hipError_t e = hipHostMalloc((void **)&c->ring->mem, XF_SLOTS * slot, hipHostMallocDefault);
     for (int q = 0; q < XF_SLOTS && e == hipSuccess; q++) {
         c->ring->buf[q] = c->ring->mem + q * slot;
         e = hipEventCreateWithFlags(&c->ring->ev[q], hipEventDisableTiming);
     }
-    if (e != hipSuccess) {
-        ring_free(c);
-        HIPCHK(c, e);
-    }
-    return 0;
+    if (e == hipSuccess) return 0;
+    (void)hipGetLastError();
+    ring_free(c);
+    return 1;
 }
 // chunk q of the host array to or from its slot
 static void chunk_convert(char *slot, bool dbl, double *host, size_t m, bool to_dev)
@@ -666,20 +676,42 @@ static void chunk_convert(char *slot, bool dbl, double *host, size_t m, bool to_
     else if (to_dev) for (size_t e = 0; e < m; e++) f[e] = (float)host[e];
     else for (size_t e = 0; e < m; e++) host[e] = f[e];
 }
+// the same without the ring
+static int move_plain(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, bool to_dev)
+{
+    std::unique_ptr<float[]> tmp(dbl ? nullptr : new (std::nothrow) float[n]);
+    if (!dbl && !tmp) return fail(c, TBL_EARG, "no host memory for a field's conversion");
+    if (!dbl && to_dev)
+        for (size_t e = 0; e < n; e++) tmp[e] = (float)host[e];
+    void *h = dbl ? (void *)host : (void *)tmp.get();
+    const size_t b = n * (dbl ? sizeof(double) : sizeof(float));
+    HIPCHK(c, to_dev ? hipMemcpyAsync(dev, h, b, hipMemcpyHostToDevice, c->s)
+                     : hipMemcpyAsync(h, dev, b, hipMemcpyDeviceToHost, c->s));
+    HIPCHK(c, hipStreamSynchronize(c->s));
+    if (!dbl && !to_dev)
+        for (size_t e = 0; e < n; e++) host[e] = tmp[e];
+    return 0;
+}
+// page-locked host memory, which the copy engine reads and writes itself
+static bool is_pinned(const void *p)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeHost;
+    (void)hipGetLastError();                   // memory that the runtime does not know
+    return false;
+}
 // n elements between dev (double or float) and host, in stream order; returns
 // when they have arrived
 static int move_field(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, bool to_dev)
 {
-    if (dbl && n < (to_dev ? 12 : 2) * XF_CHUNK) {
-        HIPCHK(c, to_dev ? hipMemcpyAsync(dev, host, n * sizeof(double), hipMemcpyHostToDevice, c->s)
-                         : hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c->s));
-        HIPCHK(c, hipStreamSynchronize(c->s));
-        return 0;
-    }
-    CHK(ring_get(c));
+    const size_t least = dbl ? (to_dev ? XF_D_UP : XF_D_DOWN) : 0;
+    const long nch = (long)((n + XF_CHUNK - 1) / XF_CHUNK);
+    std::unique_ptr<std::atomic<char>[]> done;                  // chunk q is converted
+    if (n >= least && !(dbl && is_pinned(host)) && !ring_get(c)) done.reset(new (std::nothrow) std::atomic<char>[nch]);
+    if (!done) return move_plain(c, dev, dbl, host, n, to_dev);
+    for (long q = 0; q < nch; q++) done[q].store(0, std::memory_order_relaxed);
     XferRing &R = *c->ring;
     const size_t es = dbl ? sizeof(double) : sizeof(float);
-    const long nch = (long)((n + XF_CHUNK - 1) / XF_CHUNK);
     auto len = [&](long q) { return std::min(XF_CHUNK, n - (size_t)q * XF_CHUNK); };
     auto copy = [&](long q) -> hipError_t {                     // chunk q between its slot and the device
         char *d = (char *)dev + (size_t)q * XF_CHUNK * es, *h = R.buf[q % XF_SLOTS];
@@ -692,8 +724,6 @@ static int move_field(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, b
     // done[q] follows
     std::atomic<long> next{0}, ready{to_dev ? std::min(nch, (long)XF_SLOTS) : 0};
     std::atomic<int> err{0};
-    std::vector<std::atomic<char>> done(nch);
-    for (auto &d : done) d.store(0, std::memory_order_relaxed);
     auto convert = [&](long q) {
         if (!to_dev) {
             const hipError_t e = hipEventSynchronize(R.ev[q % XF_SLOTS]);
