@@ -196,6 +196,16 @@ def test_no_step_is_tried_that_cannot_be_accepted(tbl, errtol):
     assert n == out["cycles"] + out["iters"]
 
 
+# FP32 fields on both sides of the sizes from which a transfer goes through the
+# pinned ring (393216 values from the device, 1310720 to it)
+@pytest.mark.parametrize("grid", [(64, 64, 94), (64, 64, 96), (128, 128, 78), (128, 128, 80)])
+def test_converted_transfers(tbl, grid):
+    with _solver(tbl, grid, precision="mixed", kmax=1) as sv:
+        x = np.asfortranarray(np.random.default_rng(7).standard_normal(grid))
+        sv.set_field(tbl.F_PRESS, x)
+        assert np.array_equal(sv.get_field(tbl.F_PRESS), x.astype(np.float32))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_transfers_of_page_locked_arrays(tbl, precision):
     """a size that goes through the ring from pageable memory"""

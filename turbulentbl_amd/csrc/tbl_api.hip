@@ -623,18 +623,25 @@ static void *field_ptr(tbl_ctx *c, int f, bool *is_double)
 // by 10 %, 2 take half as long again from the device, chunks of 64 k values twice
 // as long.  Four threads, which sleep while they wait for each other: eight that
 // yielded ran a process whose other threads were busy into its CPU quota (16
-// cores), and an upload of 18 M values that takes 4 ms took 38.
+// cores), and an upload of 18 M values that takes 4 ms took 38.  The waits for the
+// copy engine spin (a download of 25 M values takes 5.1 ms and 20 ms of CPU):
+// asking and sleeping in turn halves the CPU time and changes nothing on an idle
+// host, but beside 16 busy threads that download takes 14 instead of 10 ms.
 //
 // A plain copy (move_plain) is the sooner one, and is taken,
 //  * from and to page-locked memory in FP64, which the copy engine reads and
 //    writes itself: 512x128x128 velocity 3.5 ms, through the ring 5.1;
 //  * below the sizes XF_*: FP64 to the device 3 M values (128x80x80 velocity 0.56
-//    against 0.66 ms), from it half a million;
+//    against 0.66 ms), from it half a million; FP32, converted by the caller's
+//    thread, 1.3 M (1.1 M values 0.23 against 0.25 ms, 1.5 M 0.34 against 0.30) and
+//    0.4 M (0.29 M values 0.12 against 0.15, 0.5 M 0.18 against 0.15);
 //  * where there is no pinned memory for the ring.
 #define XF_SLOTS 8
 #define XF_CHUNK ((size_t)1 << 18)       // elements per chunk: 2 MB of doubles
 #define XF_D_UP (12 * XF_CHUNK)          // least elements through the ring
 #define XF_D_DOWN (2 * XF_CHUNK)
+#define XF_F_UP (5 * XF_CHUNK)
+#define XF_F_DOWN (3 * XF_CHUNK / 2)
 #define XF_THREADS 4
 #define XF_NAP std::this_thread::sleep_for(std::chrono::microseconds(10))
 struct XferRing {
@@ -704,7 +711,7 @@ static bool is_pinned(const void *p)
 // when they have arrived
 static int move_field(tbl_ctx *c, void *dev, bool dbl, double *host, size_t n, bool to_dev)
 {
-    const size_t least = dbl ? (to_dev ? XF_D_UP : XF_D_DOWN) : 0;
+    const size_t least = dbl ? (to_dev ? XF_D_UP : XF_D_DOWN) : (to_dev ? XF_F_UP : XF_F_DOWN);
     const long nch = (long)((n + XF_CHUNK - 1) / XF_CHUNK);
     std::unique_ptr<std::atomic<char>[]> done;                  // chunk q is converted
     if (n >= least && !(dbl && is_pinned(host)) && !ring_get(c)) done.reset(new (std::nothrow) std::atomic<char>[nch]);
