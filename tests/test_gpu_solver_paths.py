@@ -225,3 +225,30 @@ def test_transfers_of_page_locked_arrays(tbl, precision):
         assert np.array_equal(a, x if precision == "fp64" else x.astype(np.float32))
         hip.lib.hipHostFree(p)
         assert np.array_equal(sv.get_field(tbl.F_UT).ravel(order="F"), x if precision == "fp64" else x.astype(np.float32))
+
+
+def test_window_without_memory_for_the_adjoint_fields(tbl):
+    """the forward sweep needs the snapshots only: J is there when the call fails"""
+    grid = (900, 96, 64)
+    N = int(np.prod(grid))
+    rng = np.random.default_rng(9)
+    with _solver(tbl, grid, kmax=1) as sv:
+        U = sv.zeros(3)
+        U[..., 0] = 19.8 * np.tanh(4.0 * sv.mesh()["x3"])
+        U[I] += 0.02 * rng.standard_normal(U[I].shape, dtype=np.float32)
+
+        def window(forward_only):
+            sv.upload(U, sv.zeros(), sv.zeros())
+            sv.set_state()
+            o, J = tbl.AdjointOpts(2, 1, 500, 800, forward_only, 0), C.c_double(-1.0)
+            grad = np.zeros(grid[:2], order="F")
+            rc = sv.lib.tbl_adjoint_window(sv.h, C.byref(o), None, C.byref(J), None if forward_only else grad.ctypes.data,
+                                           None, None)
+            return rc, J.value
+
+        rc, J = window(1)
+        assert rc == 0 and J > 0.0
+        # three snapshots of 40 bytes a cell; the adjoint fields take 72
+        with _hip().left((3 * 40 + 36) * N):
+            rc, Jg = window(0)
+        assert rc != 0 and Jg == J

@@ -1902,13 +1902,13 @@ extern "C" int tbl_step(tbl_ctx *c, int nsteps, tbl_diag *diag)
 }
 
 // ------------------------------------------------------------------ discrete adjoint
-// Work buffers of one adjoint window: one allocation per call (mem: the
-// adjoint fields, cleared, then the snapshots, which are stored before they are
-// read).  A forward evaluation needs none.  An allocation and a clear for each
-// of ten buffers, the snapshots' included, and the start state stored for a
-// forward evaluation too, took 0.1 of the 1.25 ms of a forward call at 64x32x48,
-// 1.3 of the 35.4 ms of a gradient at 256x64x96 and 2.1 of the 69.0 ms at
-// 1024x192x160 mixed.
+// Work buffers of one adjoint window, two allocations a call: the snapshots,
+// which are stored before they are read, then the adjoint fields, cleared, once
+// the forward sweep has given J.  A forward evaluation needs none.  An
+// allocation and a clear for each of ten buffers, the snapshots' included, and
+// the start state stored for a forward evaluation too, took 0.1 of the 1.25 ms
+// of a forward call at 64x32x48, 1.3 of the 35.4 ms of a gradient at 256x64x96
+// and 2.1 of the 69.0 ms at 1024x192x160 mixed.
 struct AdjWin {
     char *mem = nullptr;
     double *lamU = nullptr, *lamP = nullptr, *lamQ = nullptr, *lamPhi = nullptr, *lamB = nullptr;
@@ -1934,11 +1934,10 @@ static int adj_alloc(tbl_ctx *c, AdjWin &A)
     auto up = [](size_t n) { return (n + 31) & ~(size_t)31; };   // 256 bytes
     size_t fields = 0;
     for (auto &f : sub) fields += up(f.n);
-    HIPCHK(c, hipMalloc((void **)&A.mem, fields * 8 + (size_t)A.nslots * A.slot_bytes));
+    HIPCHK(c, hipMalloc((void **)&A.mem, fields * 8));
     HIPCHK(c, hipMemsetAsync(A.mem, 0, fields * 8, c->s));
     double *q = (double *)A.mem;
     for (auto &f : sub) { *f.p = q; q += up(f.n); }
-    A.snapbuf = (char *)q;
     return 0;
 }
 // snapshot = Ut (3N), Press (N) in the storage type, PCorr (N, double) and
@@ -2207,7 +2206,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         HIPCHK(c, hipMemsetAsync(A.Jd, 0, 8, c->s));
         A.slot_bytes = (4 * N * c->es + N * 8 + 255) & ~(size_t)255;
         if (!o->forward_only) {
-            CHK(adj_alloc(c, A));
+            HIPCHK(c, hipMalloc((void **)&A.snapbuf, (size_t)A.nslots * A.slot_bytes));
             CHK(snap_store(c, A, 0));
         }
         std::vector<int> at;
@@ -2223,6 +2222,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         if (o->forward_only) return 0;
         const int fin = A.nslots - 1;
         CHK(snap_store(c, A, fin));
+        CHK(adj_alloc(c, A));
         if (c->mixed) launch_adj_save_end<float>(c->g, F<float>(c->Ut), A.E, c->s);
         else launch_adj_save_end<double>(c->g, F<double>(c->Ut), A.E, c->s);
         launch_adj_tau(c->g, A.lamU, A.i0, A.i1, A.cJ, c->s);
@@ -2237,6 +2237,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
     if (nadj) *nadj = A.nadj;
     hipStreamSynchronize(c->s);
     if (A.mem) hipFree(A.mem);
+    if (A.snapbuf) hipFree(A.snapbuf);
     return rc;
 }
 
