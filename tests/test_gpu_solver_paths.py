@@ -252,3 +252,4 @@ def test_window_without_memory_for_the_adjoint_fields(tbl):
         with _hip().left((3 * 40 + 36) * N):
             rc, Jg = window(0)
         assert rc != 0 and Jg == J
+        assert window(0) == (0, J)               # and the next call is not taken for failed

@@ -112,11 +112,13 @@ struct HostPub {
     double gs[16], dd[DD_NCOUNT];
 };
 
+// (a failed call's error is cleared: it would be taken for that of the next launch)
 #define HIPCHK(ctx, call)                                                                    \
     do {                                                                                     \
         hipError_t e_ = (call);                                                              \
         if (e_ != hipSuccess) {                                                              \
             (ctx)->err = std::string(#call) + ": " + hipGetErrorString(e_);                  \
+            (void)hipGetLastError();                                                         \
             return (int)e_;                                                                  \
         }                                                                                    \
     } while (0)
