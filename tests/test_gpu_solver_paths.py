@@ -6,6 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+from oracle import orc
 from tests.case_util import gpu_from_case, make_case
 
 pytestmark = pytest.mark.gpu
@@ -253,3 +254,34 @@ def test_window_without_memory_for_the_adjoint_fields(tbl):
             rc, Jg = window(0)
         assert rc != 0 and Jg == J
         assert window(0) == (0, J)               # and the next call is not taken for failed
+
+
+# thin slabs, whose sweeps' copy is larger than the rest of the context: with that
+# much memory gone the context is made all the same and sweeps in place
+@pytest.mark.parametrize("grid,P,precision,leave", [((1024, 8, 130), 43, "fp64", 0.6), ((1024, 8, 130), 43, "mixed", 0.6),
+                                                    ((512, 130, 60), 20, "fp64", 0.87)])
+def test_slab_sweeps_without_memory_for_their_copy(tbl, grid, P, precision, leave):
+    g, s = make_case(grid, seed=2, P=P)
+    _, Q = g.momentum_rhs(s.Ut, s.Press)
+    x = g.zeros()
+    x[I] = np.random.default_rng(5).standard_normal([n - 2 for n in grid])
+    kw = dict(precision=precision, helm_mode=tbl.TBL_HELM_LEX_SLAB, precond=tbl.TBL_PC_SSOR_BLOCK, slabs=P, kmax=2)
+    got, held = [], []
+
+    def sweeps(sv):
+        sv.set_field(tbl.F_Q, Q)
+        y = sv.apply_operator(1, x)
+        sw, _ = sv.diffusion_solve(1e-30, 2)
+        got.append((sv.get_field(tbl.F_UT), y, list(sw)))
+        held.append(sv.device_bytes)
+
+    with gpu_from_case(g, s, **kw) as sv:
+        sweeps(sv)
+    with _hip().left(leave * held[0]), gpu_from_case(g, s, **kw) as sv:
+        sweeps(sv)
+    assert held[1] < 0.9 * held[0]
+    assert got[1][2] == got[0][2] and np.array_equal(got[1][0], got[0][0]) and np.array_equal(got[1][1], got[0][1])
+    if precision == "fp64":
+        Uo = s.Ut.copy(order="F")
+        g.diffusion_solve(Q, Uo, order=orc.GS_LEX_BLOCK, errorstop=1e-30, mmax=2)
+        assert np.array_equal(got[1][0], Uo) and np.array_equal(got[1][1][I], g.precond_apply(x, orc.PC_SSOR_BLOCK)[I])

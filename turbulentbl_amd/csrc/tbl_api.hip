@@ -334,10 +334,10 @@ static int create_impl(tbl_ctx *c)
     CHK(dalloc(c, &c->r, N * c->es));
     if (p.tol_mode == TBL_TOL_TRUE) CHK(dalloc(c, &c->Z, (size_t)p.kmax * c->ldv * c->es));
     if (p.helm_mode == TBL_HELM_ZEBRA) CHK(dalloc(c, &c->Ualt, 3 * N * c->es));
-    c->g.nslab = 0; c->g.nkmax = 0; c->g.slab = nullptr;
+    c->g.nslab = 0; c->g.nkmax = 0; c->g.skew = 0; c->g.slab = nullptr;
     c->g.rblk = c->mixed ? 8192 : 2048;
     c->g.rpl = c->mixed ? p.nZ : 12;
-    size_t nscr = N;
+    size_t nscr = N, ncopy = 0;                // of scr; with the slab sweeps' copy in it
     if (p.helm_mode == TBL_HELM_LEX_SLAB || p.precond == TBL_PC_SSOR_BLOCK) {
         // the reference's slab bounds (dnssetbl.f90:76-92): nZ/P planes per
         // rank, the remainder to the high ranks; the first and last rank
@@ -368,9 +368,10 @@ static int create_impl(tbl_ctx *c)
         CHK(dalloc(c, &c->slab, sizeof(int) * 2 * P));
         HIPCHK(c, hipMemcpyAsync(c->slab, sl.data(), sizeof(int) * 2 * P, hipMemcpyHostToDevice, c->s));
         c->g.slab = c->slab;
-        nscr = std::max((size_t)N, slab_scratch(c->g, p.helm_mode == TBL_HELM_LEX_SLAB));
+        const bool lex = p.helm_mode == TBL_HELM_LEX_SLAB;
+        if (slab_copy_pays(c->g)) ncopy = std::max(nscr, slab_scratch(c->g, lex));
+        nscr = std::max(nscr, slab_scratch_inplace(c->g, lex));
     }
-    CHK(dalloc(c, &c->scr, nscr * c->es));
     if (p.helm_mode == TBL_HELM_ZLINE_RB || p.helm_mode == TBL_HELM_ZEBRA) {
         // elimination factors of the partitioned wall-normal line solve (the
         // line matrix a = -h Ab, b = 1 - h Ap, c = -h At is the same for every
@@ -491,6 +492,9 @@ static int create_impl(tbl_ctx *c)
     std::vector<int> nk(p.nZ);
     for (int k = 0; k < p.nZ; k++) nk[k] = (k < p.nZ - 1) ? k + 1 : p.nZ - 1;
     HIPCHK(c, hipMemcpyAsync(c->newk, nk.data(), sizeof(int) * p.nZ, hipMemcpyHostToDevice, c->s));
+    // last, so that the copy takes nothing that the context cannot do without
+    c->g.skew = ncopy && !try_alloc(c, &c->scr, ncopy * c->es);
+    if (!c->scr) CHK(dalloc(c, &c->scr, nscr * c->es));
     HIPCHK(c, hipStreamSynchronize(c->s));
     return 0;
 }

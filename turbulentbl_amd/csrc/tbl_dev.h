@@ -26,8 +26,9 @@ struct Geo {
     int scheme;              // TBL_SCHEME_*
     double forc[3];          // body force (TBL_SCHEME_DNSTBL)
     // wall-normal slabs of the reference's decomposition (per-slab orderings):
-    // count, thickest slab in planes, 0-based first/last interior plane pairs
-    int nslab, nkmax;
+    // count, thickest slab in planes, whether the sweeps work on a skewed copy,
+    // 0-based first/last interior plane pairs
+    int nslab, nkmax, skew;
     const int *slab;
     int rblk, rpl;           // reduction kernels: blocks aimed at, most planes per block (rtiles_of)
 };

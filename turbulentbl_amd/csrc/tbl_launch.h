@@ -35,6 +35,8 @@ template <class T> void launch_copy_faces3(const Geo &g, const T *src, T *dst, v
 // (lex) or the block SSOR needs
 template <class T> void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *scr, const void *ctrl, hipStream_t s);
 size_t slab_scratch(const Geo &g, bool lex);
+bool slab_copy_pays(const Geo &g);
+size_t slab_scratch_inplace(const Geo &g, bool lex);     // ... without the skewed copy (g.skew 0)
 int slab_threads(const Geo &g, int nkmax);
 size_t gs_ctrl_bytes();
 void gs_ctrl_read(const void *host, int *active, int *sweeps, double *res);

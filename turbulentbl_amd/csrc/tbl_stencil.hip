@@ -2254,6 +2254,91 @@ __global__ __launch_bounds__(MT) void k_ssor_block(Geo g, Skew sk, T *S, const i
     ring_tail<0, NS>(bwd, t, steps);
 }
 
+// ----------------------------------------------------------------------------
+// The same sweeps on the fields themselves: the same wavefront and the same values,
+// each neighbour read from memory, where a value formed in an earlier step is
+// visible after that step's barrier.  For contexts
+//  * that have no memory for the copy (six fields padded by 64 / (nY-2) and
+//    (planes + 2) / planes, with thin slabs more than the rest of the context);
+//  * whose sweeps are short: a step costs about 1 us more than on the copy, the
+//    copies 10 to 20 us.  8x8x258 in 128 slabs (12 steps), FP64: 27 us a Gauss-Seidel
+//    sweep, on the copy 43; 21x12x15 in 3 (32 steps) 12 us both, an
+//    Arnoldi step with SSOR 69 and 56; 90x80x50 in 5 (174 steps) 425 and 206, 725
+//    and 183.
+// ----------------------------------------------------------------------------
+// snapshot of the planes below and above every slab; layout [component][slab]
+// [below, above] x (nX nY)
+template <class T>
+__global__ void k_slab_halo(Geo g, const T *__restrict__ Ut, T *__restrict__ halo, const GsCtrl *__restrict__ ctrl)
+{
+    const int p = blockIdx.z, hs = blockIdx.y, r = hs >> 1;
+    if (!ctrl->active[p]) return;
+    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= g.sZ) return;
+    const int k = (hs & 1) ? g.slab[2 * r + 1] + 1 : g.slab[2 * r] - 1;
+    halo[((long)p * 2 * g.nslab + hs) * g.sZ + e] = Ut[(long)p * g.N + (long)k * g.sZ + e];
+}
+template <class T>
+__global__ __launch_bounds__(1024) void k_lex_inplace(Geo g, const T *__restrict__ Qall, T *Uall,
+                                                      const T *__restrict__ halo, const GsCtrl *__restrict__ ctrl, int KL,
+                                                      int nyp)
+{
+    const int r = blockIdx.x, p = blockIdx.y;
+    if (!ctrl->active[p]) return;
+    const int jj = threadIdx.x % nyp, l0 = threadIdx.x / nyp * KL, j = jj + 1;
+    const int nx = g.nX - 2, ny = g.nY - 2;
+    const int kb = g.slab[2 * r], nk = g.slab[2 * r + 1] - kb + 1, steps = nx + ny + nk - 2;
+    const long nX = g.nX, sZ = g.sZ;
+    T *u = Uall + (long)p * g.N;
+    const T *q = Qall + (long)p * g.N, *hb = halo + (long)(p * 2 * g.nslab + 2 * r) * sZ, *ht = hb + sZ;
+    const long dn = jj == ny - 1 ? -(ny - 1) * nX : nX, ds = jj == 0 ? (ny - 1) * nX : -nX;   // rows j+1, j-1 (wrapped)
+    const T h = T(g.dt) / T(g.Re), Ae = T(g.Ae), Aw = T(g.Aw), An = T(g.An), As = T(g.As);
+    for (int t = 0; t < steps; t++) {
+        for (int kk = l0; kk < l0 + KL; kk++) {
+            const int i = t - jj - kk + 1, k = kb + kk;
+            if (jj >= ny || kk >= nk || i < 1 || i > nx) continue;
+            const long pl = i + nX * j, c = pl + sZ * k;
+            const T ub = kk == 0 ? hb[pl] : u[c - sZ], ut = kk == nk - 1 ? ht[pl] : u[c + sZ];
+            const T a = Ae * u[c + 1] + Aw * u[c - 1] + An * u[c + dn] + As * u[c + ds];
+            u[c] = (q[c] + h * (a + (T(g.At[k]) * ut + T(g.Ab[k]) * ub))) / (T(1.0) - h * T(g.Ap[k]));
+        }
+        __syncthreads();
+    }
+}
+// forward the unscaled values, scaled where the backward sweep reads its operand
+template <class T>
+__global__ __launch_bounds__(1024) void k_ssor_inplace(Geo g, const T *__restrict__ rin, T *out,
+                                                       const int *__restrict__ active, int KL, int nyp)
+{
+    if (active && !*active) return;
+    const int r = blockIdx.x;
+    const int jj = threadIdx.x % nyp, l0 = threadIdx.x / nyp * KL, j = jj + 1;
+    const int nx = g.nX - 2, ny = g.nY - 2;
+    const int kb = g.slab[2 * r], nk = g.slab[2 * r + 1] - kb + 1, steps = nx + ny + nk - 2;
+    const long nX = g.nX, sZ = g.sZ;
+    const T om = T(g.omega), back = (T(2) - om) / om;
+    const T Ae = T(g.Ae), Aw = T(g.Aw), An = T(g.An), As = T(g.As);
+    for (int s = 0; s < 2 * steps; s++) {
+        const int t = s < steps ? s : 2 * steps - 1 - s;
+        for (int kk = l0; kk < l0 + KL; kk++) {
+            const int i = t - jj - kk + 1, k = kb + kk;
+            if (jj >= ny || kk >= nk || i < 1 || i > nx) continue;
+            const long c = i + nX * j + sZ * k;
+            T a;
+            if (s < steps)
+                a = rin[c] + Aw * (i == 1 ? T(0) : out[c - 1]) + As * (jj == 0 ? T(0) : out[c - nX]) +
+                    T(g.Ab[k]) * (kk == 0 ? T(0) : out[c - sZ]);
+            else
+                a = back * T(g.Ap[k]) * out[c] + Ae * (i == nx ? T(0) : out[c + 1]) +
+                    An * (jj == ny - 1 ? T(0) : out[c + nX]) + T(g.At[k]) * (kk == nk - 1 ? T(0) : out[c + sZ]);
+            out[c] = -om * a * T(g.rAp[k]);
+        }
+        __syncthreads();
+    }
+}
+bool slab_copy_pays(const Geo &g) { return g.nX + g.nY + g.nkmax - 6 >= 20; }
+size_t slab_scratch_inplace(const Geo &g, bool lex) { return lex ? 6 * (size_t)g.nslab * g.sZ : 0; }
+
 // CASE(KL, threads, steps that Gauss-Seidel and SSOR load ahead): what the
 // registers of the workgroup's threads hold, of KL + 2 loads a line and one a line
 #define SLAB_CASES(CASE)                                                                                             \
@@ -2270,8 +2355,14 @@ void launch_helm_lex(const Geo &g, const T *Q, T *Ut, T *scr, const void *ctrl, 
 {
     int KL, nkc, nyp;
     const int nt = slab_shape(g, g.nkmax, KL, nkc, nyp);
-    const Skew sk = skew_of(g);
     const GsCtrl *gc = (const GsCtrl *)ctrl;
+    if (!g.skew) {
+        hipLaunchKernelGGL(k_slab_halo<T>, dim3((unsigned)((g.sZ + 255) / 256), 2 * g.nslab, 3), dim3(256), 0, s, g,
+                           (const T *)Ut, scr, gc);
+        hipLaunchKernelGGL(k_lex_inplace<T>, dim3(g.nslab, 3), dim3(nt), 0, s, g, Q, Ut, (const T *)scr, gc, KL, nyp);
+        return;
+    }
+    const Skew sk = skew_of(g);
     const size_t ring = sizeof(T) * (size_t)(nkc * KL) * (g.nY - 2);
     launch_skew<T, true>(g, sk, Ut, Q, scr, nullptr, gc->active, 1, 6, s);
 #define LEX_CASE(kl, mt, sd, sds) \
@@ -2285,6 +2376,10 @@ static void launch_ssor_block(const Geo &g, const T *r, T *scr, T *out, const in
 {
     int KL, nkc, nyp;
     const int nt = slab_shape(g, g.nkmax, KL, nkc, nyp);
+    if (!g.skew) {
+        hipLaunchKernelGGL(k_ssor_inplace<T>, dim3(g.nslab), dim3(nt), 0, s, g, r, out, active, KL, nyp);
+        return;
+    }
     const Skew sk = skew_of(g);
     launch_skew<T, true>(g, sk, r, nullptr, scr, nullptr, active, 0, 1, s);
 #define SSOR_CASE(kl, mt, sd, sds) \
