@@ -702,13 +702,7 @@ __global__ __launch_bounds__(64 * ZL_MAXC) void k_helm_zline(Geo g, const T *__r
     // blocks run span-row-first inside panels of pw column tiles, so that the
     // rows j-1, j, j+1 (the span neighbours of row j) are swept at nearly the
     // same time and their second and third reads hit L2
-    // a block sweeps one component (component slowest): the three do not read
-    // each other, a small grid gets three times the blocks of its serial
-    // chains, and on a large one a block's barriers wait less on each other.
-    // One pass: FP64 64x32x48 33.5 -> 11 us, 256x64x96 40 -> 20 us,
-    // 512x128x128 95 -> 83 us; FP32 1024x256x192 275 -> 259 us
-    const int p = (int)(blockIdx.x / nblk);
-    const unsigned L = xcd_remap(blockIdx.x - (unsigned)p * nblk, nblk);
+    const unsigned L = xcd_remap(blockIdx.x, nblk);
     const unsigned nyr = nblk / nbx;
     const unsigned P = L / (pw * nyr), w_ = min(pw, nbx - P * pw), rem = L - P * pw * nyr;
     const int bx = (int)(P * pw + rem % w_), j = (int)(rem / w_) + 1;
