@@ -159,7 +159,9 @@ int tbl_download(tbl_ctx *ctx, double *Ut, double *Press, double *PCorr);
 /* named work fields for block-level calls: see TBL_F_*.  TBL_F_UTOLD: the step
  * reads Utold only at the inflow plane of u (dnssetbl.f90:791), so
  * tbl_begin_step saves only Ut(1,:,:,1) there; its other entries keep what
- * was last set. */
+ * was last set.  TBL_F_WORK: a work vector, its boundary entries kept zero; pressure
+ * solves by the reference's rule, direct solves (TBL_HELM_DIRECT, adjoint windows)
+ * and tbl_apply_operator overwrite it. */
 enum { TBL_F_UT = 0, TBL_F_UTOLD = 1, TBL_F_PRESS = 2, TBL_F_PCORR = 3, TBL_F_PRHS = 4,
        TBL_F_Q = 5, TBL_F_WORK = 6 };
 int tbl_field_set(tbl_ctx *ctx, int field, const double *host);

@@ -102,10 +102,6 @@ struct tbl_ctx {
     std::string err;
 };
 
-// device diagnostics record; the mass-flux partials (5 * MF_BLK) follow it
-enum { DD_DIV = 0, DD_MASS = 1, DD_KE = 6, DD_BNORM = 7, DD_GUARD = 8, DD_NCOUNT = 9,
-       DD_J = DD_NCOUNT + 5 * MF_BLK };   // behind the mass-flux partials: the objective of an adjoint window
-
 struct HostPub {
     unsigned seq, pad;
     GmStatus gm;
@@ -1348,7 +1344,7 @@ static int gmres_impl(tbl_ctx *c, double errtol, int kmax, int mmax, int *cycles
     double *part_z = c->part + nbr + 8;        // norm partials (and dot partials)
     const bool fuse_dot = poisson_blocks(g, c->mixed) <= c->npart - nbr - 8;
     if (c->p.pc_extrap) {
-        // initial guess 2 PCorr(n-1) - PCorr(n-2); the face values are zeroed below
+        // initial guess 2 PCorr(n-1) - PCorr(n-2), both with zero faces
         if (!c->PCprev) CHK(dalloc(c, &c->PCprev, (size_t)N * sizeof(double)));
         if (c->pc_hist >= 2) launch_pc_extrap(c->PCorr, c->PCprev, N, c->s);
         else HIPCHK(c, hipMemcpyAsync(c->PCprev, c->PCorr, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, c->s));

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void k_mass_flux(Geo g, const T *__restrict__ 
 }
 // last kernel of the diagnostics: the divergence sum (as k_fin_sum), the mass
 // fluxes, and the record to the host
-struct DiagRec { double w[9]; };
+struct DiagRec { double w[DD_NCOUNT]; };
 __global__ __launch_bounds__(1024) void k_fin_diag(const double *part, int nb, const double *__restrict__ mpart,
                                                   double denom, double *rec, Pub pub)
 {
@@ -157,14 +157,14 @@ __global__ __launch_bounds__(1024) void k_fin_diag(const double *part, int nb, c
         const int q = threadIdx.x - 64;
         double a = 0.0;
         for (int b = 0; b < MF_BLK; b++) a += mpart[q * MF_BLK + b];
-        rec[1 + q] = a / denom;
+        rec[DD_MASS + q] = a / denom;
     }
     double a = 0.0;
 #pragma unroll 8
     for (int q = threadIdx.x; q < nb; q += 1024) a += part[q];
     const double s = block_sum<1024>(a, sh, threadIdx.x);
     if (threadIdx.x != 0) return;
-    if (nb > 0) rec[0] = s;
+    if (nb > 0) rec[DD_DIV] = s;
     publish(pub, (const DiagRec *)rec);
 }
 void launch_fin_diag(const double *part, int nb, const double *mpart, double denom, double *rec, const Pub &pub, hipStream_t s)
@@ -172,6 +172,8 @@ void launch_fin_diag(const double *part, int nb, const double *mpart, double den
     hipLaunchKernelGGL(k_fin_diag, dim3(1), dim3(1024), 0, s, part, nb, mpart, denom, rec, pub);
 }
 
+// ---------------------------------------------------------------- a14
+// thread per (i,k); the span sum runs in the reference's j order
 template <class T>
 __global__ __launch_bounds__(256) void k_stats(Geo g, const T *__restrict__ Ut, double *__restrict__ sums)
 {

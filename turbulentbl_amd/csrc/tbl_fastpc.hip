@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void k_xform64(const double *__restrict__ A, d
         // even, 62 span rows loaded six groups for four, and 43 planes formed four
         // for three: the transforms of 256x64x96, three components, 30.5 -> 28.5
         // and 24 -> 22.4 us, one 13.6 -> 11.7 and 10.7 -> 8.8; a step of 90x80x50
-        // 341 -> 327 us.
+        // 341 -> 332 us.
         for (; kg + 3 < KG; kg += 2) {
             step(kg, p0, std::true_type{});
             step(kg + 1, p1, std::true_type{});
@@ -710,7 +710,7 @@ void fastpc_destroy(FastPC *f)
 // The FP32 solve is bound by instruction issue, not by HBM: it takes its
 // reciprocals from v_rcp_f32 (1 ulp), one instruction where a correctly
 // rounded division is about ten; the solve is a preconditioner, which FP32
-// rounding of this size does not change.  FP64 divides exactly.
+// rounding of this size does not change.  FP64 divides.
 #define LS_WAVES 2
 template <class T> __device__ __forceinline__ T ls_div(T a, T b) { return a / b; }
 template <> __device__ __forceinline__ float ls_div<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }

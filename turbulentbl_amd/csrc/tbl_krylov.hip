@@ -170,7 +170,7 @@ __device__ __forceinline__ void open_cycle(GmCtrl *c, double rho)
 // mode).  dnssetbl.f90:536-546.
 __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_r, int nb_r,
                                                  const double *part_z, int nb_z, int first,
-                                                 const double *part_b, Pub pub)
+                                                 const double *part_b)
 {
     __shared__ double sh[FB / 64];
     __shared__ double rho_s;
@@ -199,7 +199,6 @@ __global__ __launch_bounds__(FB) void k_fin_start(GmCtrl *c, const double *part_
     } else {
         start_true(c, rho);
     }
-    publish(pub, &st);
 }
 
 // A cycle whose preconditioner inverts A nearly exactly needs no Arnoldi step:
@@ -490,9 +489,9 @@ void launch_norm2(const T *x, long N, double *part, const int *active, hipStream
     hipLaunchKernelGGL(k_norm2<T>, dim3(vec_blocks(N, sizeof(T) == 4)), dim3(VB), 0, s, x, N, part, active);
 }
 void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
-                      const double *part_b, const Pub &pub)
+                      const double *part_b)
 {
-    hipLaunchKernelGGL(k_fin_start, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, first, part_b, pub);
+    hipLaunchKernelGGL(k_fin_start, dim3(1), dim3(FB), 0, s, c, part_r, nb_r, part_z, nb_z, first, part_b);
 }
 void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, const Pub &pub, hipStream_t s)
 {

@@ -105,7 +105,7 @@ void launch_fill(double *x, double v, long n, hipStream_t s);
 template <class T> void launch_norm2(const T *x, long N, double *part, const int *active, hipStream_t s);
 // part_b (optional): nb_r block partials of ||pRhs||^2 (start of a true-residual solve)
 void launch_fin_start(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, int first, hipStream_t s,
-                      const double *part_b = nullptr, const Pub &pub = Pub());
+                      const double *part_b = nullptr);
 // judges the tentative unit step: residual partials part_r, and the block
 // partials of its preconditioned residual (part_z, reference's stopping rule)
 void launch_fin_unit(GmCtrl *c, const double *part_r, int nb_r, const double *part_z, int nb_z, const Pub &pub, hipStream_t s);
@@ -134,9 +134,12 @@ void launch_fin_sum(const double *part, int nb, double *out, hipStream_t s);
 // out2[0] = |sum of part| / nint, out2[1] = the sum
 void launch_fin_div(const double *part, int nb, double nint, double *out2, hipStream_t s);
 #define MF_BLK 64   // mass-flux partial blocks per plane
+// device diagnostics record; the mass-flux partials (5 * MF_BLK) follow it
+enum { DD_DIV = 0, DD_MASS = 1, DD_KE = 6, DD_BNORM = 7, DD_GUARD = 8, DD_NCOUNT = 9,
+       DD_J = DD_NCOUNT + 5 * MF_BLK };   // behind the mass-flux partials: the objective of an adjoint window
 template <class T> void launch_mass_flux(const Geo &g, const T *Ut, const int *planes, double *part, hipStream_t s);
-// rec[0] = sum of the nb divergence partials (nb > 0), rec[1..5] = mass flux
-// (mpart given); publishes the nine words of rec
+// rec[DD_DIV] = sum of the nb divergence partials (nb > 0), rec[DD_MASS..] = mass
+// flux (mpart given); publishes the record
 void launch_fin_diag(const double *part, int nb, const double *mpart, double denom, double *rec, const Pub &pub, hipStream_t s);
 template <class T> void launch_stats(const Geo &g, const T *Ut, double *sums, hipStream_t s);
 template <class T> void launch_rescale(const Geo &g, int i_rec0, int nsamples, const T *Ut, double *sums,

@@ -1883,7 +1883,7 @@ __global__ __launch_bounds__(256) void k_skew(Geo g, Skew sk, const T *__restric
     __shared__ T sh[64][65];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     // row m of the tile: column c0 + m - jr of span row jr
-    const int c0 = 64 * blockIdx.x, rows = min(g.nY - 2 - 64 * wb, 64), ncol = g.nX + 63;
+    const int c0 = 64 * blockIdx.x, rows = min(g.nY - 2 - 64 * wb, 64);
     T *Sb = S + f * sk.fs + r * sk.ss + (long)(c0 + 64 * wb + kk + 1) * sk.len + (kk + 1) * sk.nyp + 64 * wb;
     const long f0 = (long)k * g.sZ + (long)(64 * wb + 1) * g.nX;
     if constexpr (IN) {
