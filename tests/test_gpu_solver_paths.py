@@ -285,3 +285,50 @@ def test_slab_sweeps_without_memory_for_their_copy(tbl, grid, P, precision, leav
         Uo = s.Ut.copy(order="F")
         g.diffusion_solve(Q, Uo, order=orc.GS_LEX_BLOCK, errorstop=1e-30, mmax=2)
         assert np.array_equal(got[1][0], Uo) and np.array_equal(got[1][1][I], g.precond_apply(x, orc.PC_SSOR_BLOCK)[I])
+
+
+# a tolerance between what a solve is expected to reach on this grid and what it
+# reaches: the unit step is tried, refused, and the Arnoldi steps start from V_0
+def test_refused_unit_step_by_the_reference_rule(tbl):
+    grid, errtol = (33, 128, 40), 3e-11
+    with _solver(tbl, grid, precond=tbl.TBL_PC_FAST, kmax=8) as sv:
+        b, got = sv.zeros(), []
+        b[I] = np.random.default_rng(1).standard_normal([n - 2 for n in grid])
+        sv.set_field(tbl.F_PRHS, b)
+        sv.timer_enable(["precond"])
+        out = sv.ppe_solve(errtol, 8, 50)
+        n = sv.timer_read()["precond"]["count"]
+        x = sv.get_field(tbl.F_PCORR)
+        r = b - sv.apply_operator(0, x)
+        for q in range(3):
+            f = np.moveaxis(r, q, 0)
+            f[0] = f[-1] = 0.0
+        rel = np.linalg.norm(sv.apply_operator(1, r)) / np.linalg.norm(sv.apply_operator(1, b))
+    assert n == out["cycles"] + out["iters"] + 1 and out["iters"] > 1
+    # the rule's last test is the Arnoldi estimate; it and the residual of the
+    # solution differ by the rounding of the solves
+    assert rel <= 2 * errtol
+
+
+# true residual: a tolerance that rounding does not let be met, so that no step of
+# the cycle is accepted in the end; refused at once (V_0 in the first vector), or
+# after an accepted step (V_0 in the other one)
+@pytest.mark.parametrize("inner_tol,accepted", [(1e-16, 0), (1e-6, 1)])
+def test_refused_unit_step_by_the_true_residual(tbl, inner_tol, accepted):
+    g, s = make_case(GRID, seed=4)
+    b, got = _rhs(g), []
+    bn = np.linalg.norm(b[I])
+    for errtol, timed in ((1e-9, False), (1e-17, False), (1e-17, True)):
+        with gpu_from_case(g, s, precond=tbl.TBL_PC_FAST, tol_mode=tbl.TBL_TOL_TRUE, inner_tol=inner_tol, kmax=6) as sv:
+            # timed, the next step's first transform is not queued ahead
+            sv.timer_enable(["precond", "poisson"] if timed else [])
+            out, x = _solve(tbl, sv, g, b, errtol=errtol, kmax=6, mmax=3)
+            n = sv.timer_read()
+        rn = np.linalg.norm(b[I] - g.poisson_apply(x)[I])
+        assert abs(out["true_res"] - rn) <= 1e-6 * rn + 1e-15 * bn
+        got.append((out, x, rn))
+    assert got[0][0]["iters"] == 1
+    assert got[1][0] == got[2][0] and np.array_equal(got[1][1], got[2][1])
+    # the steps that follow work at rounding level and leave no more than it
+    assert got[1][0]["cycles"] == 3 and n["poisson"]["count"] == got[1][0]["iters"] - accepted
+    assert got[1][2] <= 2 * got[0][2]
