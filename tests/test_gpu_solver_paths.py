@@ -332,3 +332,33 @@ def test_refused_unit_step_by_the_true_residual(tbl, inner_tol, accepted):
     # the steps that follow work at rounding level and leave no more than it
     assert got[1][0]["cycles"] == 3 and n["poisson"]["count"] == got[1][0]["iters"] - accepted
     assert got[1][2] <= 2 * got[0][2]
+
+
+def test_window_whose_solves_go_one_by_one(tbl):
+    """a gradient on a grid beyond the size of batched solves, FP64 (central
+    differences, the switches replayed: 1e-5 as on small grids) and mixed (against
+    FP64: J 1e-6, gradient 1e-4, as on small grids)"""
+    grid, i0, i1 = (1100, 100, 98), 600, 900
+    rng = np.random.default_rng(9)
+    w = 1e-2 * rng.standard_normal(grid[:2])
+    d = rng.standard_normal(grid[:2])
+    noise = 0.02 * rng.standard_normal([n - 2 for n in grid] + [3], dtype=np.float32)
+    got = []
+    for precision in ("fp64", "mixed"):
+        with _solver(tbl, grid, precision=precision, precond=tbl.TBL_PC_FAST, kmax=1) as sv:
+            U = sv.zeros(3)
+            U[..., 0] = 19.8 * np.tanh(4.0 * sv.mesh()["x3"])
+            U[I] += noise
+
+            def window(wall, **kw):
+                sv.upload(U, sv.zeros(), sv.zeros())
+                sv.set_state()
+                return sv.adjoint_window(2, i0, i1, wall_w=wall, nsnap=1, **kw)
+
+            got.append(window(w, branch_mode=1)[:2])
+            if precision == "fp64":
+                eps, ad = 1e-5, float((got[0][1] * d).sum())
+                Jp, Jm = (window(w + q * eps * d, forward_only=True, branch_mode=2)[0] for q in (1, -1))
+                assert abs((Jp - Jm) / (2 * eps) - ad) <= 1e-5 * abs(ad)
+    (J, grad), (Jx, gx) = got
+    assert abs(Jx - J) <= 1e-6 * abs(J) and np.abs(gx - grad).max() <= 1e-4 * np.abs(grad).max()
