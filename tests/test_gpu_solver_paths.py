@@ -254,6 +254,8 @@ def test_window_without_memory_for_the_adjoint_fields(tbl):
             rc, Jg = window(0)
         assert rc != 0 and Jg == J
         assert window(0) == (0, J)               # and the next call is not taken for failed
+        with _hip().left((3 * 40 + 72) * N + 200e6):
+            assert window(0) == (0, J)
 
 
 # thin slabs, whose sweeps' copy is larger than the rest of the context: with that

@@ -1904,15 +1904,17 @@ extern "C" int tbl_step(tbl_ctx *c, int nsteps, tbl_diag *diag)
 }
 
 // ------------------------------------------------------------------ discrete adjoint
-// Work buffers of one adjoint window, two allocations a call: the snapshots,
-// which are stored before they are read, then the adjoint fields, cleared, once
-// the forward sweep has given J.  A forward evaluation needs none.  An
-// allocation and a clear for each of ten buffers, the snapshots' included, and
-// the start state stored for a forward evaluation too, took 0.1 of the 1.25 ms
-// of a forward call at 64x32x48, 1.3 of the 35.4 ms of a gradient at 256x64x96
-// and 2.1 of the 69.0 ms at 1024x192x160 mixed.
+// Work buffers of one adjoint window, one allocation a call: the adjoint fields,
+// cleared, then the snapshots, which are stored before they are read.  A forward
+// evaluation needs none.  An allocation and a clear for each of ten buffers, the
+// snapshots' included, and the start state stored for a forward evaluation too,
+// took 0.1 of the 1.25 ms of a forward call at 64x32x48, 1.3 of the 35.4 ms of a
+// gradient at 256x64x96 and 2.1 of the 69.0 ms at 1024x192x160 mixed; two
+// allocations, 0.3 of the 6.7 ms at 303x62x105 mixed.  Where there is no memory
+// for both, the snapshots are taken alone and the fields after the forward sweep,
+// so that J is there if the call fails for them.
 struct AdjWin {
-    char *mem = nullptr;
+    char *mem = nullptr, *own = nullptr; // own: the snapshots, if they are an allocation of their own
     double *lamU = nullptr, *lamP = nullptr, *lamQ = nullptr, *lamPhi = nullptr, *lamB = nullptr;
     double *grad = nullptr;
     double *E = nullptr, *Enew = nullptr;   // end-of-step boundary values (launch_adj_save_end): of this step, of the one before
@@ -1928,18 +1930,43 @@ struct AdjWin {
     int nstep0 = 0;
     int brmode = 0;          // 1 record the Peclet switches, 2 replay them (first sweep only)
 };
-static int adj_alloc(tbl_ctx *c, AdjWin &A)
+// bytes of the adjoint fields, each from a multiple of 256; with mem, set up there
+static size_t adj_fields(tbl_ctx *c, AdjWin &A, char *mem)
 {
     const size_t N = (size_t)c->g.N, ne = (size_t)adj_end_len(c->g), nw = (size_t)c->p.nX * c->p.nY;
     struct { double **p; size_t n; } sub[] = {{&A.lamU, 3 * N}, {&A.lamP, N}, {&A.lamQ, 3 * N}, {&A.lamPhi, N},
                                               {&A.lamB, N}, {&A.E, ne}, {&A.Enew, ne}, {&A.grad, nw}};
-    auto up = [](size_t n) { return (n + 31) & ~(size_t)31; };   // 256 bytes
-    size_t fields = 0;
-    for (auto &f : sub) fields += up(f.n);
-    HIPCHK(c, hipMalloc((void **)&A.mem, fields * 8));
-    HIPCHK(c, hipMemsetAsync(A.mem, 0, fields * 8, c->s));
-    double *q = (double *)A.mem;
-    for (auto &f : sub) { *f.p = q; q += up(f.n); }
+    size_t at = 0;
+    for (auto &f : sub) {
+        if (mem) *f.p = (double *)(mem + at);
+        at += (f.n * 8 + 255) & ~(size_t)255;
+    }
+    return at;
+}
+// the snapshots, and the adjoint fields if both find room
+static int adj_alloc(tbl_ctx *c, AdjWin &A)
+{
+    const size_t snaps = (size_t)A.nslots * A.slot_bytes, fields = adj_fields(c, A, nullptr);
+    if (hipMalloc((void **)&A.mem, fields + snaps) == hipSuccess) {
+        adj_fields(c, A, A.mem);
+        A.snapbuf = A.mem + fields;
+        HIPCHK(c, hipMemsetAsync(A.mem, 0, fields, c->s));
+        return 0;
+    }
+    (void)hipGetLastError();
+    A.mem = nullptr;
+    HIPCHK(c, hipMalloc((void **)&A.own, snaps));
+    A.snapbuf = A.own;
+    return 0;
+}
+// the adjoint fields, if they are not there yet
+static int adj_alloc_fields(tbl_ctx *c, AdjWin &A)
+{
+    if (A.mem) return 0;
+    const size_t fields = adj_fields(c, A, nullptr);
+    HIPCHK(c, hipMalloc((void **)&A.mem, fields));
+    adj_fields(c, A, A.mem);
+    HIPCHK(c, hipMemsetAsync(A.mem, 0, fields, c->s));
     return 0;
 }
 // snapshot = Ut (3N), Press (N) in the storage type, PCorr (N, double) and
@@ -2208,7 +2235,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         HIPCHK(c, hipMemsetAsync(A.Jd, 0, 8, c->s));
         A.slot_bytes = (4 * N * c->es + N * 8 + 255) & ~(size_t)255;
         if (!o->forward_only) {
-            HIPCHK(c, hipMalloc((void **)&A.snapbuf, (size_t)A.nslots * A.slot_bytes));
+            CHK(adj_alloc(c, A));
             CHK(snap_store(c, A, 0));
         }
         std::vector<int> at;
@@ -2224,7 +2251,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
         if (o->forward_only) return 0;
         const int fin = A.nslots - 1;
         CHK(snap_store(c, A, fin));
-        CHK(adj_alloc(c, A));
+        CHK(adj_alloc_fields(c, A));
         if (c->mixed) launch_adj_save_end<float>(c->g, F<float>(c->Ut), A.E, c->s);
         else launch_adj_save_end<double>(c->g, F<double>(c->Ut), A.E, c->s);
         launch_adj_tau(c->g, A.lamU, A.i0, A.i1, A.cJ, c->s);
@@ -2239,7 +2266,7 @@ extern "C" int tbl_adjoint_window(tbl_ctx *c, const tbl_adjoint_opts *o, const d
     if (nadj) *nadj = A.nadj;
     hipStreamSynchronize(c->s);
     if (A.mem) hipFree(A.mem);
-    if (A.snapbuf) hipFree(A.snapbuf);
+    if (A.own) hipFree(A.own);
     return rc;
 }
 
