@@ -60,11 +60,23 @@ class _hip:
 
     @contextlib.contextmanager
     def left(self, nbytes):
-        """all but nbytes of the device's memory is taken"""
-        held = []
-        while self.free() - nbytes > 32e6 and len(held) < 8:      # a large allocation may come out smaller
-            held.append(C.c_void_p())
-            assert self.lib.hipMalloc(C.byref(held[-1]), int(self.free() - nbytes)) == 0
+        """no more than nbytes of the device's memory are to be had: they are taken,
+        then all the rest down to 16 MB (what the runtime keeps of freed memory
+        too), then given back"""
+        def take(size):
+            p = C.c_void_p()
+            return p if self.lib.hipMalloc(C.byref(p), int(size)) == 0 else None
+
+        spare, held, size = take(nbytes), [], self.free()
+        assert spare
+        while size >= 16e6:
+            p = take(size)
+            if p:
+                held.append(p)
+            else:
+                size /= 2
+        self.lib.hipFree(spare)
+        self.lib.hipGetLastError()               # of the allocations that failed
         try:
             yield
         finally:
